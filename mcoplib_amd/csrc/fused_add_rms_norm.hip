@@ -23,12 +23,21 @@ namespace mcop {
 
 // With eight vectors a lane the kernel asks for four waves per SIMD (at most 128 VGPRs, met
 // without spilling; 138 and three waves left free): rows of 20480-24576 bf16 elements ran 5-9%
-// faster.  fp16 would spill under that bound and keeps the default.
+// faster.  fp16 would spill under that bound and keeps the default, and so does the bf16 EX form
+// (at most 256 rows at this width: one workgroup a CU whatever its registers).  The fp32 EX form
+// is to beat the generic one's four waves or give way to it: it asks for five, which it misses by
+// two registers, so its rows take the generic form.
 // EX (exact): one row per workgroup and every lane in the row (tpr == blockDim.x, NV * tpr ==
 // hidden / VEC): uniform row index, scalar base addresses with 32-bit offsets, no bounds tests.
+template <class E, int NV, bool EX>
+__host__ __device__ constexpr int h1_waves() {
+  if (NV != 8 || std::is_same<E, F16>::value) return 1;
+  if (!EX) return 4;
+  return std::is_same<E, F32>::value ? 5 : 1;
+}
 template <class E, int VEC, int NV, bool EX = false>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
-__attribute__((amdgpu_waves_per_eu(NV == 8 && !std::is_same<E, F16>::value ? 4 : 1)))
+__attribute__((amdgpu_waves_per_eu(h1_waves<E, NV, EX>())))
 k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
                      typename E::S* __restrict__ res, const typename E::S* __restrict__ w,
                      int64_t rows, int hidden, int tpr, float eps) {
@@ -49,8 +58,11 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
   };
 
   Pack<S, VEC> xv[NV], rv[NV], wv[NV];
+  // fp16 at sixteen vectors a lane requests the last of the weight only after x and the residual
+  // are summed (the latency falls into the reduction): all three at once spill.
+  constexpr int w_early = NV >= 16 && std::is_same<E, F16>::value ? 12 : NV;
 #pragma unroll
-  for (int v = 0; v < NV; ++v) wv[v] = ld<S, VEC>(row_elem<EX>(w, 0, lj_of(v)));
+  for (int v = 0; v < w_early; ++v) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj_of(v)));
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -59,11 +71,12 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
     rv[v] = ld_nt<S, VEC>(row_elem<EX>(res, rlbase, lj));
   }
 
+  const int slt = EX ? p.lt : store_lane<NV>(p.lt);
   float z[NV][VEC];
   double ss = 0.0;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int j = vec_index(v, tpr, p.lt);
+    const int j = vec_index(v, tpr, slt);
     const bool in = EX || j < nvec;
     Pack<S, VEC> o;
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
@@ -79,19 +92,21 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
     if (p.live && in) st_nt<S, VEC>(row_elem<EX>(res, rbase, (int64_t)j * VEC), o);
   }
 
-  ss = row_reduce<EX>(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  if constexpr (w_early < NV) {
+    shared_loads_first();
+#pragma unroll
+    for (int v = w_early; v < NV; ++v) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj_of(v)));
+    shared_loads_first();
+  }
+  ss = row_reduce<EX, (NV < 8)>(ss, red_sum, tpr, SumOp());
+  const float rho = row_inv_rms(ss, hidden, eps);
 
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int j = vec_index(v, tpr, p.lt);
+    const int j = vec_index(v, tpr, slt);
     if (p.live && (EX || j < nvec)) {
-      Pack<S, VEC> o;
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        o.v[e] = E::from_f(rnd<E>(z[v][e] * rho) * E::to_f(wv[v].v[e]));
-      }
-      st_nt<S, VEC>(row_elem<EX>(x, xbase, (int64_t)j * VEC), o);
+      st_nt<S, VEC>(row_elem<EX>(x, xbase, (int64_t)j * VEC),
+                    norm_store<E, VEC>(z[v], rho, wv[v]));
     }
   }
 }
@@ -148,16 +163,13 @@ k_fused_add_rms_norm_split(typename E::S* __restrict__ x, int64_t x_stride,
   SplitRowReduce red{red_sum, nullptr, tpr, ws, row, slices, sl,
                      ws + split_ws_words(rows, slices) - 1, timeout_ticks, &x_sum, nullptr};
   ss = red.sum(ss);
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  const float rho = row_inv_rms(ss, hidden, eps);
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     if (in_of(v)) {
-      Pack<S, VEC> o;
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        o.v[e] = E::from_f(rnd<E>(E::to_f(xv[v].v[e]) * rho) * E::to_f(wv[v].v[e]));
-      }
-      st_nt<S, VEC>(row_elem<true>(x, xbase, lj_of(v)), o);
+      float z[VEC];
+      widen<E, VEC>(z, xv[v]);
+      st_nt<S, VEC>(row_elem<true>(x, xbase, lj_of(v)), norm_store<E, VEC>(z, rho, wv[v]));
     }
   }
 }
@@ -263,18 +275,15 @@ k_fused_add_rms_norm_wide(typename E::S* __restrict__ x, int64_t x_stride,
   const int tail0 = (NC + NL) * tpr + tid;
   for (int j = tail0; j < nvec; j += tpr) ss += sum_sq(z_of(j * VEC));
   ss = row_reduce(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  const float rho = row_inv_rms(ss, hidden, eps);
   // the lane index again, opaque to the compiler: the second pass recomputes its addresses
   // instead of holding the first pass's in registers across the reduction
   int tid2 = tid;
   asm volatile("" : "+v"(tid2));
   auto y_of = [&](const Pack<S, VEC>& z, const Pack<S, VEC>& wv) {
-    Pack<S, VEC> y;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      y.v[e] = E::from_f(rnd<E>(E::to_f(z.v[e]) * rho) * E::to_f(wv.v[e]));
-    }
-    return y;
+    float zf[VEC];
+    widen<E, VEC>(zf, z);
+    return norm_store<E, VEC>(zf, rho, wv);
   };
 #pragma unroll
   for (int g = 0; g < NC; g += G) {

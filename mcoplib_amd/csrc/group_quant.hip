@@ -29,40 +29,39 @@
 
 namespace mcop {
 
-// max over aligned runs of `lanes` consecutive lanes (a power of two <= 64) of one wave: DPP
+// max (of values >= +0, not NaN) over aligned runs of `lanes` consecutive lanes (a power of two <= 64) of one wave: DPP
 // moves within 16-lane rows, LDS-routed shuffles across them
-__device__ __forceinline__ float group_max(float v, int lanes) {
-  const MaxOp op;
+__device__ __forceinline__ float group_max(float m, int lanes) {
+  const AbsMaxOp op;
+  uint32_t v = __builtin_bit_cast(uint32_t, m);
   if (lanes >= 2) v = op(v, dpp_mov<kDppXor1>(v));
   if (lanes >= 4) v = op(v, dpp_mov<kDppXor2>(v));
   if (lanes >= 8) v = op(v, dpp_mov<kDppHalfMirror>(v));
   if (lanes >= 16) v = op(v, dpp_mov<kDppMirror>(v));
   if (lanes >= 32) v = op(v, __shfl_xor(v, 16, 64));
   if (lanes >= 64) v = op(v, __shfl_xor(v, 32, 64));
-  return v;
+  return __builtin_bit_cast(float, v);
 }
 
 // Scale (*s) and codes of one vector of y in a group whose absmax is m (the multi-pass kernel's
 // form of the register-resident kernel's inline epilogue).
 template <class E, int VEC, bool FP8>
-__device__ __forceinline__ Pack<uint8_t, VEC> group_codes(const float* y, float m, bool has_ub,
+__device__ __forceinline__ Codes<VEC> group_codes(const float* y, float m, bool has_ub,
                                                           float ub, float* s_out) {
   const float A = has_ub ? __builtin_fminf(m, ub) : m;
-  const float s = FP8 ? __builtin_fmaxf(mcop_div_rn(A, 448.0f), 1.0f / 229376.0f)
-                      : __builtin_fmaxf(mcop_div_rn(A, 127.0f), FLT_EPSILON);
+  const float s = FP8 ? __builtin_fmaxf(div_floored<448>(A), 1.0f / 229376.0f)
+                      : __builtin_fmaxf(div_floored<127>(A), FLT_EPSILON);
   *s_out = s;
-  const float inv = mcop_div_rn(1.0f, s);
-  Pack<uint8_t, VEC> q;
+  const float inv = row_rcp(s);
+  Codes<VEC> q;
   if constexpr (FP8) {
     const bool bounded = A == m && s <= 0x1p100f;
     q = fp8_quotient_codes<VEC>(y, s, inv, mcop_divisor_ok(s), bounded);
   } else if constexpr (std::is_same_v<E, F32>) {
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) q.v[e] = q_i8<-128>(y[e] * inv);
+    q = i8_codes<-128, VEC>(y, inv);
   } else {
     // |y * inv| <= 127 * (1 + 2^-22) < 127.5 (int8 takes no scale bound)
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) q.v[e] = q_i8_in_range(y[e], inv);
+    q = i8_codes_in_range<VEC>(y, inv);
   }
   return q;
 }
@@ -93,7 +92,7 @@ k_rms_norm_group_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
 
   Pack<S, VEC> xv[NV], rv[NV], wv[NV];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) wv[v] = ld<S, VEC>(row_elem<EX>(w, 0, lj_of(v)));
+  for (int v = 0; v < NV; ++v) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj_of(v)));
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -127,8 +126,8 @@ k_rms_norm_group_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
       }
     }
   }
-  ss = row_reduce<EX>(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  ss = row_reduce<EX, (NV < 8)>(ss, red_sum, tpr, SumOp());
+  const float rho = row_inv_rms(ss, hidden, eps);
 
   // Groups are whole (hidden % group == 0), so a group's lanes are all inside the row or all
   // past its end; the latter compute on copies and store nothing.
@@ -136,12 +135,9 @@ k_rms_norm_group_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     m[v] = 0.0f;
+    norm_weigh<E, VEC, true>(a[v], rho, wv[v]);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const float y = rnd<E>(rnd<E>(a[v][e] * rho) * E::to_f(wv[v].v[e]));
-      a[v][e] = y;
-      m[v] = __builtin_fmaxf(m[v], __builtin_fabsf(y));
-    }
+    for (int e = 0; e < VEC; ++e) m[v] = __builtin_fmaxf(m[v], __builtin_fabsf(a[v][e]));
   }
   if constexpr (BLOCKED) {
     float mm = m[0];
@@ -163,26 +159,24 @@ k_rms_norm_group_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     // kept inline (group_codes computes the same): the helper's order (codes before the scale
     // store) measured 1.4% slower here
     const float A = scale_ub != nullptr ? __builtin_fminf(m[v], ub) : m[v];
-    const float s = FP8 ? __builtin_fmaxf(mcop_div_rn(A, 448.0f), 1.0f / 229376.0f)
-                        : __builtin_fmaxf(mcop_div_rn(A, 127.0f), FLT_EPSILON);
+    const float s = FP8 ? __builtin_fmaxf(div_floored<448>(A), 1.0f / 229376.0f)
+                        : __builtin_fmaxf(div_floored<127>(A), FLT_EPSILON);
     const int g = (int)(((int64_t)j * VEC) / group);
     if ((((int64_t)j * VEC) % group) == 0) {
       scales[p.row * scale_row_stride + (int64_t)g * scale_group_stride] = s;
     }
-    const float inv = mcop_div_rn(1.0f, s);
-    Pack<uint8_t, VEC> q;
+    const float inv = row_rcp(s);
+    Codes<VEC> q;
     if constexpr (FP8) {
       const bool bounded = A == m[v] && s <= 0x1p100f;
       q = fp8_quotient_codes<VEC>(a[v], s, inv, mcop_divisor_ok(s), bounded);
     } else if constexpr (std::is_same_v<E, F32>) {
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) q.v[e] = q_i8<-128>(a[v][e] * inv);
+      q = i8_codes<-128, VEC>(a[v], inv);
     } else {
       // |y * inv| <= 127 * (1 + 2^-22) < 127.5 (int8 takes no scale bound)
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) q.v[e] = q_i8_in_range(a[v][e], inv);
+      q = i8_codes_in_range<VEC>(a[v], inv);
     }
-    st_nt<uint8_t, VEC>(row_elem<EX>(out, base, (int64_t)j * VEC), q);
+    st_codes_nt<VEC>(row_elem<EX>(out, base, (int64_t)j * VEC), q);
   }
 }
 
@@ -255,29 +249,28 @@ k_rms_norm_group_quant_split(uint8_t* __restrict__ out, float* __restrict__ scal
                      ws + split_ws_words(rows, slices) - 1, timeout_ticks, &x_sum, nullptr,
                      &x_fail};
   ss = red.sum(ss);
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  const float rho = row_inv_rms(ss, hidden, eps);
   const float ub = scale_ub != nullptr ? *scale_ub : 0.0f;
   const bool failed = red.failed();  // a failed exchange: NaN scales
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     float m = 0.0f;
+    norm_weigh<E, VEC, true>(a[v], rho, wv[v]);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      const float y = rnd<E>(rnd<E>(a[v][e] * rho) * E::to_f(wv[v].v[e]));
-      a[v][e] = y;
-      m = __builtin_fmaxf(m, __builtin_fabsf(y));
+      m = __builtin_fmaxf(m, __builtin_fabsf(a[v][e]));
     }
     m = group_max(m, group / VEC);
     if (!in_of(v)) continue;
     float s;
-    const Pack<uint8_t, VEC> q =
+    const Codes<VEC> q =
         group_codes<E, VEC, FP8>(a[v], m, scale_ub != nullptr, ub, &s);
     const int64_t o = lj_of(v);
     if (o % group == 0) {
       scales[row * scale_row_stride + (o / group) * scale_group_stride] =
           failed ? __builtin_nanf("") : s;
     }
-    st_nt<uint8_t, VEC>(row_elem<true>(out, base, o), q);
+    st_codes_nt<VEC>(row_elem<true>(out, base, o), q);
   }
 }
 
@@ -372,22 +365,19 @@ k_rms_norm_group_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scale
     for (int e = 0; e < U; ++e) ss = __builtin_fma((double)t[e], (double)t[e], ss);
   }
   ss = row_reduce(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  const float rho = row_inv_rms(ss, hidden, eps);
   const float ub = scale_ub != nullptr ? *scale_ub : 0.0f;
   auto emit = [&](int64_t o, const float* t) {
-    float wf[U], y[U];
-    const Pack<S, U> wv = raw(w + o);
+    float y[U];
 #pragma unroll
-    for (int e = 0; e < U; ++e) wf[e] = E::to_f(wv.v[e]);
+    for (int e = 0; e < U; ++e) y[e] = t[e];
+    norm_weigh<E, U, true>(y, rho, raw(w + o));
     float m = 0.0f;
 #pragma unroll
-    for (int e = 0; e < U; ++e) {
-      y[e] = rnd<E>(rnd<E>(t[e] * rho) * wf[e]);
-      m = __builtin_fmaxf(m, __builtin_fabsf(y[e]));
-    }
+    for (int e = 0; e < U; ++e) m = __builtin_fmaxf(m, __builtin_fabsf(y[e]));
     m = group_max(m, group / U);
     float s;
-    const Pack<uint8_t, U> q = group_codes<E, U, FP8>(y, m, scale_ub != nullptr, ub, &s);
+    const Codes<U> q = group_codes<E, U, FP8>(y, m, scale_ub != nullptr, ub, &s);
     if (o % group == 0) {
       scales[(int64_t)blockIdx.x * scale_row_stride + (o / group) * scale_group_stride] = s;
     }
@@ -403,10 +393,10 @@ k_rms_norm_group_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scale
       }
     }
     if constexpr (VECLD) {
-      st<uint8_t, U>(out + base + o, q);
+      st_codes<U>(out + base + o, q);
     } else {
 #pragma unroll
-      for (int e = 0; e < U; ++e) out[base + o + e] = q.v[e];
+      for (int e = 0; e < U; ++e) out[base + o + e] = code_of<U>(q, e);
     }
   };
 #pragma unroll

@@ -84,8 +84,12 @@ __device__ __forceinline__ Pack<typename E::S, VEC> norm_out(const float* a,
                                                              int rms_div) {
   Pack<typename E::S, VEC> o;
   if (mode == NORM_VLLM) {
+    float t[VEC];
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(rnd<E>(a[e] * rho) * w.at(e));
+    for (int e = 0; e < VEC; ++e) t[e] = a[e] * rho;
+    rnd_all<E, VEC>(t);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(t[e] * w.at(e));
   } else if (mode == NORM_MC || !rms_div) {
     const float d = (mode == NORM_MC && rms_div) ? inv_rho : rho;
 #pragma unroll
@@ -166,8 +170,8 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
     }
   }
   ss = row_reduce<EX>(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
-  const float inv_rho = mcop_div_rn(1.0f, rho);
+  const float rho = row_inv_rms(ss, hidden, eps);
+  const float inv_rho = row_rcp(rho);
   // The division form: the wave divides in the short form when every lane's elements are in its
   // domain (every a^2 <= ss (1 + 2^-6), rounded or not, for every a that is finite).  Only an
   // fp16 rounding of the residual sum can turn a finite sum (|x + r| >= 65520) into an infinite
@@ -201,7 +205,10 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
     Pack<S, VEC> o;
     if (mode == NORM_VLLM) {
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(rnd<E>(a[v][e] * rho) * wv[v].at(e));
+      for (int e = 0; e < VEC; ++e) a[v][e] *= rho;
+      rnd_all<E, VEC>(a[v]);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(a[v][e] * wv[v].at(e));
     } else if (mode == NORM_MC || !rms_div) {
       const float d = (mode == NORM_MC && rms_div) ? inv_rho : rho;
 #pragma unroll
@@ -286,8 +293,8 @@ k_rms_norm_split(typename E::S* __restrict__ out, typename E::S* __restrict__ ar
   SplitRowReduce red{red_sum, nullptr, tpr, ws, row, slices, sl,
                      ws + split_ws_words(rows, slices) - 1, timeout_ticks, &x_sum, nullptr};
   ss = red.sum(ss);
-  const float rho = mcop_inv_rms(ss, hidden, eps);
-  const float inv_rho = mcop_div_rn(1.0f, rho);
+  const float rho = row_inv_rms(ss, hidden, eps);
+  const float inv_rho = row_rcp(rho);
   // the register kernel's choice of division form, per wave (both forms give the correctly
   // rounded quotient)
   constexpr bool kRoundOverflows = RES && sizeof(S) == 2 && !__is_same(E, BF16);
@@ -318,7 +325,10 @@ k_rms_norm_split(typename E::S* __restrict__ out, typename E::S* __restrict__ ar
     Pack<S, VEC> o;
     if (mode == NORM_VLLM) {
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(rnd<E>(av[e] * rho) * wv[v].at(e));
+      for (int e = 0; e < VEC; ++e) av[e] *= rho;
+      rnd_all<E, VEC>(av);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(av[e] * wv[v].at(e));
     } else if (mode == NORM_MC || !rms_div) {
       const float d = (mode == NORM_MC && rms_div) ? inv_rho : rho;
 #pragma unroll
@@ -418,8 +428,8 @@ k_rms_norm_wide(typename E::S* __restrict__ out, typename E::S* __restrict__ are
     for (int e = 0; e < VEC; ++e) ss = __builtin_fma((double)t[e], (double)t[e], ss);
   }
   ss = row_reduce(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
-  const float inv_rho = mcop_div_rn(1.0f, rho);
+  const float rho = row_inv_rms(ss, hidden, eps);
+  const float inv_rho = row_rcp(rho);
   auto emit = [&](int64_t o, float* t) {
     if constexpr (RES) {
       Pack<S, VEC> r;

@@ -39,7 +39,7 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
                             int64_t pad_bytes, int tpr, float eps) {
   using E = BF16;
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   RowPos p;
   if constexpr (EX) {
     p = row_pos_one();
@@ -57,7 +57,7 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
 
   Pack<uint16_t, VEC> xv[NV], rv[NV], wv[NV];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) wv[v] = ld<uint16_t, VEC>(row_elem<EX>(w, 0, lj_of(v)));
+  for (int v = 0; v < NV; ++v) wv[v] = ld<uint16_t, VEC>(row_elem<true>(w, 0, lj_of(v)));
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -76,6 +76,7 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
     const int j = vec_index(v, tpr, p.lt);
     const bool in = EX || j < nvec;
     double vs = 0.0;
+    float m[VEC];
     Pack<uint16_t, VEC> o;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
@@ -83,26 +84,27 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
       const double d = (double)t;
       vs = __builtin_fma(d, d, vs);
       o.v[e] = E::from_f(t);
-      const float wf = E::to_f(wv[v].v[e]);
-      float m;
-      if constexpr (OPT) {
-        a[v][e] = t * wf;
-        m = a[v][e];
-      } else {
-        a[v][e] = E::to_f(o.v[e]);
-        m = rnd<E>(a[v][e] * wf);
-      }
-      // lanes past the row end hold a copy of vector 0, possibly of the updated residual
-      amax = __builtin_fmaxf(amax, (full || in) ? __builtin_fabsf(m) : 0.0f);
+      if constexpr (OPT) a[v][e] = m[e] = t * E::to_f(wv[v].v[e]);
+    }
+    if constexpr (!OPT) {
+      widen<E, VEC>(a[v], o);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) m[e] = a[v][e] * E::to_f(wv[v].v[e]);
+      rnd_all<E, VEC>(m);
+    }
+    // lanes past the row end hold a copy of vector 0, possibly of the updated residual
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      amax = __builtin_fmaxf(amax, (full || in) ? __builtin_fabsf(m[e]) : 0.0f);
     }
     ss += in ? vs : 0.0;
     if (p.live && in) st_nt<uint16_t, VEC>(row_elem<EX>(res, base, (int64_t)j * VEC), o);
   }
   ss = row_reduce<EX>(ss, red_sum, tpr, SumOp());
-  amax = row_reduce<EX>(amax, red_max, tpr, MaxOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
-  const float s = __builtin_fmaxf(mcop_div_rn(amax * rho, 127.0f), FLT_EPSILON);
-  const float inv = mcop_div_rn(1.0f, s);
+  amax = row_absmax<EX>(amax, red_max, tpr);
+  const float rho = row_inv_rms(ss, hidden, eps);
+  const float s = __builtin_fmaxf(div_floored<127>(amax * rho), FLT_EPSILON);
+  const float inv = row_rcp(s);
   if (p.live && p.lt == 0) {
     scales[p.row] = s;
     uint8_t* sp = padded + pbase + hidden;
@@ -120,22 +122,17 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
     const int j = vec_index(v, tpr, p.lt);
     if (p.live && (EX || j < nvec)) {
       Pack<uint16_t, VEC> o;
-      Pack<uint8_t, VEC> q;
+      if constexpr (OPT) {
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) {
-        float y;
-        if constexpr (OPT) {
-          y = a[v][e] * rho;
-          o.v[e] = E::from_f(y);
-        } else {
-          o.v[e] = E::from_f(rnd<E>(a[v][e] * rho) * E::to_f(wv[v].v[e]));
-          y = E::to_f(o.v[e]);
-        }
-        q.v[e] = q_i8<-127>(y * inv);
+        for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(a[v][e] *= rho);
+      } else {
+        o = norm_store<E, VEC>(a[v], rho, wv[v]);
+        widen<E, VEC>(a[v], o);
       }
+      const Codes<VEC> q = i8_codes<-127, VEC>(a[v], inv);
       st_nt<uint16_t, VEC>(row_elem<EX>(rms, base, (int64_t)j * VEC), o);
-      st_nt<uint8_t, VEC>(row_elem<EX>(q_out, base, (int64_t)j * VEC), q);
-      st_nt<uint8_t, VEC>(row_elem<EX>(padded, pbase, (int64_t)j * VEC), q);
+      st_codes_nt<VEC>(row_elem<EX>(q_out, base, (int64_t)j * VEC), q);
+      st_codes_nt<VEC>(row_elem<EX>(padded, pbase, (int64_t)j * VEC), q);
     }
   }
 }
@@ -157,7 +154,7 @@ k_add_rms_norm_quant_padded_split(uint8_t* __restrict__ padded, uint16_t* __rest
   using E = BF16;
   constexpr int VEC = 8;
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   __shared__ double x_sum;
   __shared__ float x_max;
   __shared__ int x_fail;
@@ -189,27 +186,29 @@ k_add_rms_norm_quant_padded_split(uint8_t* __restrict__ padded, uint16_t* __rest
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     double vs = 0.0;
-    float vm = 0.0f;
+    float vm = 0.0f, m[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       const float t = E::to_f(xv[v].v[e]) + E::to_f(rv[v].v[e]);
       const double d = (double)t;
       vs = __builtin_fma(d, d, vs);
       xv[v].v[e] = E::from_f(t);  // z = b(a), the residual value the generic chain re-reads
-      vm = __builtin_fmaxf(vm, __builtin_fabsf(rnd<E>(E::to_f(xv[v].v[e]) *
-                                                      E::to_f(wv[v].v[e]))));
+      m[e] = E::to_f(xv[v].v[e]) * E::to_f(wv[v].v[e]);
     }
+    rnd_all<E, VEC>(m);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) vm = __builtin_fmaxf(vm, __builtin_fabsf(m[e]));
     ss += in_of(v) ? vs : 0.0;
     amax = __builtin_fmaxf(amax, in_of(v) ? vm : 0.0f);
     if (in_of(v)) st_nt<uint16_t, VEC>(row_elem<true>(res, base, lj_of(v)), xv[v]);
   }
   ss = row_reduce<true>(ss, red_sum, tpr, SumOp());
-  amax = row_reduce<true>(amax, red_max, tpr, MaxOp());
+  amax = row_absmax<true>(amax, red_max, tpr);
   split_sum_max(ws, row, slices, sl, kSplitTag, &ss, &amax, ws + split_ws_words(rows, slices) - 1,
                 timeout_ticks, &x_sum, &x_max, &x_fail);
-  const float rho = mcop_inv_rms(ss, hidden, eps);
-  const float s = __builtin_fmaxf(mcop_div_rn(amax * rho, 127.0f), FLT_EPSILON);
-  const float inv = mcop_div_rn(1.0f, s);
+  const float rho = row_inv_rms(ss, hidden, eps);
+  const float s = __builtin_fmaxf(div_floored<127>(amax * rho), FLT_EPSILON);
+  const float inv = row_rcp(s);
   // slice 0 stores the scale; a slice whose exchange failed stores NaN (split_row.h)
   if (lt == 0 && (sl == 0 || x_fail != 0)) {
     const float s_out = x_fail != 0 ? __builtin_nanf("") : s;
@@ -226,17 +225,15 @@ k_add_rms_norm_quant_padded_split(uint8_t* __restrict__ padded, uint16_t* __rest
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     if (!in_of(v)) continue;
-    Pack<uint16_t, VEC> o;
-    Pack<uint8_t, VEC> q;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      o.v[e] = E::from_f(rnd<E>(E::to_f(xv[v].v[e]) * rho) * E::to_f(wv[v].v[e]));
-      q.v[e] = q_i8<-127>(E::to_f(o.v[e]) * inv);
-    }
+    float f[VEC];
+    widen<E, VEC>(f, xv[v]);
+    const Pack<uint16_t, VEC> o = norm_store<E, VEC>(f, rho, wv[v]);
+    widen<E, VEC>(f, o);
+    const Codes<VEC> q = i8_codes<-127, VEC>(f, inv);
     const int64_t lj = lj_of(v);
     st_nt<uint16_t, VEC>(row_elem<true>(rms, base, lj), o);
-    st_nt<uint8_t, VEC>(row_elem<true>(q_out, base, lj), q);
-    st_nt<uint8_t, VEC>(row_elem<true>(padded, pbase, lj), q);
+    st_codes_nt<VEC>(row_elem<true>(q_out, base, lj), q);
+    st_codes_nt<VEC>(row_elem<true>(padded, pbase, lj), q);
   }
 }
 
@@ -258,7 +255,7 @@ k_add_rms_norm_quant_padded_wide(uint8_t* __restrict__ padded, uint16_t* __restr
   using E = BF16;
   constexpr int NC = VEC > 1 ? 8 : 16, NL = VEC > 1 ? 8 : 0;
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   __shared__ Pack<uint16_t, VEC> lds[NL > 0 ? NL : 1][kWideLanes];
   const int nvec = hidden / VEC;
   const int tpr = (int)blockDim.x, tid = (int)threadIdx.x;
@@ -272,13 +269,17 @@ k_add_rms_norm_quant_padded_wide(uint8_t* __restrict__ padded, uint16_t* __restr
     const Pack<uint16_t, VEC> rv = ld<uint16_t, VEC>(res + base + o);
     const Pack<uint16_t, VEC> wv = ld<uint16_t, VEC>(w + o);
     Pack<uint16_t, VEC> z;
+    float m[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       const float t = E::to_f(xv.v[e]) + E::to_f(rv.v[e]);
       ss = __builtin_fma((double)t, (double)t, ss);
       z.v[e] = E::from_f(t);
-      amax = __builtin_fmaxf(amax, __builtin_fabsf(rnd<E>(E::to_f(z.v[e]) * E::to_f(wv.v[e]))));
+      m[e] = E::to_f(z.v[e]) * E::to_f(wv.v[e]);
     }
+    rnd_all<E, VEC>(m);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) amax = __builtin_fmaxf(amax, __builtin_fabsf(m[e]));
     return z;
   };
   Pack<uint16_t, VEC> zc[NC];
@@ -294,10 +295,10 @@ k_add_rms_norm_quant_padded_wide(uint8_t* __restrict__ padded, uint16_t* __restr
   const int tail0 = (NC + NL) * tpr + tid;
   for (int j = tail0; j < nvec; j += tpr) (void)fold((int64_t)j * VEC);
   ss = row_reduce(ss, red_sum, tpr, SumOp());
-  amax = row_reduce(amax, red_max, tpr, MaxOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
-  const float s = __builtin_fmaxf(mcop_div_rn(amax * rho, 127.0f), FLT_EPSILON);
-  const float inv = mcop_div_rn(1.0f, s);
+  amax = row_absmax(amax, red_max, tpr);
+  const float rho = row_inv_rms(ss, hidden, eps);
+  const float s = __builtin_fmaxf(div_floored<127>(amax * rho), FLT_EPSILON);
+  const float inv = row_rcp(s);
   if (threadIdx.x == 0) {
     scales[blockIdx.x] = s;
     uint8_t* sp = padded + pbase + hidden;
@@ -311,16 +312,14 @@ k_add_rms_norm_quant_padded_wide(uint8_t* __restrict__ padded, uint16_t* __restr
   }
   auto emit = [&](const Pack<uint16_t, VEC>& z, int64_t o) {
     const Pack<uint16_t, VEC> wv = ld<uint16_t, VEC>(w + o);
-    Pack<uint16_t, VEC> ro;
-    Pack<uint8_t, VEC> q;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      ro.v[e] = E::from_f(rnd<E>(E::to_f(z.v[e]) * rho) * E::to_f(wv.v[e]));
-      q.v[e] = q_i8<-127>(E::to_f(ro.v[e]) * inv);
-    }
+    float f[VEC];
+    widen<E, VEC>(f, z);
+    const Pack<uint16_t, VEC> ro = norm_store<E, VEC>(f, rho, wv);
+    widen<E, VEC>(f, ro);
+    const Codes<VEC> q = i8_codes<-127, VEC>(f, inv);
     st<uint16_t, VEC>(rms + base + o, ro);
-    st<uint8_t, VEC>(q_out + base + o, q);
-    st<uint8_t, VEC>(padded + pbase + o, q);
+    st_codes<VEC>(q_out + base + o, q);
+    st_codes<VEC>(padded + pbase + o, q);
   };
 #pragma unroll
   for (int c = 0; c < NC + NL; ++c) {

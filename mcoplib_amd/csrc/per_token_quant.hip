@@ -47,21 +47,21 @@ __device__ __forceinline__ PtqRow ptq_row(float mx, float nmn, const float* scal
     const bool degenerate = !(r.s > 0.0f);
     // zp = rne(-128 - mn / s) converted with saturation (it lies in [-128, 127] for s > 0)
     r.zp = degenerate ? -128 : cvt_rne_i32(-128.0f - mcop_div_rn(mn, r.s));
-    r.inv = degenerate ? 0.0f : mcop_div_rn(1.0f, r.s);
+    r.inv = degenerate ? 0.0f : row_rcp(r.s);
     // a subnormal s (a row of tiny values) makes inv infinite, and the products infinite: the
     // 64-bit sum then keeps -inf at -128 where an int32 sum would wrap
     r.narrow = r.zp >= -(1 << 29) && r.zp <= (1 << 29) && r.inv <= FLT_MAX;
   } else if constexpr (MODE == PTQ_INT8) {
-    r.s = mcop_div_rn(mx, 127.0f);
-    r.inv = mx > 0.0f ? mcop_div_rn(127.0f, mx) : 0.0f;
+    r.s = row_div<127>(mx);
+    r.inv = mx > 0.0f ? row_ratio(127.0f, mx) : 0.0f;
     // an absmax below 127 / FLT_MAX (tiny bf16 rows) makes inv infinite: the products of the
     // row's nonzero values are then infinite and saturate, and 0 * inf = NaN codes 0
     r.in_range = r.inv <= FLT_MAX;
   } else {
     float A = mx;
     if (scale_ub != nullptr) A = __builtin_fminf(A, *scale_ub);
-    r.s = __builtin_fmaxf(mcop_div_rn(A, 448.0f), 1.0f / 229376.0f);
-    r.inv = mcop_div_rn(1.0f, r.s);
+    r.s = __builtin_fmaxf(div_floored<448>(A), 1.0f / 229376.0f);
+    r.inv = row_rcp(r.s);
     r.s_ok = mcop_divisor_ok(r.s);
     r.bounded = A == mx && r.s <= 0x1p100f;
   }
@@ -70,8 +70,8 @@ __device__ __forceinline__ PtqRow ptq_row(float mx, float nmn, const float* scal
 
 // Codes of one vector of v.
 template <class E, int VEC, int MODE>
-__device__ __forceinline__ Pack<uint8_t, VEC> ptq_codes(const float* a, const PtqRow& r) {
-  Pack<uint8_t, VEC> q;
+__device__ __forceinline__ Codes<VEC> ptq_codes(const float* a, const PtqRow& r) {
+  Codes<VEC> q;
   if constexpr (MODE == PTQ_INT8_AZP) {
     // float_to_int32_rn of the reference clamps with fmin/fmax before the saturating
     // conversion, so a NaN product becomes 2^31 -> INT32_MAX and codes 127.  Every finite v lies
@@ -80,34 +80,41 @@ __device__ __forceinline__ Pack<uint8_t, VEC> ptq_codes(const float* a, const Pt
     // 2^30 in magnitude:
     // clamping NaN to 2^30 instead still codes 127, and the int32 sum with zp cannot overflow.
     // Otherwise the sum is formed in 64 bits.  The sum saturates to int8.
+    uint32_t c[VEC];
     if (r.narrow) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         const int t = cvt_rne_i32(__builtin_fminf(a[e] * r.inv, 0x1p30f)) + r.zp;
-        q.v[e] = (uint8_t)(int8_t)(t < -128 ? -128 : (t > 127 ? 127 : t));
+        c[e] = (uint32_t)(t < -128 ? -128 : (t > 127 ? 127 : t));
       }
     } else {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         const int64_t t = (int64_t)cvt_rne_i32(__builtin_fminf(a[e] * r.inv, 0x1p31f)) + r.zp;
-        q.v[e] = (uint8_t)(int8_t)(t < -128 ? -128 : (t > 127 ? 127 : t));
+        c[e] = (uint32_t)(t < -128 ? -128 : (t > 127 ? 127 : t));
       }
     }
+    q = low_bytes<VEC>(c);
   } else if constexpr (MODE == PTQ_INT8) {
     if (std::is_same_v<E, F32> || !r.in_range) {
       // fp32 inputs can carry NaN payloads in the low byte, and an infinite inv gives infinite
       // products: round, convert and saturate
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) q.v[e] = q_i8<-127>(a[e] * r.inv);
+      q = i8_codes<-127, VEC>(a, r.inv);
     } else {
       // |v * inv| <= 127 * (1 + 2^-23) < 127.5, so the code never saturates
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) q.v[e] = q_i8_in_range(a[e], r.inv);
+      q = i8_codes_in_range<VEC>(a, r.inv);
     }
   } else {
     q = fp8_quotient_codes<VEC>(a, r.s, r.inv, r.s_ok, r.bounded);
   }
   return q;
+}
+
+// The row's max (max of v for the zero point, max of |v| otherwise) from the lanes'.
+template <int MODE, bool ONE>
+__device__ __forceinline__ float ptq_row_max(float mx, float* lds, int tpr) {
+  if constexpr (MODE == PTQ_INT8_AZP) return row_reduce<ONE>(mx, lds, tpr, MaxOp());
+  else return row_absmax<ONE>(mx, reinterpret_cast<uint32_t*>(lds), tpr);
 }
 
 template <int MODE>
@@ -158,7 +165,7 @@ k_per_token_quant(uint8_t* __restrict__ out, float* __restrict__ scales, int32_t
       ptq_fold<MODE>(a[v][e], mx, nmn);
     }
   }
-  mx = row_reduce<EX>(mx, red_a, tpr, MaxOp());
+  mx = ptq_row_max<MODE, EX>(mx, red_a, tpr);
   if constexpr (MODE == PTQ_INT8_AZP) nmn = row_reduce<EX>(nmn, red_b, tpr, MaxOp());
   const PtqRow r = ptq_row<MODE>(mx, nmn, scale_ub);
   if (p.live && p.lt == 0) {
@@ -169,7 +176,7 @@ k_per_token_quant(uint8_t* __restrict__ out, float* __restrict__ scales, int32_t
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
     if (p.live && (EX || j < nvec)) {
-      st_nt<uint8_t, VEC>(row_elem<EX>(out, obase, (int64_t)j * VEC), ptq_codes<E, VEC, MODE>(a[v], r));
+      st_codes_nt<VEC>(row_elem<EX>(out, obase, (int64_t)j * VEC), ptq_codes<E, VEC, MODE>(a[v], r));
     }
   }
 }
@@ -222,8 +229,8 @@ k_per_token_quant_split(uint8_t* __restrict__ out, float* __restrict__ scales,
     split_max2(split_slots(ws, row, slices, 0), slices, sl, kSplitTag, &mx, &nmn, err,
                timeout_ticks, x_max, &x_fail);
   } else {
-    SplitRowReduce red{nullptr, red_a, tpr, ws, row, slices, sl, err, timeout_ticks, nullptr,
-                       x_max, &x_fail};
+    SplitRowReduce red{nullptr, reinterpret_cast<uint32_t*>(red_a), tpr, ws, row, slices, sl, err,
+                       timeout_ticks, nullptr, x_max, &x_fail};
     mx = red.max(mx);
   }
   const PtqRow r = ptq_row<MODE>(mx, nmn, scale_ub);
@@ -238,7 +245,7 @@ k_per_token_quant_split(uint8_t* __restrict__ out, float* __restrict__ scales,
     float a[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) a[e] = E::to_f(xv[v].v[e]);
-    st_nt<uint8_t, VEC>(row_elem<true>(out, row * out_stride, lj_of(v)),
+    st_codes_nt<VEC>(row_elem<true>(out, row * out_stride, lj_of(v)),
                         ptq_codes<E, VEC, MODE>(a, r));
   }
 }
@@ -289,7 +296,7 @@ k_per_token_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales,
 #pragma unroll
     for (int e = 0; e < VEC; ++e) ptq_fold<MODE>(E::to_f(xv.v[e]), mx, nmn);
   }
-  mx = row_reduce(mx, red_a, tpr, MaxOp());
+  mx = ptq_row_max<MODE, false>(mx, red_a, tpr);
   if constexpr (MODE == PTQ_INT8_AZP) nmn = row_reduce(nmn, red_b, tpr, MaxOp());
   const PtqRow r = ptq_row<MODE>(mx, nmn, scale_ub);
   if (threadIdx.x == 0) {
@@ -300,8 +307,8 @@ k_per_token_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales,
     float a[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) a[e] = E::to_f(xv.v[e]);
-    const Pack<uint8_t, VEC> q = ptq_codes<E, VEC, MODE>(a, r);
-    if (in) st<uint8_t, VEC>(orow + o, q);
+    const Codes<VEC> q = ptq_codes<E, VEC, MODE>(a, r);
+    if (in) st_codes<VEC>(orow + o, q);
   };
   // The lane index, opaque to the compiler: the codes pass recomputes its vectors' offsets
   // instead of holding them from the loads.

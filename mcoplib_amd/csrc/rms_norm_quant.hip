@@ -48,48 +48,40 @@ __device__ __forceinline__ float row_scale(float amax, float rho, const float* s
   if (MODE != QM_MC_7168 && scale_ub != nullptr) a = __builtin_fminf(a, *scale_ub);
   *A = a;
   if constexpr (FP8) {
-    return __builtin_fmaxf(mcop_div_rn(a, 448.0f), 1.0f / 229376.0f);
+    return __builtin_fmaxf(div_floored<448>(a), 1.0f / 229376.0f);
   } else if constexpr (MODE == QM_MC_7168) {
-    return __builtin_fmaxf(mcop_div_rn(a * rho, 127.0f), FLT_EPSILON);
+    return __builtin_fmaxf(div_floored<127>(a * rho), FLT_EPSILON);
   } else {
-    return __builtin_fmaxf(mcop_div_rn(a, 127.0f), MODE == QM_MC ? 1.5e-6f : FLT_EPSILON);
+    return __builtin_fmaxf(div_floored<127>(a), MODE == QM_MC ? 1.5e-6f : FLT_EPSILON);
   }
 }
 
 // Codes of one vector of y (of p = a * w for QM_MC_7168).  `bounded`: no scale bound cut the
 // row's absmax; `has_ub`: a scale bound was given.
 template <class E, int VEC, bool FP8, int MODE>
-__device__ __forceinline__ Pack<uint8_t, VEC> row_codes(const float* y, float rho, float s,
+__device__ __forceinline__ Codes<VEC> row_codes(const float* y, float rho, float s,
                                                         float inv, bool s_ok, bool bounded,
                                                         bool has_ub) {
-  Pack<uint8_t, VEC> q;
   constexpr int LO = MODE == QM_VLLM ? -128 : -127;
-  if constexpr (FP8) {
-    q = fp8_quotient_codes<VEC>(y, s, inv, s_ok, bounded);
-  } else if (std::is_same_v<E, F32> || (MODE != QM_MC_7168 && has_ub)) {
+  if constexpr (FP8) return fp8_quotient_codes<VEC>(y, s, inv, s_ok, bounded);
+  float t[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) t[e] = MODE == QM_MC_7168 ? y[e] * rho : y[e];
+  if (std::is_same_v<E, F32> || (MODE != QM_MC_7168 && has_ub)) {
     // fp32 inputs can carry NaN payloads in the low byte, and a scale bound lets |y * inv|
     // exceed 127: round, convert and saturate
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const float t = MODE == QM_MC_7168 ? y[e] * rho : y[e];
-      q.v[e] = q_i8<LO>(t * inv);
-    }
-  } else {
-    // |t * inv| < 127.5: the code cannot saturate (nor reach -128)
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-      const float t = MODE == QM_MC_7168 ? y[e] * rho : y[e];
-      q.v[e] = q_i8_in_range(t, inv);
-    }
+    return i8_codes<LO, VEC>(t, inv);
   }
-  return q;
+  // |t * inv| < 127.5: the code cannot saturate (nor reach -128)
+  return i8_codes_in_range<VEC>(t, inv);
 }
 
 // With eight vectors a lane the bf16 int8 kernel asks for four waves per SIMD (at most 128
 // VGPRs, which it meets without spilling): left free it took 140 VGPRs and three waves, one
 // 512-lane workgroup per CU, and rows of 20480-32768 bf16 elements ran 14-20% slower.  The fp8
 // forms, and fp16 (whose conversions need more registers), would spill under that bound and keep
-// the default.
+// the default, and so do the EX forms (at most 256 rows at this width: one workgroup a CU
+// whatever their registers).
 // EX (exact): the workgroup holds one row and every lane owns NV vectors of it (tpr ==
 // blockDim.x, NV * tpr == hidden / VEC, one workgroup per row).  The row index is then uniform,
 // so the row's base addresses are scalar and each vector's 32-bit offset serves every tensor,
@@ -97,14 +89,14 @@ __device__ __forceinline__ Pack<uint8_t, VEC> row_codes(const float* y, float rh
 // 12% less per decode call at T = 1-64 x 5120, about 0.5% at 8192 x 8192).
 template <class E, int VEC, int NV, bool FP8, bool RES, int MODE, bool EX = false>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
-__attribute__((amdgpu_waves_per_eu(NV == 8 && !FP8 && std::is_same<E, BF16>::value ? 4 : 1)))
+__attribute__((amdgpu_waves_per_eu(NV == 8 && !EX && !FP8 && std::is_same<E, BF16>::value ? 4 : 1)))
 k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
                  const typename E::S* __restrict__ x, const typename E::S* __restrict__ w,
                  const float* __restrict__ scale_ub, typename E::S* __restrict__ res,
                  int64_t rows, int hidden, int tpr, float eps) {
   using S = typename E::S;
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   RowPos p;
   if constexpr (EX) {
     p = row_pos_one();
@@ -112,8 +104,7 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     p = row_pos(rows, tpr);
   }
   const int nvec = hidden / VEC;
-  const int64_t base = p.row * (int64_t)hidden;
-  const int64_t lbase = p.lrow * (int64_t)hidden;
+  const int64_t base = p.lrow * (int64_t)hidden;  // the lane's row, where it stores at all
   auto lj_of = [&](int v) {  // element offset of the lane's vector v (loads)
     const int j = vec_index(v, tpr, p.lt);
     return (int64_t)(EX ? j : load_index(j, nvec)) * VEC;
@@ -123,24 +114,25 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   Pack<S, VEC> xv[NV], rv[NV], wv[NV];
   if constexpr (NV >= 4) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) wv[v] = ld<S, VEC>(row_elem<EX>(w, 0, lj_of(v)));
+    for (int v = 0; v < NV; ++v) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj_of(v)));
     shared_loads_first();
   }
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int64_t lj = lj_of(v);
-    xv[v] = ld_nt<S, VEC>(row_elem<EX>(x, lbase, lj));
-    if constexpr (RES) rv[v] = ld_nt<S, VEC>(row_elem<EX>(res, lbase, lj));
+    xv[v] = ld_nt<S, VEC>(row_elem<EX>(x, base, lj));
+    if constexpr (RES) rv[v] = ld_nt<S, VEC>(row_elem<EX>(res, base, lj));
     // with fewer vectors per lane the weight loads interleave with the streamed ones (measured
     // 1.5% faster at 8192 x 8192, two vectors per lane; shared-first won at four)
-    if constexpr (NV < 4) wv[v] = ld<S, VEC>(row_elem<EX>(w, 0, lj));
+    if constexpr (NV < 4) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj));
   }
 
+  const int slt = store_lane<NV>(p.lt);
   float a[NV][VEC];
   double ss = 0.0;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int j = vec_index(v, tpr, p.lt);
+    const int j = vec_index(v, tpr, slt);
     const bool in = EX || j < nvec;
     // Lanes past the row end hold a copy of vector 0: it must not count in the sum.
     double vs = 0.0;
@@ -163,8 +155,8 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     }
   }
 
-  ss = row_reduce<EX>(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  ss = row_reduce<EX, (NV < 8)>(ss, red_sum, tpr, SumOp());
+  const float rho = row_inv_rms(ss, hidden, eps);
 
   // The absmax must skip the copies of vector 0 held past the row end: with an in-place
   // residual that copy may read vector 0's residual after its owner stored the sum there.
@@ -173,33 +165,30 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   float amax = 0.0f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const bool in = full || vec_index(v, tpr, p.lt) < nvec;
+    const bool in = full || vec_index(v, tpr, slt) < nvec;
+    // QM_MC_7168 keeps p = a * w unrounded (its code is rne((p * rho) * inv))
+    norm_weigh<E, VEC, MODE != QM_MC_7168>(a[v], rho, wv[v]);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      // QM_MC_7168 keeps p = a * w unrounded (its code is rne((p * rho) * inv))
-      const float y = MODE == QM_MC_7168
-                          ? a[v][e] * E::to_f(wv[v].v[e])
-                          : rnd<E>(rnd<E>(a[v][e] * rho) * E::to_f(wv[v].v[e]));
-      a[v][e] = y;
-      amax = __builtin_fmaxf(amax, in ? __builtin_fabsf(y) : 0.0f);
+      amax = __builtin_fmaxf(amax, in ? __builtin_fabsf(a[v][e]) : 0.0f);
     }
   }
-  amax = row_reduce<EX>(amax, red_max, tpr, MaxOp());
+  amax = row_absmax<EX, (NV < 8)>(amax, red_max, tpr);
 
   float A;
   const float s = row_scale<FP8, MODE>(amax, rho, scale_ub, &A);
   if (p.live && p.lt == 0) scales[p.row] = s;
-  const float inv = mcop_div_rn(1.0f, s);
+  const float inv = row_rcp(s);
   const bool s_ok = mcop_divisor_ok(s);
   const bool bounded = A == amax && s <= 0x1p100f;  // no scale bound cut the row's absmax
 
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int j = vec_index(v, tpr, p.lt);
+    const int j = vec_index(v, tpr, slt);
     if (p.live && (EX || j < nvec)) {
-      const Pack<uint8_t, VEC> q =
+      const Codes<VEC> q =
           row_codes<E, VEC, FP8, MODE>(a[v], rho, s, inv, s_ok, bounded, scale_ub != nullptr);
-      st_nt<uint8_t, VEC>(row_elem<EX>(out, base, (int64_t)j * VEC), q);
+      st_codes_nt<VEC>(row_elem<EX>(out, base, (int64_t)j * VEC), q);
     }
   }
 }
@@ -221,7 +210,7 @@ k_rms_norm_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales,
   using S = typename E::S;
   constexpr int NC = VEC > 1 ? (RES ? 5 : (FP8 && std::is_same<E, F16>::value ? 7 : 8)) : 16;
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   const int nvec = hidden / VEC;
   const int tpr = (int)blockDim.x;
   const int64_t base = (int64_t)blockIdx.x * hidden;
@@ -296,11 +285,12 @@ k_rms_norm_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales,
     for (int e = 0; e < VEC; ++e) ss = __builtin_fma((double)a[e], (double)a[e], ss);
   }
   ss = row_reduce(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  const float rho = row_inv_rms(ss, hidden, eps);
   auto y_of = [&](int64_t o, const float* a, float* y) {
     const Pack<S, VEC> wv = ld<S, VEC>(w + o);
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) y[e] = rnd<E>(rnd<E>(a[e] * rho) * E::to_f(wv.v[e]));
+    for (int e = 0; e < VEC; ++e) y[e] = a[e];
+    norm_weigh<E, VEC, true>(y, rho, wv);
   };
   float amax = 0.0f;
 #pragma unroll
@@ -321,11 +311,11 @@ k_rms_norm_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales,
 #pragma unroll
     for (int e = 0; e < VEC; ++e) amax = __builtin_fmaxf(amax, __builtin_fabsf(y[e]));
   }
-  amax = row_reduce(amax, red_max, tpr, MaxOp());
+  amax = row_absmax(amax, red_max, tpr);
   float A;
   const float s = row_scale<FP8, MODE>(amax, rho, scale_ub, &A);
   if (threadIdx.x == 0) scales[blockIdx.x] = s;
-  const float inv = mcop_div_rn(1.0f, s);
+  const float inv = row_rcp(s);
   const bool s_ok = mcop_divisor_ok(s);
   const bool bounded = A == amax && s <= 0x1p100f;
   auto emit = [&](int64_t o, const float* a) {
@@ -337,7 +327,7 @@ k_rms_norm_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales,
     }
     float y[VEC];
     y_of(o, a, y);
-    st<uint8_t, VEC>(out + base + o,
+    st_codes<VEC>(out + base + o,
                      row_codes<E, VEC, FP8, MODE>(y, rho, s, inv, s_ok, bounded,
                                                   scale_ub != nullptr));
   };
@@ -376,7 +366,7 @@ k_rms_norm_quant_split(uint8_t* __restrict__ out, float* __restrict__ scales,
   static_assert(MODE != QM_MC_7168, "7168-wide rows fit the register-resident kernel");
   using S = typename E::S;
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   __shared__ double x_sum;
   __shared__ float x_max;
   __shared__ int x_fail;
@@ -430,15 +420,14 @@ k_rms_norm_quant_split(uint8_t* __restrict__ out, float* __restrict__ scales,
   SplitRowReduce red{red_sum, red_max, tpr, ws, row, slices, sl, err, timeout_ticks, &x_sum,
                      &x_max, &x_fail};
   ss = red.sum(ss);
-  const float rho = mcop_inv_rms(ss, hidden, eps);
+  const float rho = row_inv_rms(ss, hidden, eps);
   float amax = 0.0f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
+    norm_weigh<E, VEC, true>(a[v], rho, wv[v]);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      const float y = rnd<E>(rnd<E>(a[v][e] * rho) * E::to_f(wv[v].v[e]));
-      a[v][e] = y;
-      amax = __builtin_fmaxf(amax, in_of(v) ? __builtin_fabsf(y) : 0.0f);
+      amax = __builtin_fmaxf(amax, in_of(v) ? __builtin_fabsf(a[v][e]) : 0.0f);
     }
   }
   amax = red.max(amax);
@@ -447,13 +436,13 @@ k_rms_norm_quant_split(uint8_t* __restrict__ out, float* __restrict__ scales,
   // slice 0 stores the scale; a slice whose exchange failed stores NaN (split_row.h)
   const bool failed = red.failed();
   if (lt == 0 && (sl == 0 || failed)) scales[row] = failed ? __builtin_nanf("") : s;
-  const float inv = mcop_div_rn(1.0f, s);
+  const float inv = row_rcp(s);
   const bool s_ok = mcop_divisor_ok(s);
   const bool bounded = A == amax && s <= 0x1p100f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     if (in_of(v)) {
-      st_nt<uint8_t, VEC>(out + base + lj_of(v),
+      st_codes_nt<VEC>(out + base + lj_of(v),
                           row_codes<E, VEC, FP8, MODE>(a[v], rho, s, inv, s_ok, bounded,
                                                        scale_ub != nullptr));
     }

@@ -12,6 +12,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cfloat>
+#include <type_traits>
+
 #include "numerics.h"
 
 namespace mcop {
@@ -54,6 +57,26 @@ struct F32 {
 template <class E>
 __device__ __forceinline__ float rnd(float f) {
   return E::to_f(E::from_f(f));
+}
+
+// The same for the N values of one vector.  bf16 values are converted in pairs: one conversion and
+// one register for two values, where converting each alone takes two of both.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+template <class E, int N>
+__device__ __forceinline__ void rnd_all(float* f) {
+  if constexpr (std::is_same_v<E, BF16> && N % 2 == 0) {
+#pragma unroll
+    for (int e = 0; e < N; e += 2) {
+      const uint32_t u = __builtin_bit_cast(
+          uint32_t, __builtin_convertvector((f32x2{f[e], f[e + 1]}), bf16x2));
+      f[e] = __builtin_bit_cast(float, u << 16);
+      f[e + 1] = __builtin_bit_cast(float, u & 0xffff0000u);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; ++e) f[e] = rnd<E>(f[e]);
+  }
 }
 
 // N elements of type T as one aligned register block, so that a 4-, 8- or 16-byte block is one
@@ -120,6 +143,41 @@ __device__ __forceinline__ void st_nt(T* p, const Pack<T, N>& v) {
   }
 }
 
+// One vector of a, normalized and weighted in place: b(b(a * rho) * w), or with ROUND false the
+// unrounded a * w.
+template <class E, int N, bool ROUND>
+__device__ __forceinline__ void norm_weigh(float* a, float rho, const Pack<typename E::S, N>& w) {
+  if constexpr (ROUND) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) a[e] *= rho;
+    rnd_all<E, N>(a);
+  }
+#pragma unroll
+  for (int e = 0; e < N; ++e) a[e] *= E::to_f(w.v[e]);
+  if constexpr (ROUND) rnd_all<E, N>(a);
+}
+
+// One vector of the same, stored: b(b(a * rho) * w).
+template <class E, int N>
+__device__ __forceinline__ Pack<typename E::S, N> norm_store(const float* a, float rho,
+                                                             const Pack<typename E::S, N>& w) {
+  float t[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) t[e] = a[e] * rho;
+  rnd_all<E, N>(t);
+  Pack<typename E::S, N> o;
+#pragma unroll
+  for (int e = 0; e < N; ++e) o.v[e] = E::from_f(t[e] * E::to_f(w.v[e]));
+  return o;
+}
+
+// The values of one stored vector.
+template <class E, int N>
+__device__ __forceinline__ void widen(float* f, const Pack<typename E::S, N>& p) {
+#pragma unroll
+  for (int e = 0; e < N; ++e) f[e] = E::to_f(p.v[e]);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Quantizers.
 
@@ -132,29 +190,80 @@ __device__ __forceinline__ int cvt_rne_i32(float v) {
   return r;
 }
 
-// int8 code of v: saturate(rne(v)) to [LO, 127]; NaN -> 0.
-template <int LO>
-__device__ __forceinline__ uint8_t q_i8(float v) {
-  const int i = cvt_rne_i32(v);
-  return (uint8_t)(i < LO ? LO : (i > 127 ? 127 : i));
+// One vector's codes, four to a dword where they fill dwords: as bytes they were taken apart and
+// put together again wherever two branches (with and without a scale bound, say) met.
+template <int N>
+using Codes = std::conditional_t<N % 4 == 0, Pack<uint32_t, (N + 3) / 4>, Pack<uint8_t, N>>;
+
+template <int N>
+__device__ __forceinline__ uint8_t code_of(const Codes<N>& q, int e) {
+  if constexpr (N % 4 == 0) return (uint8_t)(q.v[e / 4] >> (8 * (e % 4)));
+  else return q.v[e];
 }
 
-// int8 code of t = y * inv when |t| <= 127.5 is guaranteed (absmax scaling, no scale bound):
-// RN(t + 1.5 * 2^23) holds rne(t) in the low mantissa bits (exact for |t| < 2^22), so its low
-// byte is the two's-complement code.  Two operations instead of round / convert / clamp; the
-// empty asm keeps the product rounded on its own (no fused multiply-add).  A NaN t keeps the
-// payload of y, whose low 13 bits are zero for bf16 / fp16 values, so NaN codes 0 as in q_i8.
-__device__ __forceinline__ uint8_t q_i8_in_range(float y, float inv) {
-  float t = y * inv;
-  asm("" : "+v"(t));
-  return (uint8_t)__builtin_bit_cast(uint32_t, t + 12582912.0f);
+template <int N>
+__device__ __forceinline__ void st_codes(uint8_t* p, const Codes<N>& q) {
+  if constexpr (N % 4 == 0) st<uint32_t, N / 4>(reinterpret_cast<uint32_t*>(p), q);
+  else st<uint8_t, N>(p, q);
+}
+template <int N>
+__device__ __forceinline__ void st_codes_nt(uint8_t* p, const Codes<N>& q) {
+  if constexpr (N % 4 == 0) st_nt<uint32_t, N / 4>(reinterpret_cast<uint32_t*>(p), q);
+  else st_nt<uint8_t, N>(p, q);
+}
+
+// The low bytes of N words as codes, four to a dword by three byte permutes.
+template <int N>
+__device__ __forceinline__ Codes<N> low_bytes(const uint32_t* t) {
+  Codes<N> p;
+  if constexpr (N % 4 == 0) {
+#pragma unroll
+    for (int k = 0; k < N / 4; ++k) {
+      const uint32_t lo = __builtin_amdgcn_perm(t[4 * k + 1], t[4 * k], 0x0c0c0400u);
+      const uint32_t hi = __builtin_amdgcn_perm(t[4 * k + 3], t[4 * k + 2], 0x0c0c0400u);
+      p.v[k] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; ++e) p.v[e] = (uint8_t)t[e];
+  }
+  return p;
+}
+
+// int8 codes of y[e] * inv: saturate(rne(.)) to [LO, 127]; NaN -> 0.
+template <int LO, int N>
+__device__ __forceinline__ Codes<N> i8_codes(const float* y, float inv) {
+  uint32_t t[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    const int i = cvt_rne_i32(y[e] * inv);
+    t[e] = (uint32_t)(i < LO ? LO : (i > 127 ? 127 : i));
+  }
+  return low_bytes<N>(t);
+}
+
+// The same where every |y[e] * inv| <= 127.5 (absmax scaling, no scale bound): RN(t + 1.5 * 2^23)
+// holds rne(t) in the low mantissa bits (exact for |t| < 2^22), so its low byte is the
+// two's-complement code.  Two operations instead of round / convert / clamp; the empty asm keeps
+// the product rounded on its own (no fused multiply-add).  A NaN t keeps the payload of y, whose
+// low 13 bits are zero for bf16 / fp16 values, so NaN codes 0 as in i8_codes.
+template <int N>
+__device__ __forceinline__ Codes<N> i8_codes_in_range(const float* y, float inv) {
+  uint32_t t[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    float f = y[e] * inv;
+    asm("" : "+v"(f));
+    t[e] = __builtin_bit_cast(uint32_t, f + 12582912.0f);
+  }
+  return low_bytes<N>(t);
 }
 
 // OCP fp8 e4m3fn codes of N values in [-448 - 2^-15, 448] (v_cvt_pk_fp8_f32: RNE, so a value
 // one ulp beyond -448 codes -448).
 template <int N>
-__device__ __forceinline__ Pack<uint8_t, N> cvt_fp8(const float* c) {
-  Pack<uint8_t, N> p;
+__device__ __forceinline__ Codes<N> cvt_fp8(const float* c) {
+  Codes<N> p;
   if constexpr (N == 1) {
     const int r = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[0], 0, false);
     p.v[0] = (uint8_t)(r & 0xff);
@@ -162,10 +271,8 @@ __device__ __forceinline__ Pack<uint8_t, N> cvt_fp8(const float* c) {
     static_assert(N % 4 == 0, "fp8 packs are built 4 codes per dword");
 #pragma unroll
     for (int d = 0; d < N / 4; ++d) {
-      int r = __builtin_amdgcn_cvt_pk_fp8_f32(c[4 * d + 0], c[4 * d + 1], 0, false);
-      r = __builtin_amdgcn_cvt_pk_fp8_f32(c[4 * d + 2], c[4 * d + 3], r, true);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) p.v[4 * d + k] = (uint8_t)((uint32_t)r >> (8 * k));
+      const int r = __builtin_amdgcn_cvt_pk_fp8_f32(c[4 * d + 0], c[4 * d + 1], 0, false);
+      p.v[d] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c[4 * d + 2], c[4 * d + 3], r, true);
     }
   }
   return p;
@@ -241,8 +348,8 @@ __device__ __forceinline__ float clamp_fp8(float v) {
 // give the same code, so only the upper clamp is applied: it sends NaN to +448 as the two-sided
 // clamp does.  Rows that are not bounded take div_by_const and the two-sided clamp.
 template <int N>
-__device__ __forceinline__ Pack<uint8_t, N> fp8_quotient_codes(const float* a, float b, float inv,
-                                                               bool b_ok, bool bounded) {
+__device__ __forceinline__ Codes<N> fp8_quotient_codes(const float* a, float b, float inv,
+                                                       bool b_ok, bool bounded) {
   float c[N];
   if (bounded) {
 #pragma unroll
@@ -260,17 +367,99 @@ __device__ __forceinline__ Pack<uint8_t, N> fp8_quotient_codes(const float* a, f
 }
 
 // ---------------------------------------------------------------------------------------------
+// Per-row (or per-group) scalars.  Every lane of a row computes them, in a chain that nothing
+// else of the row overlaps with on the latency path, so each is the shortest sequence that gives
+// the correctly rounded binary32 result.  The compiler's own division takes 10 instructions and
+// its binary64 square root 22 of twice the latency; the forms below take 3 and 7.  They are
+// Newton steps from the hardware's approximations, and were compared with the IEEE operations
+// over every binary32 value of the domains stated (1.7e9 values each): no difference.  Outside
+// these domains (wave-uniform branches: the values are the row's) the IEEE operations stand.
+constexpr float kRowMin = 0x1p-100f, kRowMax = 0x1p100f;
+
+// RN(1/b) for b in [2^-100, 2^100].
+__device__ __forceinline__ float rcp_in_domain(float b) {
+  const float r = __builtin_amdgcn_rcpf(b);
+  return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
+}
+// RN(1/b) for every b.
+__device__ __forceinline__ float row_rcp(float b) {
+  if (__builtin_expect(b >= kRowMin && b <= kRowMax, 1)) return rcp_in_domain(b);
+  return 1.0f / b;
+}
+
+// RN(a / D) for a in [2^-100, FLT_MAX], +inf for +inf; a value below 2^-100 for a < 2^-100 (a
+// caller whose scale has a larger floor needs no more).
+template <int D>
+__device__ __forceinline__ float div_floored(float a) {
+  constexpr float inv = 1.0f / (float)D;
+  const float q = a * inv;
+  const float r = __builtin_fmaf(__builtin_fmaf(-q, (float)D, a), inv, q);
+  return a <= FLT_MAX ? r : a;
+}
+// RN(a / D) for a >= 0 or NaN.
+template <int D>
+__device__ __forceinline__ float row_div(float a) {
+  if (__builtin_expect(a >= kRowMin && a <= FLT_MAX, 1)) return div_floored<D>(a);
+  return a / (float)D;
+}
+// RN(n / a) for a constant n in [1, 1024] and a > 0.
+__device__ __forceinline__ float row_ratio(float n, float a) {
+  if (__builtin_expect(a >= kRowMin && a <= kRowMax, 1)) {
+    const float r = rcp_in_domain(a);
+    const float q = n * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, a, n), r, q);
+  }
+  return n / a;
+}
+
+// A value that is the same in every lane, moved to a scalar register.
+__device__ __forceinline__ float uniform(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+
+// mcop_inv_rms, bit for bit: ss/H by Markstein's division, the square root by one coupled Newton
+// step on the hardware's reciprocal root and its remainder, then RN(1/root).
+__device__ __forceinline__ float row_inv_rms(double ss64, int hidden, float eps) {
+  // opaque here, so that these two are not computed (and held) ahead of the row's loads
+  asm volatile("" : "+s"(hidden));
+  const float h = uniform((float)hidden);
+  const float inv_h = uniform(rcp_in_domain(h));
+  const float ss = (float)ss64;
+  const float q = ss * inv_h;
+  const float v = __builtin_fmaf(__builtin_fmaf(-q, h, ss), inv_h, q) + eps;
+  // ss in [2^-60, 2^100] keeps the quotient and its remainder normal (H < 2^32)
+  const bool ok = ss >= 0x1p-60f && ss <= kRowMax && v >= kRowMin && v <= kRowMax;
+  if (__builtin_expect(!ok, 0)) return 1.0f / __builtin_sqrtf(ss / h + eps);
+  const float y = __builtin_amdgcn_rsqf(v);
+  const float g0 = v * y, h0 = 0.5f * y;
+  const float e = __builtin_fmaf(-h0, g0, 0.5f);
+  const float g = __builtin_fmaf(g0, e, g0), hh = __builtin_fmaf(h0, e, h0);
+  return rcp_in_domain(__builtin_fmaf(__builtin_fmaf(-g, g, v), hh, g));
+}
+
+// ---------------------------------------------------------------------------------------------
 // Row reductions.  Every thread of the workgroup must call them (they may contain a barrier).
 // `lds` holds one slot per wave of the workgroup (at most 16).  The sum is of fp64 partials;
 // its result is independent of the order up to fp64 rounding, which the single rounding to
 // fp32 afterwards absorbs.
 
 struct SumOp {
+  static constexpr bool kIdempotent = false;  // op(a, a) == a
   __device__ __forceinline__ double operator()(double a, double b) const { return a + b; }
 };
 struct MaxOp {
+  static constexpr bool kIdempotent = true;
   __device__ __forceinline__ float operator()(float a, float b) const {
     return __builtin_fmaxf(a, b);
+  }
+};
+// The larger of two values that are >= +0 and not NaN (an absmax that starts at 0 and ignores
+// NaN), on their bits, whose order is theirs: an unsigned maximum takes its partner lane as a DPP
+// operand, where the float one needs the move and a canonicalizing step of its own.
+struct AbsMaxOp {
+  static constexpr bool kIdempotent = true;
+  __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const {
+    return a > b ? a : b;
   }
 };
 
@@ -280,6 +469,10 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
   return __builtin_bit_cast(
       float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_mov(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
 }
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov(double v) {
@@ -308,6 +501,9 @@ __device__ __forceinline__ T reduce16(T v, Op op) {
 __device__ __forceinline__ float lane_value(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
 __device__ __forceinline__ double lane_value(double v, int lane) {
   const uint64_t u = __builtin_bit_cast(uint64_t, v);
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
@@ -325,7 +521,14 @@ __device__ __forceinline__ T wave_reduce(T v, Op op) {
 }
 
 // ONE: the workgroup holds exactly one row (tpr == blockDim.x), so its first wave is wave 0.
-template <bool ONE = false, class T, class Op>
+// The row's waves meet in LDS: each writes its value to its slot, and every lane combines the
+// slots: two or four of them directly, more by reading one slot a lane and combining those within
+// each 16-lane segment.  Either way LDS is waited for once; a loop over the slots waited once a
+// wave (64 x 5120, five waves a row and two reductions: 66 us for 16 calls replayed from a graph,
+// 60.5 with this and the shorter scalar chain above).
+// FEW: the direct forms are there too (kernels of eight or more vectors a lane, whose rows have
+// more waves and which have no register to spare, do without).
+template <bool ONE = false, bool FEW = true, class T, class Op>
 __device__ __forceinline__ T row_reduce(T v, T* lds, int tpr, Op op) {
   if (!ONE && tpr < 64) {  // several rows per wave: all-reduce within each row's aligned segment
     v = reduce16(v, op);
@@ -334,14 +537,28 @@ __device__ __forceinline__ T row_reduce(T v, T* lds, int tpr, Op op) {
   }
   v = wave_reduce(v, op);
   if (tpr == 64) return v;  // the row is one wave
-  const int wave = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) lds[wave] = v;
-  __syncthreads();
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // opaque here: slot addresses are not held ahead of the loads
+  const int wave = tid >> 6, slot = tid & 15;
   const int wpr = tpr >> 6;
-  const int first = ONE ? 0 : (wave / wpr) * wpr;
-  T t = lds[first];
-  for (int i = 1; i < wpr; ++i) t = op(t, lds[first + i]);
-  return t;
+  if ((tid & 63) == 0) lds[wave] = v;
+  __syncthreads();
+  // a workgroup with more than one row of several waves holds two of two waves each
+  const int first = !ONE && wpr == 2 ? wave & ~1 : 0;
+  if constexpr (FEW) {
+    if (wpr == 2) return op(lds[first], lds[first + 1]);
+    if (wpr == 4) return op(op(lds[0], lds[1]), op(lds[2], lds[3]));
+  }
+  T t = lds[first + (slot < wpr ? slot : wpr - 1)];
+  if constexpr (!Op::kIdempotent) t = slot < wpr ? t : T(0);
+  return reduce16(t, op);
+}
+
+// The row's absmax from the lanes' (each >= +0 and not NaN).
+template <bool ONE = false, bool FEW = true>
+__device__ __forceinline__ float row_absmax(float v, uint32_t* lds, int tpr) {
+  return __builtin_bit_cast(
+      float, row_reduce<ONE, FEW>(__builtin_bit_cast(uint32_t, v), lds, tpr, AbsMaxOp()));
 }
 
 // Issue order of a lane's loads: the vectors every row shares (weights, smooth scales; L2
@@ -395,14 +612,17 @@ __device__ __forceinline__ RowPos row_pos_one() {
   return p;
 }
 
-// Element j of a row that starts at element `row` of tensor t.  In the exact-row form of a kernel
-// (EX: the workgroup holds one row, so `row` is uniform) a row pointer plus a 32-bit offset (j <
-// hidden, an int), which keeps the row base in scalar registers and lets one offset serve every
-// tensor; otherwise one 64-bit address per lane, as the generic form has always computed it.
-template <bool EX, class T>
+// Element j of a row that starts at element `row` of tensor t.  Where `row` is uniform (UNI: the
+// exact-row form of a kernel, whose workgroup holds one row; a split row's slice; a vector that
+// every row shares, row 0) a row pointer plus a 32-bit byte offset (such rows have at most 2^22
+// elements), which keeps the row base in scalar registers and lets one offset serve every
+// tensor; otherwise one 64-bit address per lane.
+template <bool UNI, class T>
 __device__ __forceinline__ T* row_elem(T* t, int64_t row, int64_t j) {
-  if constexpr (EX) {
-    return (t + row) + (uint32_t)j;
+  if constexpr (UNI) {
+    using B = std::conditional_t<std::is_const_v<T>, const char, char>;
+    return reinterpret_cast<T*>(reinterpret_cast<B*>(t + row) +
+                                (uint32_t)j * (uint32_t)sizeof(T));
   } else {
     return t + row + j;
   }
@@ -425,6 +645,15 @@ __device__ __forceinline__ RowPos row_pos_of(int64_t num_rows, int tpr, int k, i
   p.live = p.row < num_rows;
   p.lrow = p.live ? p.row : num_rows - 1;
   return p;
+}
+
+// The lane index its stores use: with eight or more vectors a lane, one that the compiler cannot
+// tell from another value, so that the stores' addresses are computed again instead of being
+// held from the loads (16 registers, which these kernels do not have).
+template <int NV>
+__device__ __forceinline__ int store_lane(int lt) {
+  if constexpr (NV >= 8) asm volatile("" : "+v"(lt));
+  return lt;
 }
 
 // Vector index of a lane's v-th vector, and the index its loads use (0 when past the row end,

@@ -28,7 +28,7 @@ __global__ void __launch_bounds__(max_tpr(VEC, NV))
 k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
                       const uint16_t* __restrict__ x, const float* __restrict__ sm, int64_t rows,
                       int hidden, int tpr) {
-  __shared__ float red_max[16 * R];
+  __shared__ uint32_t red_max[16 * R];
   const int nvec = hidden / VEC;
   RowPos p[R];
 #pragma unroll
@@ -37,7 +37,8 @@ k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   Pack<float, VEC> sv[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    sv[v] = ld<float, VEC>(sm + (int64_t)load_index(vec_index(v, tpr, p[0].lt), nvec) * VEC);
+    sv[v] = ld<float, VEC>(
+        row_elem<true>(sm, 0, (int64_t)load_index(vec_index(v, tpr, p[0].lt), nvec) * VEC));
   }
   shared_loads_first();
   Pack<uint16_t, VEC> xv[R][NV];
@@ -67,21 +68,19 @@ k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     }
   }
 #pragma unroll
-  for (int k = 0; k < R; ++k) amax[k] = row_reduce(amax[k], red_max + 16 * k, tpr, MaxOp());
+  for (int k = 0; k < R; ++k) amax[k] = row_absmax(amax[k], red_max + 16 * k, tpr);
 
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     if (p[k].live && p[k].lt == 0) scales[p[k].row] = amax[k] * 0.00787401574803f;
-    const float inv = amax[k] > 0.0f ? mcop_div_rn(127.0f, amax[k]) : 0.0f;
+    const float inv = amax[k] > 0.0f ? row_ratio(127.0f, amax[k]) : 0.0f;
     const int64_t base = p[k].row * (int64_t)hidden;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       const int j = vec_index(v, tpr, p[k].lt);
       if (p[k].live && j < nvec) {
-        Pack<uint8_t, VEC> q;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) q.v[e] = q_i8<-128>(a[k][v][e] * inv);
-        st_nt<uint8_t, VEC>(out + base + (int64_t)j * VEC, q);
+        const Codes<VEC> q = i8_codes<-128, VEC>(a[k][v], inv);
+        st_codes_nt<VEC>(out + base + (int64_t)j * VEC, q);
       }
     }
   }
@@ -101,7 +100,7 @@ k_scale_dynamic_quant_split(uint8_t* __restrict__ out, float* __restrict__ scale
                             int64_t groups, int64_t rows, int hidden, int slices, int slice_vecs,
                             uint64_t* __restrict__ ws, int64_t timeout_ticks) {
   static_assert(R == 1 || R == 2, "one or two rows a workgroup");
-  __shared__ float red_max[16 * R];
+  __shared__ uint32_t red_max[16 * R];
   __shared__ float x_max[2];
   __shared__ int x_fail;
   const int nvec = hidden / VEC;
@@ -156,8 +155,8 @@ k_scale_dynamic_quant_split(uint8_t* __restrict__ out, float* __restrict__ scale
                        x_max, &x_fail};
     amax[0] = red.max(amax[0]);
   } else {
-    amax[0] = row_reduce<true>(amax[0], red_max, tpr, MaxOp());
-    amax[1] = row_reduce<true>(amax[1], red_max + 16, tpr, MaxOp());
+    amax[0] = row_absmax<true>(amax[0], red_max, tpr);
+    amax[1] = row_absmax<true>(amax[1], red_max + 16, tpr);
     split_max2(split_slots(ws, g, slices, 0), slices, sl, kSplitTag, &amax[0], &amax[1], err,
                timeout_ticks, x_max, &x_fail);
   }
@@ -166,14 +165,12 @@ k_scale_dynamic_quant_split(uint8_t* __restrict__ out, float* __restrict__ scale
     if (!live[k]) continue;
     // slice 0 stores the scale; a slice whose exchange failed stores it too (NaN: split_row.h)
     if (lt == 0 && (sl == 0 || x_fail != 0)) scales[row[k]] = amax[k] * 0.00787401574803f;
-    const float inv = amax[k] > 0.0f ? mcop_div_rn(127.0f, amax[k]) : 0.0f;
+    const float inv = amax[k] > 0.0f ? row_ratio(127.0f, amax[k]) : 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       if (in_of(v)) {
-        Pack<uint8_t, VEC> q;
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) q.v[e] = q_i8<-128>(a[k][v][e] * inv);
-        st_nt<uint8_t, VEC>(out + row[k] * (int64_t)hidden + lj_of(v), q);
+        const Codes<VEC> q = i8_codes<-128, VEC>(a[k][v], inv);
+        st_codes_nt<VEC>(out + row[k] * (int64_t)hidden + lj_of(v), q);
       }
     }
   }
@@ -190,7 +187,7 @@ k_scale_dynamic_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales
                            const uint16_t* __restrict__ x, const float* __restrict__ sm,
                            int hidden) {
   constexpr int NC = VEC > 1 ? 8 : 16, NL = VEC > 1 ? 8 : 0;
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   __shared__ Pack<uint16_t, VEC> lds[NL > 0 ? NL : 1][kWideLanes];
   const int nvec = hidden / VEC;
   const int tpr = (int)blockDim.x, tid = (int)threadIdx.x;
@@ -230,16 +227,15 @@ k_scale_dynamic_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales
 #pragma unroll
     for (int e = 0; e < VEC; ++e) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[e]));
   }
-  amax = row_reduce(amax, red_max, tpr, MaxOp());
+  amax = row_absmax(amax, red_max, tpr);
   if (threadIdx.x == 0) scales[blockIdx.x] = amax * 0.00787401574803f;
-  const float inv = amax > 0.0f ? mcop_div_rn(127.0f, amax) : 0.0f;
+  const float inv = amax > 0.0f ? row_ratio(127.0f, amax) : 0.0f;
   auto emit = [&](const Pack<uint16_t, VEC>& xv, int64_t o, bool in) {
     float v[VEC];
     v_from(xv, o, v);
-    Pack<uint8_t, VEC> q;
-#pragma unroll
-    for (int e = 0; e < VEC; ++e) q.v[e] = q_i8<-128>(v[e] * inv);
-    if (in) st<uint8_t, VEC>(out + base + o, q);
+    Codes<VEC> q;
+    q = i8_codes<-128, VEC>(v, inv);
+    if (in) st_codes<VEC>(out + base + o, q);
   };
   __asm__ volatile("" : "+v"(lt));
   if ((NC + NL) * tpr <= nvec) {  // the head is whole: no store needs a lane test

@@ -41,13 +41,13 @@ struct WVec {
 // (fp8_quotient_codes; `bounded`: 2^-18 <= s <= 2^100, where the short form is exact); a row
 // whose absmax is 0 has s = 0 and codes 0.
 template <int VEC>
-__device__ __forceinline__ Pack<uint8_t, VEC> sq_fp8_codes(const float* v, float amax, float s,
-                                                           float inv, bool s_ok, bool bounded) {
-  if (amax > 0.0f) return fp8_quotient_codes<VEC>(v, s, inv, s_ok, bounded);
-  Pack<uint8_t, VEC> z;
+__device__ __forceinline__ Codes<VEC> sq_fp8_codes(const float* v, float amax, float s, float inv,
+                                                   bool s_ok, bool bounded) {
+  Codes<VEC> q = fp8_quotient_codes<VEC>(v, s, inv, s_ok, bounded);
+  constexpr int M = (int)(sizeof(q.v) / sizeof(q.v[0]));
 #pragma unroll
-  for (int e = 0; e < VEC; ++e) z.v[e] = 0;
-  return z;
+  for (int k = 0; k < M; ++k) q.v[k] = amax > 0.0f ? q.v[k] : 0;
+  return q;
 }
 
 // The lane's streamed vectors of one row's slice [j0, j0 + jn) (the whole row: 0, nvec): x
@@ -73,10 +73,10 @@ __device__ __forceinline__ void sq_load(const RowPos& p, int j0, int jn,
 template <bool EX>
 struct WgRowReduce {
   double* red_sum;
-  float* red_max;
+  uint32_t* red_max;
   int tpr;
   __device__ __forceinline__ double sum(double v) { return row_reduce<EX>(v, red_sum, tpr, SumOp()); }
-  __device__ __forceinline__ float max(float v) { return row_reduce<EX>(v, red_max, tpr, MaxOp()); }
+  __device__ __forceinline__ float max(float v) { return row_absmax<EX>(v, red_max, tpr); }
 };
 
 // One row (or, for tpr < blockDim, one of the workgroup's rows; or one slice [j0, j0 + jn) of a
@@ -84,12 +84,15 @@ struct WgRowReduce {
 // vectors.  `red` combines the row's partial sum of squares and absmax (WgRowReduce, or the
 // split-row exchange).  UA: the row index is uniform and the row's element offsets fit 32 bits
 // (scalar row base, one 32-bit offset per vector: row_elem<true>).
+// `shared(v, w, s)` gives the lane's v-th weight and smooth vectors: loaded ahead of the row's, or
+// (LATE) when it is called: then they are requested two vectors ahead, and b(a) is held in the
+// dtype until its vector's turn.
 template <class E, class EW, class ES, int VEC, int NV, bool FP8, bool RES, bool EX, bool UA,
-          class Red>
+          bool LATE, class Shared, class Red>
 __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
                                        const Pack<typename E::S, VEC>* xv,
                                        const Pack<typename E::S, VEC>* rv,
-                                       const WVec<EW, VEC>* wv, const WVec<ES, VEC>* sv,
+                                       Shared&& shared,
                                        uint8_t* __restrict__ out, float* __restrict__ scales,
                                        typename E::S* __restrict__ ares,
                                        typename E::S* __restrict__ anorm, int hidden, int tpr,
@@ -97,13 +100,16 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
   using S = typename E::S;
   const int64_t base = p.row * (int64_t)hidden;
 
+  const int slt = EX ? p.lt : store_lane<NV>(p.lt);
   float a[NV][VEC];
+  Pack<S, VEC> z[LATE ? NV : 1];
   double ss = 0.0;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int k = vec_index(v, tpr, p.lt);
+    const int k = vec_index(v, tpr, LATE ? store_lane<8>(slt) : slt);
     const int j = j0 + k;
     const bool in = EX || k < jn;
+    if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
     Pack<S, VEC> o;
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
 #pragma unroll
@@ -115,13 +121,14 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
       vs = __builtin_fma(d, d, vs);
       a[v][e] = E::to_f(o.v[e]);  // b(a): what the later passes of the reference re-read
     }
+    if constexpr (LATE) z[v] = o;
     ss += in ? vs : 0.0;
     if (ares != nullptr && p.live && in) st_nt<S, VEC>(row_elem<UA>(ares, base, (int64_t)j * VEC), o);
   }
 
   ss = red.sum(ss);
-  const float rho = mcop_inv_rms(ss, hidden, eps);
-  const float inv_rho = mcop_div_rn(1.0f, rho);
+  const float rho = row_inv_rms(ss, hidden, eps);
+  const float inv_rho = row_rcp(rho);
   const bool rho_ok = mcop_divisor_ok(rho);
   const bool standard = (flags & MCOP_SQ_STANDARD_NORM) != 0;
   // The literal form: the wave divides in the short form when every lane's elements are in its
@@ -136,6 +143,10 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     float amx = 0.0f;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
+      if constexpr (LATE) {
+        __builtin_amdgcn_sched_barrier(0);
+        widen<E, VEC>(a[v], z[v]);
+      }
 #pragma unroll
       for (int e = 0; e < VEC; ++e) {
         amin = __builtin_fminf(amin, __builtin_fabsf(a[v][e]));
@@ -147,12 +158,35 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     short_div = __builtin_amdgcn_ballot_w64(!in_domain) == 0;
   }
 
+  constexpr int kAhead = 2;
+  WVec<EW, VEC> wb[NV];
+  WVec<ES, VEC> sb[NV];
+  if constexpr (LATE) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < kAhead && v < NV; ++v) shared(v, wb[v], sb[v]);
+  }
   float amax = 0.0f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int k = vec_index(v, tpr, p.lt);
+    const int k = vec_index(v, tpr, LATE ? store_lane<8>(slt) : slt);
     const int j = j0 + k;
     Pack<S, VEC> o;
+    if constexpr (LATE) {
+      __builtin_amdgcn_sched_barrier(0);  // the loads stay kAhead vectors ahead of their use
+      if (v + kAhead < NV) shared(v + kAhead, wb[v + kAhead], sb[v + kAhead]);
+      // opaque: the test above widened it too, and would keep that
+      if constexpr (VEC > 1) {
+        u32x4 u = __builtin_bit_cast(u32x4, z[v]);
+        asm volatile("" : "+v"(u));
+        z[v] = __builtin_bit_cast(Pack<S, VEC>, u);
+      }
+      widen<E, VEC>(a[v], z[v]);
+    } else {
+      shared(v, wb[v], sb[v]);
+    }
+    const WVec<EW, VEC>& wv = wb[v];
+    const WVec<ES, VEC>& sv = sb[v];
     float n[VEC];
     if (standard) {
 #pragma unroll
@@ -164,9 +198,9 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     }
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      const float u = n[e] * wv[v].at(e);
+      const float u = n[e] * wv.at(e);
       o.v[e] = E::from_f(u);
-      const float vv = u * sv[v].at(e);
+      const float vv = u * sv.at(e);
       a[v][e] = vv;
       amax = __builtin_fmaxf(amax, __builtin_fabsf(vv));
     }
@@ -176,25 +210,25 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
   }
   amax = red.max(amax);
 
-  const float s = mcop_div_rn(amax, FP8 ? 448.0f : 127.0f);
+  const float s = row_div<FP8 ? 448 : 127>(amax);
   if (p.live && p.lt == 0) scales[p.row] = s;
-  const float inv = amax > 0.0f ? mcop_div_rn(1.0f, s) : 0.0f;
+  const float inv = amax > 0.0f ? row_rcp(s) : 0.0f;
   const bool s_ok = mcop_divisor_ok(s);
   const bool bounded = s >= 0x1p-18f && s <= 0x1p100f;
 
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int k = vec_index(v, tpr, p.lt);
+    const int k = vec_index(v, tpr, LATE ? store_lane<8>(slt) : slt);
     const int j = j0 + k;
+    if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
     if (p.live && (EX || k < jn)) {
-      Pack<uint8_t, VEC> q;
+      Codes<VEC> q;
       if constexpr (FP8) {
         q = sq_fp8_codes<VEC>(a[v], amax, s, inv, s_ok, bounded);
       } else {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) q.v[e] = q_i8<-127>(a[v][e] * inv);
+        q = i8_codes<-127, VEC>(a[v], inv);
       }
-      st_nt<uint8_t, VEC>(row_elem<UA>(out, base, (int64_t)j * VEC), q);
+      st_codes_nt<VEC>(row_elem<UA>(out, base, (int64_t)j * VEC), q);
     }
   }
 }
@@ -211,28 +245,47 @@ k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
                         typename E::S* __restrict__ anorm, const typename E::S* __restrict__ res,
                         int64_t rows, int hidden, int tpr, float eps, uint32_t flags) {
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   const int nvec = hidden / VEC;
-  WVec<EW, VEC> wv[NV];
-  WVec<ES, VEC> sv[NV];
   RowPos p;
   if constexpr (EX) {
     p = row_pos_one();
   } else {
     p = row_pos(rows, tpr);
   }
-#pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int j = vec_index(v, tpr, p.lt);
+  auto load_shared = [&](int v, WVec<EW, VEC>& w_, WVec<ES, VEC>& s_) {
+    const int j = vec_index(v, tpr, EX ? p.lt : store_lane<NV>(p.lt));
     const int64_t lj = (int64_t)(EX ? j : load_index(j, nvec)) * VEC;
-    wv[v].p = ld<typename EW::S, VEC>(row_elem<EX>(w, 0, lj));
-    sv[v].p = ld<typename ES::S, VEC>(row_elem<EX>(sm, 0, lj));
+    w_.p = ld<typename EW::S, VEC>(row_elem<EX>(w, 0, lj));
+    s_.p = ld<typename ES::S, VEC>(row_elem<EX>(sm, 0, lj));
+  };
+  // With eight or more 16-bit vectors a lane they are loaded after the first reduction, vector by
+  // vector: held from the start they took half the registers (bf16 at eight vectors with fp32
+  // smooth scales: 216 against 163; 2048 rows of 20480 and 32768 ran 81.6 and 98.8 us, now 73.9
+  // and 92.2).  At four they only are for fp16 with both in fp32, which would spend a third
+  // wave's registers on them; bf16 ran 5% slower so.
+  constexpr bool late = !EX && VEC == 8 &&
+                        (NV >= 8 || (NV == 4 && std::is_same_v<E, F16> &&
+                                     sizeof(typename EW::S) + sizeof(typename ES::S) == 8));
+  WVec<EW, VEC> wv[late ? 1 : NV];
+  WVec<ES, VEC> sv[late ? 1 : NV];
+  if constexpr (!late) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) load_shared(v, wv[v], sv[v]);
+    shared_loads_first();
   }
-  shared_loads_first();
+  auto shared = [&](int v, WVec<EW, VEC>& w_, WVec<ES, VEC>& s_) {
+    if constexpr (late) {
+      load_shared(v, w_, s_);
+    } else {
+      w_ = wv[v];
+      s_ = sv[v];
+    }
+  };
   Pack<typename E::S, VEC> xv[NV], rv[NV];
   sq_load<E, VEC, NV, RES, EX>(p, 0, nvec, x, res, hidden, tpr, xv, rv);
   WgRowReduce<EX> red{red_sum, red_max, tpr};
-  sq_row<E, EW, ES, VEC, NV, FP8, RES, EX, EX>(p, 0, nvec, xv, rv, wv, sv, out, scales, ares,
+  sq_row<E, EW, ES, VEC, NV, FP8, RES, EX, EX, late>(p, 0, nvec, xv, rv, shared, out, scales, ares,
                                                 anorm, hidden, tpr, eps, flags, red);
 }
 
@@ -252,7 +305,7 @@ k_rms_norm_smooth_quant_split(uint8_t* __restrict__ out, float* __restrict__ sca
                               int slices, int slice_vecs, float eps, uint32_t flags,
                               uint64_t* __restrict__ ws, int64_t timeout_ticks) {
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   __shared__ double x_sum;
   __shared__ float x_max;
   __shared__ int x_fail;
@@ -266,21 +319,18 @@ k_rms_norm_smooth_quant_split(uint8_t* __restrict__ out, float* __restrict__ sca
   p.live = true;
   const int j0 = sl * slice_vecs;
   const int jn = min(slice_vecs, nvec - j0);
-  WVec<EW, VEC> wv[NV];
-  WVec<ES, VEC> sv[NV];
-#pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int64_t lj = (int64_t)(j0 + load_index(vec_index(v, tpr, p.lt), jn)) * VEC;
-    wv[v].p = ld<typename EW::S, VEC>(row_elem<true>(w, 0, lj));
-    sv[v].p = ld<typename ES::S, VEC>(row_elem<true>(sm, 0, lj));
-  }
-  shared_loads_first();
+  auto shared = [&](int v, WVec<EW, VEC>& w_, WVec<ES, VEC>& s_) {
+    const int64_t lj =
+        (int64_t)(j0 + load_index(vec_index(v, tpr, store_lane<8>(p.lt)), jn)) * VEC;
+    w_.p = ld<typename EW::S, VEC>(row_elem<true>(w, 0, lj));
+    s_.p = ld<typename ES::S, VEC>(row_elem<true>(sm, 0, lj));
+  };
   Pack<typename E::S, VEC> xv[NV], rv[NV];
   sq_load<E, VEC, NV, RES, false, true>(p, j0, jn, x, res, hidden, tpr, xv, rv);
   SplitRowReduce red{red_sum, red_max, tpr, ws, p.row, slices, sl,
                      ws + split_ws_words(rows, slices) - 1, timeout_ticks, &x_sum, &x_max,
                      &x_fail};
-  sq_row<E, EW, ES, VEC, NV, FP8, RES, false, true>(p, j0, jn, xv, rv, wv, sv, out, scales, ares,
+  sq_row<E, EW, ES, VEC, NV, FP8, RES, false, true, true>(p, j0, jn, xv, rv, shared, out, scales, ares,
                                                      anorm, hidden, tpr, eps, flags, red);
   if (red.failed() && p.lt == 0) scales[p.row] = __builtin_nanf("");
 }
@@ -306,7 +356,7 @@ k_rms_norm_smooth_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scal
   // fp8 quotient's correction steps take one vector's worth of registers.
   constexpr int NC = VEC > 1 ? (RES ? 4 : (sizeof(typename EW::S) == 4 || FP8) ? 5 : 6) : 16;
   __shared__ double red_sum[16];
-  __shared__ float red_max[16];
+  __shared__ uint32_t red_max[16];
   const int nvec = hidden / VEC;
   const int tpr = (int)blockDim.x;
   const int64_t base = (int64_t)blockIdx.x * hidden;
@@ -375,15 +425,16 @@ k_rms_norm_smooth_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scal
     for (int e = 0; e < VEC; ++e) ss = __builtin_fma((double)t[e], (double)t[e], ss);
   }
   ss = row_reduce(ss, red_sum, tpr, SumOp());
-  const float rho = mcop_inv_rms(ss, hidden, eps);
-  const float inv_rho = mcop_div_rn(1.0f, rho);
+  const float rho = row_inv_rms(ss, hidden, eps);
+  const float inv_rho = row_rcp(rho);
   const bool rho_ok = mcop_divisor_ok(rho);
   const bool standard = (flags & MCOP_SQ_STANDARD_NORM) != 0;
   // u = (b(a) / rho) * w (or (b(a) * rho) * w), v = u * smooth
   auto uv_of = [&](int64_t o, const float* t, float* u, float* v) {
     float a[VEC], n[VEC];
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) a[e] = rnd<E>(t[e]);
+    for (int e = 0; e < VEC; ++e) a[e] = t[e];
+    rnd_all<E, VEC>(a);
     if (standard) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) n[e] = a[e] * rho;
@@ -419,10 +470,10 @@ k_rms_norm_smooth_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scal
 #pragma unroll
     for (int e = 0; e < VEC; ++e) amax = __builtin_fmaxf(amax, __builtin_fabsf(v[e]));
   }
-  amax = row_reduce(amax, red_max, tpr, MaxOp());
-  const float s = mcop_div_rn(amax, FP8 ? 448.0f : 127.0f);
+  amax = row_absmax(amax, red_max, tpr);
+  const float s = row_div<FP8 ? 448 : 127>(amax);
   if (threadIdx.x == 0) scales[blockIdx.x] = s;
-  const float inv = amax > 0.0f ? mcop_div_rn(1.0f, s) : 0.0f;
+  const float inv = amax > 0.0f ? row_rcp(s) : 0.0f;
   const bool s_ok = mcop_divisor_ok(s);
   const bool bounded = s >= 0x1p-18f && s <= 0x1p100f;
   auto emit = [&](int64_t o, const float* t) {
@@ -436,14 +487,13 @@ k_rms_norm_smooth_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scal
     }
     if (ares != nullptr) st<S, VEC>(ares + base + o, ar);
     if (anorm != nullptr) st<S, VEC>(anorm + base + o, an);
-    Pack<uint8_t, VEC> q;
+    Codes<VEC> q;
     if constexpr (FP8) {
       q = sq_fp8_codes<VEC>(v, amax, s, inv, s_ok, bounded);
     } else {
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) q.v[e] = q_i8<-127>(v[e] * inv);
+      q = i8_codes<-127, VEC>(v, inv);
     }
-    st<uint8_t, VEC>(out + base + o, q);
+    st_codes<VEC>(out + base + o, q);
   };
 #pragma unroll
   for (int c = 0; c < NC + NL; ++c) {
@@ -487,9 +537,15 @@ static void launch_nv(const Geometry& g, const Args& a, hipStream_t st) {
   auto* arp = static_cast<S*>(a.ares);
   auto* anp = static_cast<S*>(a.anorm);
   auto* rp = static_cast<const S*>(a.res);
+  // Four-wave workgroups at four vectors a lane: at most three on a CU, by dynamic LDS that they
+  // do not use (their registers would let four in).  The memory side of this write-heavy row
+  // prefers fewer rows in flight: 16384 x 7168 fp8 143.4 us at three, 145.7 at four; 8192 x 4096
+  // 42.5 and 43.6.
+  const bool cap = VEC > 1 && g.nv == 4 && a.rows > 256 && g.tpr * g.rpb == 256;
+  const unsigned lds = cap ? 44 * 1024 : 0;
 #define MCOP_LAUNCH(NVV, EXX)                                                                   \
   hipLaunchKernelGGL((k_rms_norm_smooth_quant<E, EW, ES, VEC, NVV, FP8, RES, EXX>), grid,      \
-                     block, 0, st, o, a.scales, xp, wp, sp, arp, anp, rp, a.rows, a.hidden,      \
+                     block, lds, st, o, a.scales, xp, wp, sp, arp, anp, rp, a.rows, a.hidden,      \
                      g.tpr, a.eps, a.flags)
   if constexpr (VEC == 1) {
     if (g.nv == 4) MCOP_LAUNCH(4, false); else MCOP_LAUNCH(16, false);
@@ -540,7 +596,9 @@ static int launch_split(const char* name, const Args& a, hipStream_t st) {
   // vectors per CU): 450 us against 469 us at 256 lanes for 2048 x 131072 bf16 fp8
   const SplitKernel k4{reinterpret_cast<const void*>(
                            &k_rms_norm_smooth_quant_split<E, EW, ES, VEC, 4, FP8, RES>), 4, 512};
-  return split_run(name, {k4}, a.rows, a.hidden / VEC, nullptr, st,
+  const SplitKernel k8{reinterpret_cast<const void*>(
+                           &k_rms_norm_smooth_quant_split<E, EW, ES, VEC, 8, FP8, RES>), 8, 256};
+  return split_run(name, {k8, k4}, a.rows, a.hidden / VEC, nullptr, st,
                    [&](int64_t r0, int64_t n, uint64_t* ws, const SplitPlan& p, auto launch) {
     const int64_t off = r0 * (int64_t)a.hidden;
     auto* o = static_cast<uint8_t*>(a.out) + off;

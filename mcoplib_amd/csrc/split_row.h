@@ -220,7 +220,7 @@ __device__ __forceinline__ void split_max2(uint64_t* slots, int slices, int sl, 
 // then the row's workgroups through the workspace (split_sum, split_max).
 struct SplitRowReduce {
   double* red_sum;
-  float* red_max;
+  uint32_t* red_max;
   int tpr;
   uint64_t* ws;
   int64_t row;
@@ -232,12 +232,12 @@ struct SplitRowReduce {
   float* x_max;
   int* x_fail = nullptr;  // LDS: 1 after an exchange that failed (nullptr: not recorded)
   __device__ __forceinline__ double sum(double v) {
-    v = row_reduce<true>(v, red_sum, tpr, SumOp());
+    v = row_reduce<true, false>(v, red_sum, tpr, SumOp());
     return split_sum(split_slots(ws, row, slices, 0), slices, sl, kSplitTag, v, err,
                      timeout_ticks, x_sum, x_fail);
   }
   __device__ __forceinline__ float max(float v) {
-    v = row_reduce<true>(v, red_max, tpr, MaxOp());
+    v = row_absmax<true, false>(v, red_max, tpr);
     return split_max(split_slots(ws, row, slices, 1), slices, sl, kSplitTag, v, err,
                      timeout_ticks, x_max, x_fail);
   }
