@@ -147,11 +147,12 @@ static bool valid_tpr(int64_t t, int min_tpr) {
 bool row_fits(int64_t hidden, int vec, KernelOfNv kernels, int min_tpr) {
   static const int kVecNv[] = {1, 2, 4, 8, 16};
   static const int kScalarNv[] = {4, 16};
-  const int64_t nvec = hidden / vec;
+  const int64_t nvec = ceil_div(hidden, vec);
   const int* cands = vec > 1 ? kVecNv : kScalarNv;
   const int ncand = vec > 1 ? 5 : 2;
   for (int c = 0; c < ncand; ++c) {
     if (row_lanes(ceil_div(nvec, cands[c]), min_tpr) > max_tpr(vec, cands[c])) continue;
+    if (kernels(cands[c]) == nullptr) continue;
     if (!kernel_info(kernels(cands[c])).spills) return true;
   }
   return false;
@@ -277,7 +278,7 @@ bool wide_rows_ok(const char* op, int64_t rows) {
 
 bool choose_geometry(const char* op, int64_t rows, int64_t hidden, int vec, KernelOfNv kernels,
                      Geometry* g, int min_tpr, bool wide_nv4) {
-  const int64_t nvec = hidden / vec;
+  const int64_t nvec = ceil_div(hidden, vec);
   int nv = 0;
   int64_t tpr = 0;
   const int onv = g_over_nv;
@@ -286,7 +287,8 @@ bool choose_geometry(const char* op, int64_t rows, int64_t hidden, int vec, Kern
                                   : (onv == 4 || onv == 16);
   if (nv_allowed) {
     const int64_t t = otpr > 0 ? otpr : row_lanes(ceil_div(nvec, onv), min_tpr);
-    if (valid_tpr(t, min_tpr) && t <= max_tpr(vec, onv) && (int64_t)onv * t >= nvec) {
+    if (valid_tpr(t, min_tpr) && t <= max_tpr(vec, onv) && (int64_t)onv * t >= nvec &&
+        kernels(onv) != nullptr) {
       nv = onv;
       tpr = t;
     }
@@ -304,6 +306,7 @@ bool choose_geometry(const char* op, int64_t rows, int64_t hidden, int vec, Kern
       const int64_t t = row_lanes(ceil_div(nvec, cand), min_tpr);
       if (t > max_tpr(vec, cand)) continue;
       if (vec > 1 && cand == 1 && nvec > 64) continue;
+      if (kernels(cand) == nullptr) continue;
       if (kernel_info(kernels(cand)).spills) continue;
       if (fallback_nv == 0) {
         fallback_nv = cand;

@@ -29,19 +29,20 @@ namespace mcop {
 // two registers, so its rows take the generic form.
 // EX (exact): one row per workgroup and every lane in the row (tpr == blockDim.x, NV * tpr ==
 // hidden / VEC): uniform row index, scalar base addresses with 32-bit offsets, no bounds tests.
-template <class E, int NV, bool EX>
+template <class E, int NV, int FORM>
 __host__ __device__ constexpr int h1_waves() {
-  if (NV != 8 || std::is_same<E, F16>::value) return 1;
-  if (!EX) return 4;
+  if (NV != 8 || FORM == FORM_RAGGED || std::is_same<E, F16>::value) return 1;
+  if (FORM != FORM_EXACT) return 4;
   return std::is_same<E, F32>::value ? 5 : 1;
 }
-template <class E, int VEC, int NV, bool EX = false>
+template <class E, int VEC, int NV, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
-__attribute__((amdgpu_waves_per_eu(h1_waves<E, NV, EX>())))
+__attribute__((amdgpu_waves_per_eu(h1_waves<E, NV, FORM>())))
 k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
                      typename E::S* __restrict__ res, const typename E::S* __restrict__ w,
                      int64_t rows, int hidden, int tpr, float eps) {
   using S = typename E::S;
+  constexpr bool EX = FORM == FORM_EXACT;
   __shared__ double red_sum[16];
   RowPos p;
   if constexpr (EX) {
@@ -49,12 +50,12 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
   } else {
     p = row_pos(rows, tpr);
   }
-  const int nvec = hidden / VEC;
+  const int nvec = vec_count<FORM, VEC>(hidden);
+  const bool apart = FORM == FORM_RAGGED && vec_apart(nvec, tpr);
   const int64_t xbase = p.row * x_stride, xlbase = p.lrow * x_stride;
   const int64_t rbase = p.row * (int64_t)hidden, rlbase = p.lrow * (int64_t)hidden;
   auto lj_of = [&](int v) {
-    const int j = vec_index(v, tpr, p.lt);
-    return (int64_t)(EX ? j : load_index(j, nvec)) * VEC;
+    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), nvec, hidden);
   };
 
   Pack<S, VEC> xv[NV], rv[NV], wv[NV];
@@ -62,13 +63,13 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
   // are summed (the latency falls into the reduction): all three at once spill.
   constexpr int w_early = NV >= 16 && std::is_same<E, F16>::value ? 12 : NV;
 #pragma unroll
-  for (int v = 0; v < w_early; ++v) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj_of(v)));
+  for (int v = 0; v < w_early; ++v) wv[v] = ldf<FORM, S, VEC>(row_elem<true>(w, 0, lj_of(v)));
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int64_t lj = lj_of(v);
-    xv[v] = ld_nt<S, VEC>(row_elem<EX>(x, xlbase, lj));
-    rv[v] = ld_nt<S, VEC>(row_elem<EX>(res, rlbase, lj));
+    xv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(x, xlbase, lj));
+    rv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(res, rlbase, lj));
   }
 
   const int slt = EX ? p.lt : store_lane<NV>(p.lt);
@@ -78,6 +79,9 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, slt);
     const bool in = EX || j < nvec;
+    const int skip = vec_skip<FORM, VEC>(j, hidden);
+    trim<FORM>(xv[v], skip, apart);
+    trim<FORM>(rv[v], skip, apart);
     Pack<S, VEC> o;
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
 #pragma unroll
@@ -88,8 +92,9 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
       const double d = (double)t;
       vs = __builtin_fma(d, d, vs);
     }
+    vs = own_squares<FORM, E, VEC, false>(vs, o, o, skip);
     ss += in ? vs : 0.0;
-    if (p.live && in) st_nt<S, VEC>(row_elem<EX>(res, rbase, (int64_t)j * VEC), o);
+    if (p.live && in) stf_nt<FORM>(row_elem<EX>(res, rbase, (int64_t)j * VEC - skip), o, skip, apart);
   }
 
   if constexpr (w_early < NV) {
@@ -105,8 +110,9 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, slt);
     if (p.live && (EX || j < nvec)) {
-      st_nt<S, VEC>(row_elem<EX>(x, xbase, (int64_t)j * VEC),
-                    norm_store<E, VEC>(z[v], rho, wv[v]));
+      const int skip = vec_skip<FORM, VEC>(j, hidden);
+      stf_nt<FORM>(row_elem<EX>(x, xbase, (int64_t)j * VEC - skip),
+                   norm_store<E, VEC>(z[v], rho, wv[v]), skip, apart);
     }
   }
 }
@@ -319,7 +325,7 @@ k_fused_add_rms_norm_wide(typename E::S* __restrict__ x, int64_t x_stride,
   }
 }
 
-template <class E, int VEC>
+template <class E, int VEC, bool RAG = false>
 static void launch_nv(const Geometry& g, void* x, int64_t xs, void* res, const void* w,
                       int64_t rows, int hidden, float eps, hipStream_t st) {
   using S = typename E::S;
@@ -331,7 +337,14 @@ static void launch_nv(const Geometry& g, void* x, int64_t xs, void* res, const v
   hipLaunchKernelGGL((k_fused_add_rms_norm<E, VEC, NVV, EXX>), grid, block, 0, st, xp, xs, rp, wp, \
                      rows, hidden, g.tpr, eps)
   if constexpr (VEC == 1) {
-    if (g.nv == 4) MCOP_LAUNCH(4, false); else MCOP_LAUNCH(16, false);
+    MCOP_LAUNCH(4, FORM_ROWS);
+  } else if constexpr (RAG) {
+    switch (g.nv) {
+      case 1: MCOP_LAUNCH(1, FORM_RAGGED); break;
+      case 2: MCOP_LAUNCH(2, FORM_RAGGED); break;
+      case 4: MCOP_LAUNCH(4, FORM_RAGGED); break;
+      default: MCOP_LAUNCH(8, FORM_RAGGED); break;
+    }
   } else {
     // exact rows (one row per workgroup, every lane in it): the EX form at two vectors a lane,
     // and at four or eight on the latency path (at most 256 rows)
@@ -339,24 +352,37 @@ static void launch_nv(const Geometry& g, void* x, int64_t xs, void* res, const v
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == hidden / VEC &&
                     (g.nv == 2 || rows <= 256);
 #define MCOP_EX(NVV) \
-  (ex && exact_form_ok(reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, VEC, NVV, true>)))
+  (ex && exact_form_ok(reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, VEC, NVV, FORM_EXACT>)))
     switch (g.nv) {
-      case 1: MCOP_LAUNCH(1, false); break;
-      case 2: if (MCOP_EX(2)) MCOP_LAUNCH(2, true); else MCOP_LAUNCH(2, false); break;
-      case 4: if (MCOP_EX(4)) MCOP_LAUNCH(4, true); else MCOP_LAUNCH(4, false); break;
-      case 8: if (MCOP_EX(8)) MCOP_LAUNCH(8, true); else MCOP_LAUNCH(8, false); break;
-      default: MCOP_LAUNCH(16, false); break;
+      case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
+      case 2:
+        if (MCOP_EX(2)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        break;
+      case 4:
+        if (MCOP_EX(4)) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
+        break;
+      case 8:
+        if (MCOP_EX(8)) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
+        break;
+      default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
 #undef MCOP_EX
   }
 #undef MCOP_LAUNCH
 }
 
-template <class E, int VEC>
+template <class E, int VEC, bool RAG = false>
 static const void* kernel_of(int nv) {
   if constexpr (VEC == 1) {
-    return nv == 4 ? reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, 1, 4>)
-                   : reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, 1, 16>);
+    return nv == 4 ? reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, 1, 4>) : nullptr;
+  } else if constexpr (RAG) {
+    switch (nv) {
+      case 1: return reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, VEC, 1, FORM_RAGGED>);
+      case 2: return reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, VEC, 2, FORM_RAGGED>);
+      case 4: return reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, VEC, 4, FORM_RAGGED>);
+      case 8: return reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, VEC, 8, FORM_RAGGED>);
+      default: return nullptr;
+    }
   } else {
     switch (nv) {
       case 1: return reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, VEC, 1>);
@@ -396,8 +422,13 @@ static int dispatch(void* x, int64_t xs, void* res, const void* w, int64_t rows,
                     float eps, hipStream_t st) {
   constexpr int V = E::VEC;
   const bool vec_ok = hidden % V == 0 && xs % V == 0 && aligned(16, x, res, w);
-  const KernelOfNv kernels = vec_ok ? &kernel_of<E, V> : &kernel_of<E, 1>;
-  if (!row_fits(hidden, vec_ok ? V : 1, kernels)) {
+  // any other row of at least one vector takes the ragged form, narrower ones one element a load
+  const bool rag = !vec_ok && hidden >= V;
+  const int vec = vec_ok || rag ? V : 1;
+  const KernelOfNv kernels = vec_ok ? &kernel_of<E, V>
+                             : rag  ? &kernel_of<E, V, true>
+                                    : &kernel_of<E, 1>;
+  if (!row_fits(hidden, vec, kernels)) {
     if (vec_ok && split_rows_enabled()) {
       const int rc = launch_split<E, V>(x, xs, res, w, rows, (int)hidden, eps, st);
       if (rc != MCOP_E_UNSUPPORTED) return rc;
@@ -417,11 +448,13 @@ static int dispatch(void* x, int64_t xs, void* res, const void* w, int64_t rows,
     return check_launch("fused_add_rms_norm");
   }
   Geometry g;
-  if (!choose_geometry("fused_add_rms_norm", rows, hidden, vec_ok ? V : 1, kernels, &g)) {
+  if (!choose_geometry("fused_add_rms_norm", rows, hidden, vec, kernels, &g)) {
     return MCOP_E_UNSUPPORTED;
   }
   if (g.vec == 1) {
     launch_nv<E, 1>(g, x, xs, res, w, rows, (int)hidden, eps, st);
+  } else if (rag) {
+    launch_nv<E, V, true>(g, x, xs, res, w, rows, (int)hidden, eps, st);
   } else {
     launch_nv<E, V>(g, x, xs, res, w, rows, (int)hidden, eps, st);
   }

@@ -105,13 +105,14 @@ __device__ __forceinline__ Pack<typename E::S, VEC> norm_out(const float* a,
 
 // EX (exact): one row per workgroup and every lane in the row (tpr == blockDim.x, NV * tpr ==
 // hidden / VEC): uniform row index, scalar base addresses with 32-bit offsets, no bounds tests.
-template <class E, class EW, int VEC, int NV, bool RES, bool EX = false>
+template <class E, class EW, int VEC, int NV, bool RES, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
 k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
            const typename E::S* __restrict__ x, const typename EW::S* __restrict__ w,
            const typename E::S* __restrict__ res, RowMap map, int64_t rows, int hidden, int tpr,
            float eps, int mode, int rms_div) {
   using S = typename E::S;
+  constexpr bool EX = FORM == FORM_EXACT;
   __shared__ double red_sum[16];
   RowPos p;
   if constexpr (EX) {
@@ -119,28 +120,27 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
   } else {
     p = row_pos(rows, tpr);
   }
-  const int nvec = hidden / VEC;
+  const int nvec = vec_count<FORM, VEC>(hidden);
   const RowOffsets lo = row_offsets(map, p.lrow);
   const int64_t out_base = p.row == p.lrow ? lo.out : 0;
   const int64_t rbase = p.row * (int64_t)hidden;
   const int64_t lrbase = p.lrow * (int64_t)hidden;
   auto lj_of = [&](int v) {
-    const int j = vec_index(v, tpr, p.lt);
-    return (int64_t)(EX ? j : load_index(j, nvec)) * VEC;
+    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), nvec, hidden);
   };
 
   Pack<S, VEC> xv[NV], rv[NV];
   NormW<EW, VEC> wv[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    wv[v].p = ld<typename EW::S, VEC>(row_elem<EX>(w, lo.w, lj_of(v)));
+    wv[v].p = ldf<FORM, typename EW::S, VEC>(row_elem<EX>(w, lo.w, lj_of(v)));
   }
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int64_t lj = lj_of(v);
-    xv[v] = ld_nt<S, VEC>(row_elem<EX>(x, lo.in, lj));
-    if constexpr (RES) rv[v] = ld_nt<S, VEC>(row_elem<EX>(res, lrbase, lj));
+    xv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(x, lo.in, lj));
+    if constexpr (RES) rv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(res, lrbase, lj));
   }
 
   float a[NV][VEC];
@@ -149,6 +149,7 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
     const bool in = EX || j < nvec;
+    const int skip = vec_skip<FORM, VEC>(j, hidden);
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
     Pack<S, VEC> o;
 #pragma unroll
@@ -164,9 +165,12 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
       }
       a[v][e] = t;
     }
+    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], skip);
     ss += in ? vs : 0.0;
     if constexpr (RES) {
-      if (p.live && in) st_nt<S, VEC>(row_elem<EX>(ares, rbase, (int64_t)j * VEC), o);
+      if (p.live && in) {
+        stf_nt<FORM>(row_elem<EX>(ares, rbase, (int64_t)j * VEC - skip), o);
+      }
     }
   }
   ss = row_reduce<EX>(ss, red_sum, tpr, SumOp());
@@ -223,7 +227,8 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(n[e] * wv[v].at(e));
     }
-    st_nt<S, VEC>(row_elem<EX>(out, out_base, (int64_t)j * VEC), o);
+    const int skip = vec_skip<FORM, VEC>(j, hidden);
+    stf_nt<FORM>(row_elem<EX>(out, out_base, (int64_t)j * VEC - skip), o);
   }
 }
 
@@ -475,7 +480,7 @@ struct NormArgs {
   int rms_div;
 };
 
-template <class E, class EW, int VEC, bool RES>
+template <class E, class EW, int VEC, bool RES, bool RAG = false>
 static void norm_launch_nv(const Geometry& g, const NormArgs& a, hipStream_t st) {
   using S = typename E::S;
   const dim3 grid((unsigned)g.blocks), block((unsigned)(g.tpr * g.rpb));
@@ -488,31 +493,51 @@ static void norm_launch_nv(const Geometry& g, const NormArgs& a, hipStream_t st)
   hipLaunchKernelGGL((k_rms_norm<E, EW, VEC, NVV, RES, EXX>), grid, block, 0, st, o, arp, xp, wp, \
                      rp, a.map, a.rows, a.hidden, g.tpr, a.eps, a.mode, a.rms_div)
   if constexpr (VEC == 1) {
-    if (g.nv == 4) MCOP_LAUNCH(4, false); else MCOP_LAUNCH(16, false);
+    MCOP_LAUNCH(4, FORM_ROWS);
+  } else if constexpr (RAG) {
+    switch (g.nv) {
+      case 1: MCOP_LAUNCH(1, FORM_RAGGED); break;
+      case 2: MCOP_LAUNCH(2, FORM_RAGGED); break;
+      case 4: MCOP_LAUNCH(4, FORM_RAGGED); break;
+      default: MCOP_LAUNCH(8, FORM_RAGGED); break;
+    }
   } else {
     // exact rows (one row per workgroup, every lane in it): the EX form at two vectors a lane,
     // and at four or eight on the latency path (at most 256 rows), when it keeps its registers
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == a.hidden / VEC &&
                     (g.nv == 2 || a.rows <= 256);
 #define MCOP_EX(NVV)                                                                           \
-  (ex && exact_form_ok(reinterpret_cast<const void*>(&k_rms_norm<E, EW, VEC, NVV, RES, true>)))
+  (ex && exact_form_ok(reinterpret_cast<const void*>(&k_rms_norm<E, EW, VEC, NVV, RES, FORM_EXACT>)))
     switch (g.nv) {
-      case 1: MCOP_LAUNCH(1, false); break;
-      case 2: if (MCOP_EX(2)) MCOP_LAUNCH(2, true); else MCOP_LAUNCH(2, false); break;
-      case 4: if (MCOP_EX(4)) MCOP_LAUNCH(4, true); else MCOP_LAUNCH(4, false); break;
-      case 8: if (MCOP_EX(8)) MCOP_LAUNCH(8, true); else MCOP_LAUNCH(8, false); break;
-      default: MCOP_LAUNCH(16, false); break;
+      case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
+      case 2:
+        if (MCOP_EX(2)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        break;
+      case 4:
+        if (MCOP_EX(4)) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
+        break;
+      case 8:
+        if (MCOP_EX(8)) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
+        break;
+      default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
 #undef MCOP_EX
   }
 #undef MCOP_LAUNCH
 }
 
-template <class E, class EW, int VEC, bool RES>
+template <class E, class EW, int VEC, bool RES, bool RAG = false>
 static const void* norm_kernel_of(int nv) {
   if constexpr (VEC == 1) {
-    return nv == 4 ? reinterpret_cast<const void*>(&k_rms_norm<E, EW, 1, 4, RES>)
-                   : reinterpret_cast<const void*>(&k_rms_norm<E, EW, 1, 16, RES>);
+    return nv == 4 ? reinterpret_cast<const void*>(&k_rms_norm<E, EW, 1, 4, RES>) : nullptr;
+  } else if constexpr (RAG) {
+    switch (nv) {
+      case 1: return reinterpret_cast<const void*>(&k_rms_norm<E, EW, VEC, 1, RES, FORM_RAGGED>);
+      case 2: return reinterpret_cast<const void*>(&k_rms_norm<E, EW, VEC, 2, RES, FORM_RAGGED>);
+      case 4: return reinterpret_cast<const void*>(&k_rms_norm<E, EW, VEC, 4, RES, FORM_RAGGED>);
+      case 8: return reinterpret_cast<const void*>(&k_rms_norm<E, EW, VEC, 8, RES, FORM_RAGGED>);
+      default: return nullptr;
+    }
   } else {
     switch (nv) {
       case 1: return reinterpret_cast<const void*>(&k_rms_norm<E, EW, VEC, 1, RES>);
@@ -571,10 +596,14 @@ static int norm_dispatch(const char* name, const NormArgs& a, hipStream_t st) {
   constexpr int V = E::VEC;
   const bool vec_ok = norm_vec_ok<E, EW>(a);
   const bool r = a.res != nullptr;
+  // any other row of at least one vector takes the ragged form, narrower ones one element a load
+  const bool rag = !vec_ok && a.hidden >= V;
+  const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels =
       vec_ok ? (r ? &norm_kernel_of<E, EW, V, true> : &norm_kernel_of<E, EW, V, false>)
+      : rag  ? (r ? &norm_kernel_of<E, EW, V, true, true> : &norm_kernel_of<E, EW, V, false, true>)
              : (r ? &norm_kernel_of<E, EW, 1, true> : &norm_kernel_of<E, EW, 1, false>);
-  if (!row_fits(a.hidden, vec_ok ? V : 1, kernels)) {
+  if (!row_fits(a.hidden, vec, kernels)) {
     if (vec_ok && split_rows_enabled()) {
       const int rc = r ? norm_launch_split<E, EW, V, true>(name, a, st)
                        : norm_launch_split<E, EW, V, false>(name, a, st);
@@ -600,12 +629,15 @@ static int norm_dispatch(const char* name, const NormArgs& a, hipStream_t st) {
     return check_launch(name);
   }
   Geometry g;
-  if (!choose_geometry(name, a.rows, a.hidden, vec_ok ? V : 1, kernels, &g)) {
+  if (!choose_geometry(name, a.rows, a.hidden, vec, kernels, &g)) {
     return MCOP_E_UNSUPPORTED;
   }
   if (g.vec == 1) {
     if (r) norm_launch_nv<E, EW, 1, true>(g, a, st);
     else norm_launch_nv<E, EW, 1, false>(g, a, st);
+  } else if (rag) {
+    if (r) norm_launch_nv<E, EW, V, true, true>(g, a, st);
+    else norm_launch_nv<E, EW, V, false, true>(g, a, st);
   } else {
     if (r) norm_launch_nv<E, EW, V, true>(g, a, st);
     else norm_launch_nv<E, EW, V, false>(g, a, st);

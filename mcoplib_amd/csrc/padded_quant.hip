@@ -30,7 +30,7 @@ namespace mcop {
 
 // EX (exact): one row per workgroup and every lane in the row (tpr == blockDim.x, NV * tpr ==
 // hidden / VEC): uniform row index, scalar base addresses with 32-bit offsets, no bounds tests.
-template <int VEC, int NV, bool OPT, bool EX = false>
+template <int VEC, int NV, bool OPT, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
 k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__ rms,
                             uint8_t* __restrict__ q_out, float* __restrict__ scales,
@@ -38,6 +38,7 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
                             const uint16_t* __restrict__ w, int64_t rows, int hidden,
                             int64_t pad_bytes, int tpr, float eps) {
   using E = BF16;
+  constexpr bool EX = FORM == FORM_EXACT;
   __shared__ double red_sum[16];
   __shared__ uint32_t red_max[16];
   RowPos p;
@@ -46,24 +47,24 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
   } else {
     p = row_pos(rows, tpr);
   }
-  const int nvec = hidden / VEC;
+  const int nvec = vec_count<FORM, VEC>(hidden);
+  const bool apart = FORM == FORM_RAGGED && vec_apart(nvec, tpr);
   const int64_t base = p.row * (int64_t)hidden;
   const int64_t lbase = p.lrow * (int64_t)hidden;
   const int64_t pbase = p.row * pad_bytes;
   auto lj_of = [&](int v) {
-    const int j = vec_index(v, tpr, p.lt);
-    return (int64_t)(EX ? j : load_index(j, nvec)) * VEC;
+    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), nvec, hidden);
   };
 
   Pack<uint16_t, VEC> xv[NV], rv[NV], wv[NV];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) wv[v] = ld<uint16_t, VEC>(row_elem<true>(w, 0, lj_of(v)));
+  for (int v = 0; v < NV; ++v) wv[v] = ldf<FORM, uint16_t, VEC>(row_elem<true>(w, 0, lj_of(v)));
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int64_t lj = lj_of(v);
-    xv[v] = ld_nt<uint16_t, VEC>(row_elem<EX>(x, lbase, lj));
-    rv[v] = ld_nt<uint16_t, VEC>(row_elem<EX>(res, lbase, lj));
+    xv[v] = ldf_nt<FORM, uint16_t, VEC>(row_elem<EX>(x, lbase, lj));
+    rv[v] = ldf_nt<FORM, uint16_t, VEC>(row_elem<EX>(res, lbase, lj));
   }
 
   // a: opt keeps p = a * w (fp32); generic keeps b(a) (the residual value it re-reads)
@@ -75,6 +76,9 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
     const bool in = EX || j < nvec;
+    const int skip = vec_skip<FORM, VEC>(j, hidden);
+    trim<FORM>(xv[v], skip, apart);
+    trim<FORM>(rv[v], skip, apart);
     double vs = 0.0;
     float m[VEC];
     Pack<uint16_t, VEC> o;
@@ -97,8 +101,9 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
     for (int e = 0; e < VEC; ++e) {
       amax = __builtin_fmaxf(amax, (full || in) ? __builtin_fabsf(m[e]) : 0.0f);
     }
+    vs = own_squares<FORM, E, VEC, true>(vs, xv[v], rv[v], skip);
     ss += in ? vs : 0.0;
-    if (p.live && in) st_nt<uint16_t, VEC>(row_elem<EX>(res, base, (int64_t)j * VEC), o);
+    if (p.live && in) stf_nt<FORM>(row_elem<EX>(res, base, (int64_t)j * VEC - skip), o, skip, apart);
   }
   ss = row_reduce<EX>(ss, red_sum, tpr, SumOp());
   amax = row_absmax<EX>(amax, red_max, tpr);
@@ -130,9 +135,11 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
         widen<E, VEC>(a[v], o);
       }
       const Codes<VEC> q = i8_codes<-127, VEC>(a[v], inv);
-      st_nt<uint16_t, VEC>(row_elem<EX>(rms, base, (int64_t)j * VEC), o);
-      st_codes_nt<VEC>(row_elem<EX>(q_out, base, (int64_t)j * VEC), q);
-      st_codes_nt<VEC>(row_elem<EX>(padded, pbase, (int64_t)j * VEC), q);
+      const int skip = vec_skip<FORM, VEC>(j, hidden);
+      const int64_t at = (int64_t)j * VEC - skip;
+      stf_nt<FORM>(row_elem<EX>(rms, base, at), o, skip, apart);
+      stf_codes_nt<FORM, VEC>(row_elem<EX>(q_out, base, at), q, skip, apart);
+      stf_codes_nt<FORM, VEC>(row_elem<EX>(padded, pbase, at), q, skip, apart);
     }
   }
 }
@@ -338,11 +345,18 @@ k_add_rms_norm_quant_padded_wide(uint8_t* __restrict__ padded, uint16_t* __restr
   }
 }
 
-template <int VEC, bool OPT>
+template <int VEC, bool OPT, bool RAG = false>
 static const void* kernel_of(int nv) {
   if constexpr (VEC == 1) {
-    return nv == 4 ? reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<1, 4, OPT>)
-                   : reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<1, 16, OPT>);
+    return nv == 4 ? reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<1, 4, OPT>) : nullptr;
+  } else if constexpr (RAG) {
+    switch (nv) {
+      case 1: return reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<VEC, 1, OPT, FORM_RAGGED>);
+      case 2: return reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<VEC, 2, OPT, FORM_RAGGED>);
+      case 4: return reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<VEC, 4, OPT, FORM_RAGGED>);
+      case 8: return reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<VEC, 8, OPT, FORM_RAGGED>);
+      default: return nullptr;
+    }
   } else {
     switch (nv) {
       case 1: return reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<VEC, 1, OPT>);
@@ -368,7 +382,7 @@ struct PadArgs {
   float eps;
 };
 
-template <int VEC, bool OPT>
+template <int VEC, bool OPT, bool RAG = false>
 static void launch_nv(const Geometry& g, const PadArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)g.blocks), block((unsigned)(g.tpr * g.rpb));
 #define MCOP_LAUNCH(NVV, EXX)                                                                  \
@@ -376,20 +390,33 @@ static void launch_nv(const Geometry& g, const PadArgs& a, hipStream_t st) {
                      a.padded, a.rms, a.q, a.scales, a.x, a.res, a.w, a.rows, a.hidden,       \
                      a.pad_bytes, g.tpr, a.eps)
   if constexpr (VEC == 1) {
-    if (g.nv == 4) MCOP_LAUNCH(4, false); else MCOP_LAUNCH(16, false);
+    MCOP_LAUNCH(4, FORM_ROWS);
+  } else if constexpr (RAG) {
+    switch (g.nv) {
+      case 1: MCOP_LAUNCH(1, FORM_RAGGED); break;
+      case 2: MCOP_LAUNCH(2, FORM_RAGGED); break;
+      case 4: MCOP_LAUNCH(4, FORM_RAGGED); break;
+      default: MCOP_LAUNCH(8, FORM_RAGGED); break;
+    }
   } else {
     // exact rows (one row per workgroup, every lane in it) on the latency path (at most 256
     // rows) take the EX form, when it keeps its registers
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == a.hidden / VEC && a.rows <= 256;
 #define MCOP_EX(NVV)                                                                           \
   (ex && exact_form_ok(                                                                        \
-             reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<VEC, NVV, OPT, true>)))
+             reinterpret_cast<const void*>(&k_add_rms_norm_quant_padded<VEC, NVV, OPT, FORM_EXACT>)))
     switch (g.nv) {
-      case 1: MCOP_LAUNCH(1, false); break;
-      case 2: if (MCOP_EX(2)) MCOP_LAUNCH(2, true); else MCOP_LAUNCH(2, false); break;
-      case 4: if (MCOP_EX(4)) MCOP_LAUNCH(4, true); else MCOP_LAUNCH(4, false); break;
-      case 8: if (MCOP_EX(8)) MCOP_LAUNCH(8, true); else MCOP_LAUNCH(8, false); break;
-      default: MCOP_LAUNCH(16, false); break;
+      case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
+      case 2:
+        if (MCOP_EX(2)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        break;
+      case 4:
+        if (MCOP_EX(4)) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
+        break;
+      case 8:
+        if (MCOP_EX(8)) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
+        break;
+      default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
 #undef MCOP_EX
   }
@@ -426,8 +453,14 @@ static int dispatch(const PadArgs& a, hipStream_t st) {
   const char* name = "fused_add_rms_norm_dynamic_per_token_quant_padding_output";
   const bool vec_ok = a.hidden % 8 == 0 && a.pad_bytes % 8 == 0 &&
                       aligned(16, a.x, a.res, a.w, a.rms) && aligned(8, a.q, a.padded);
+  // any other row of at least one vector takes the ragged form, narrower ones one element a load
+  const bool rag = !vec_ok && a.hidden >= 8;
+  const int vec = vec_ok || rag ? 8 : 1;
+  const KernelOfNv kernels = vec_ok ? &kernel_of<8, OPT>
+                             : rag  ? &kernel_of<8, OPT, true>
+                                    : &kernel_of<1, OPT>;
   if constexpr (!OPT) {
-    if (!row_fits(a.hidden, vec_ok ? 8 : 1, vec_ok ? &kernel_of<8, OPT> : &kernel_of<1, OPT>)) {
+    if (!row_fits(a.hidden, vec, kernels)) {
       if (vec_ok && split_rows_enabled()) {
         const int rc = launch_split(name, a, st);
         if (rc != MCOP_E_UNSUPPORTED) return rc;
@@ -445,11 +478,11 @@ static int dispatch(const PadArgs& a, hipStream_t st) {
     }
   }
   Geometry g;
-  if (!choose_geometry(name, a.rows, a.hidden, vec_ok ? 8 : 1,
-                       vec_ok ? &kernel_of<8, OPT> : &kernel_of<1, OPT>, &g)) {
+  if (!choose_geometry(name, a.rows, a.hidden, vec, kernels, &g)) {
     return MCOP_E_UNSUPPORTED;
   }
   if (g.vec == 1) launch_nv<1, OPT>(g, a, st);
+  else if (rag) launch_nv<8, OPT, true>(g, a, st);
   else launch_nv<8, OPT>(g, a, st);
   return check_launch(name);
 }

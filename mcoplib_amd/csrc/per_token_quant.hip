@@ -129,12 +129,13 @@ __device__ __forceinline__ void ptq_fold(float t, float& mx, float& nmn) {
 
 // EX (exact): one row per workgroup and every lane in the row (tpr == blockDim.x, NV * tpr ==
 // hidden / VEC): uniform row index, scalar base addresses with 32-bit offsets, no bounds tests.
-template <class E, int VEC, int NV, int MODE, bool EX = false>
+template <class E, int VEC, int NV, int MODE, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
 k_per_token_quant(uint8_t* __restrict__ out, float* __restrict__ scales, int32_t* __restrict__ azp,
                   const typename E::S* __restrict__ x, const float* __restrict__ scale_ub,
                   int64_t rows, int hidden, int64_t in_stride, int64_t out_stride, int tpr) {
   using S = typename E::S;
+  constexpr bool EX = FORM == FORM_EXACT;
   __shared__ float red_a[16];
   __shared__ float red_b[16];
   RowPos p;
@@ -143,7 +144,7 @@ k_per_token_quant(uint8_t* __restrict__ out, float* __restrict__ scales, int32_t
   } else {
     p = row_pos(rows, tpr);
   }
-  const int nvec = hidden / VEC;
+  const int nvec = vec_count<FORM, VEC>(hidden);
   const int64_t lbase = p.lrow * in_stride;
   const int64_t obase = p.row * out_stride;
 
@@ -151,9 +152,9 @@ k_per_token_quant(uint8_t* __restrict__ out, float* __restrict__ scales, int32_t
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
-    xv[v] = ld_nt<S, VEC>(row_elem<EX>(x, lbase, (int64_t)(EX ? j : load_index(j, nvec)) * VEC));
+    xv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(x, lbase, vec_off<FORM, VEC>(j, nvec, hidden)));
   }
-  // Lanes past the row end hold a copy of vector 0 (read only: no effect on max or min).
+  // Elements past the row end are copies of the row's (read only: no effect on max or min).
   float a[NV][VEC];
   float mx = MODE == PTQ_INT8_AZP ? -__builtin_inff() : 0.0f;
   float nmn = -__builtin_inff();  // max of -v, i.e. -(min v)
@@ -176,7 +177,9 @@ k_per_token_quant(uint8_t* __restrict__ out, float* __restrict__ scales, int32_t
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
     if (p.live && (EX || j < nvec)) {
-      st_codes_nt<VEC>(row_elem<EX>(out, obase, (int64_t)j * VEC), ptq_codes<E, VEC, MODE>(a[v], r));
+      const int skip = vec_skip<FORM, VEC>(j, hidden);
+      stf_codes_nt<FORM, VEC>(row_elem<EX>(out, obase, (int64_t)j * VEC - skip),
+                              ptq_codes<E, VEC, MODE>(a[v], r));
     }
   }
 }
@@ -326,11 +329,18 @@ k_per_token_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales,
   }
 }
 
-template <class E, int VEC, int MODE>
+template <class E, int VEC, int MODE, bool RAG = false>
 static const void* kernel_of(int nv) {
   if constexpr (VEC == 1) {
-    return nv == 4 ? reinterpret_cast<const void*>(&k_per_token_quant<E, 1, 4, MODE>)
-                   : reinterpret_cast<const void*>(&k_per_token_quant<E, 1, 16, MODE>);
+    return nv == 4 ? reinterpret_cast<const void*>(&k_per_token_quant<E, 1, 4, MODE>) : nullptr;
+  } else if constexpr (RAG) {
+    switch (nv) {
+      case 1: return reinterpret_cast<const void*>(&k_per_token_quant<E, VEC, 1, MODE, FORM_RAGGED>);
+      case 2: return reinterpret_cast<const void*>(&k_per_token_quant<E, VEC, 2, MODE, FORM_RAGGED>);
+      case 4: return reinterpret_cast<const void*>(&k_per_token_quant<E, VEC, 4, MODE, FORM_RAGGED>);
+      case 8: return reinterpret_cast<const void*>(&k_per_token_quant<E, VEC, 8, MODE, FORM_RAGGED>);
+      default: return nullptr;
+    }
   } else {
     switch (nv) {
       case 1: return reinterpret_cast<const void*>(&k_per_token_quant<E, VEC, 1, MODE>);
@@ -354,7 +364,7 @@ struct PtqArgs {
   int64_t out_stride;
 };
 
-template <class E, int VEC, int MODE>
+template <class E, int VEC, int MODE, bool RAG = false>
 static void launch_nv(const Geometry& g, const PtqArgs& a, hipStream_t st) {
   using S = typename E::S;
   const dim3 grid((unsigned)g.blocks), block((unsigned)(g.tpr * g.rpb));
@@ -364,20 +374,33 @@ static void launch_nv(const Geometry& g, const PtqArgs& a, hipStream_t st) {
   hipLaunchKernelGGL((k_per_token_quant<E, VEC, NVV, MODE, EXX>), grid, block, 0, st, o, a.scales, \
                      a.azp, xp, a.scale_ub, a.rows, a.hidden, a.in_stride, a.out_stride, g.tpr)
   if constexpr (VEC == 1) {
-    if (g.nv == 4) MCOP_LAUNCH(4, false); else MCOP_LAUNCH(16, false);
+    MCOP_LAUNCH(4, FORM_ROWS);
+  } else if constexpr (RAG) {
+    switch (g.nv) {
+      case 1: MCOP_LAUNCH(1, FORM_RAGGED); break;
+      case 2: MCOP_LAUNCH(2, FORM_RAGGED); break;
+      case 4: MCOP_LAUNCH(4, FORM_RAGGED); break;
+      default: MCOP_LAUNCH(8, FORM_RAGGED); break;
+    }
   } else {
     // exact rows (one row per workgroup, every lane in it): the EX form at two vectors a lane,
     // and at four or eight on the latency path (at most 256 rows), when it keeps its registers
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == a.hidden / VEC &&
                     (g.nv == 2 || a.rows <= 256);
 #define MCOP_EX(NVV)                                                                           \
-  (ex && exact_form_ok(reinterpret_cast<const void*>(&k_per_token_quant<E, VEC, NVV, MODE, true>)))
+  (ex && exact_form_ok(reinterpret_cast<const void*>(&k_per_token_quant<E, VEC, NVV, MODE, FORM_EXACT>)))
     switch (g.nv) {
-      case 1: MCOP_LAUNCH(1, false); break;
-      case 2: if (MCOP_EX(2)) MCOP_LAUNCH(2, true); else MCOP_LAUNCH(2, false); break;
-      case 4: if (MCOP_EX(4)) MCOP_LAUNCH(4, true); else MCOP_LAUNCH(4, false); break;
-      case 8: if (MCOP_EX(8)) MCOP_LAUNCH(8, true); else MCOP_LAUNCH(8, false); break;
-      default: MCOP_LAUNCH(16, false); break;
+      case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
+      case 2:
+        if (MCOP_EX(2)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        break;
+      case 4:
+        if (MCOP_EX(4)) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
+        break;
+      case 8:
+        if (MCOP_EX(8)) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
+        break;
+      default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
 #undef MCOP_EX
   }
@@ -414,8 +437,13 @@ static int dispatch(const char* name, const PtqArgs& a, hipStream_t st) {
   constexpr int V = E::VEC;
   const bool vec_ok = a.hidden % V == 0 && a.in_stride % V == 0 && a.out_stride % V == 0 &&
                       aligned(16, a.x) && aligned(V, a.out);
-  const KernelOfNv kernels = vec_ok ? &kernel_of<E, V, MODE> : &kernel_of<E, 1, MODE>;
-  if (!row_fits(a.hidden, vec_ok ? V : 1, kernels)) {
+  // any other row of at least one vector takes the ragged form, narrower ones one element a load
+  const bool rag = !vec_ok && a.hidden >= V;
+  const int vec = vec_ok || rag ? V : 1;
+  const KernelOfNv kernels = vec_ok ? &kernel_of<E, V, MODE>
+                             : rag  ? &kernel_of<E, V, MODE, true>
+                                    : &kernel_of<E, 1, MODE>;
+  if (!row_fits(a.hidden, vec, kernels)) {
     if (vec_ok && split_rows_enabled()) {
       const int rc = launch_split<E, V, MODE>(name, a, st);
       if (rc != MCOP_E_UNSUPPORTED) return rc;
@@ -435,10 +463,11 @@ static int dispatch(const char* name, const PtqArgs& a, hipStream_t st) {
     return check_launch(name);
   }
   Geometry g;
-  if (!choose_geometry(name, a.rows, a.hidden, vec_ok ? V : 1, kernels, &g)) {
+  if (!choose_geometry(name, a.rows, a.hidden, vec, kernels, &g)) {
     return MCOP_E_UNSUPPORTED;
   }
   if (g.vec == 1) launch_nv<E, 1, MODE>(g, a, st);
+  else if (rag) launch_nv<E, V, MODE, true>(g, a, st);
   else launch_nv<E, V, MODE>(g, a, st);
   return check_launch(name);
 }

@@ -87,14 +87,15 @@ __device__ __forceinline__ Codes<VEC> row_codes(const float* y, float rho, float
 // so the row's base addresses are scalar and each vector's 32-bit offset serves every tensor,
 // and the bounds tests and the out-of-row handling drop out: a shorter per-row chain (measured
 // 12% less per decode call at T = 1-64 x 5120, about 0.5% at 8192 x 8192).
-template <class E, int VEC, int NV, bool FP8, bool RES, int MODE, bool EX = false>
+template <class E, int VEC, int NV, bool FP8, bool RES, int MODE, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
-__attribute__((amdgpu_waves_per_eu(NV == 8 && !EX && !FP8 && std::is_same<E, BF16>::value ? 4 : 1)))
+__attribute__((amdgpu_waves_per_eu(NV == 8 && FORM == FORM_ROWS && !FP8 && std::is_same<E, BF16>::value ? 4 : 1)))
 k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
                  const typename E::S* __restrict__ x, const typename E::S* __restrict__ w,
                  const float* __restrict__ scale_ub, typename E::S* __restrict__ res,
                  int64_t rows, int hidden, int tpr, float eps) {
   using S = typename E::S;
+  constexpr bool EX = FORM == FORM_EXACT;
   __shared__ double red_sum[16];
   __shared__ uint32_t red_max[16];
   RowPos p;
@@ -103,28 +104,28 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   } else {
     p = row_pos(rows, tpr);
   }
-  const int nvec = hidden / VEC;
+  const int nvec = vec_count<FORM, VEC>(hidden);
+  const bool apart = FORM == FORM_RAGGED && vec_apart(nvec, tpr);
   const int64_t base = p.lrow * (int64_t)hidden;  // the lane's row, where it stores at all
   auto lj_of = [&](int v) {  // element offset of the lane's vector v (loads)
-    const int j = vec_index(v, tpr, p.lt);
-    return (int64_t)(EX ? j : load_index(j, nvec)) * VEC;
+    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), nvec, hidden);
   };
 
   // All loads first, unconditionally (out-of-row lanes re-read vector 0 of their row).
   Pack<S, VEC> xv[NV], rv[NV], wv[NV];
   if constexpr (NV >= 4) {
 #pragma unroll
-    for (int v = 0; v < NV; ++v) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj_of(v)));
+    for (int v = 0; v < NV; ++v) wv[v] = ldf<FORM, S, VEC>(row_elem<true>(w, 0, lj_of(v)));
     shared_loads_first();
   }
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int64_t lj = lj_of(v);
-    xv[v] = ld_nt<S, VEC>(row_elem<EX>(x, base, lj));
-    if constexpr (RES) rv[v] = ld_nt<S, VEC>(row_elem<EX>(res, base, lj));
+    xv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(x, base, lj));
+    if constexpr (RES) rv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(res, base, lj));
     // with fewer vectors per lane the weight loads interleave with the streamed ones (measured
     // 1.5% faster at 8192 x 8192, two vectors per lane; shared-first won at four)
-    if constexpr (NV < 4) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj));
+    if constexpr (NV < 4) wv[v] = ldf<FORM, S, VEC>(row_elem<true>(w, 0, lj));
   }
 
   const int slt = store_lane<NV>(p.lt);
@@ -134,6 +135,11 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, slt);
     const bool in = EX || j < nvec;
+    const int skip = vec_skip<FORM, VEC>(j, hidden);
+    if constexpr (RES) {
+      trim<FORM>(xv[v], skip, apart);
+      trim<FORM>(rv[v], skip, apart);
+    }
     // Lanes past the row end hold a copy of vector 0: it must not count in the sum.
     double vs = 0.0;
 #pragma unroll
@@ -144,13 +150,14 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
       const double d = (double)t;
       vs = __builtin_fma(d, d, vs);
     }
+    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], skip);
     ss += in ? vs : 0.0;
     if constexpr (RES) {
       if (p.live && in) {
         Pack<S, VEC> o;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(a[v][e]);
-        st_nt<S, VEC>(row_elem<EX>(res, base, (int64_t)j * VEC), o);
+        stf_nt<FORM>(row_elem<EX>(res, base, (int64_t)j * VEC - skip), o, skip, apart);
       }
     }
   }
@@ -188,7 +195,9 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     if (p.live && (EX || j < nvec)) {
       const Codes<VEC> q =
           row_codes<E, VEC, FP8, MODE>(a[v], rho, s, inv, s_ok, bounded, scale_ub != nullptr);
-      st_codes_nt<VEC>(row_elem<EX>(out, base, (int64_t)j * VEC), q);
+      const int skip = vec_skip<FORM, VEC>(j, hidden);
+      stf_codes_nt<FORM, VEC>(row_elem<EX>(out, base, (int64_t)j * VEC - skip), q, skip,
+                              RES && apart);
     }
   }
 }
@@ -479,7 +488,7 @@ static int launch_split(const char* name, void* out, float* scales, const void* 
   });
 }
 
-template <class E, int VEC, bool FP8, bool RES, int MODE>
+template <class E, int VEC, bool FP8, bool RES, int MODE, bool RAG = false>
 static void launch_nv(const Geometry& g, void* out, float* scales, const void* x, const void* w,
                       const float* scale_ub, void* res, int64_t rows, int hidden, float eps,
                       hipStream_t st) {
@@ -493,7 +502,14 @@ static void launch_nv(const Geometry& g, void* out, float* scales, const void* x
   hipLaunchKernelGGL((k_rms_norm_quant<E, VEC, NVV, FP8, RES, MODE, EXX>), grid, block, 0, st, o, \
                      scales, xp, wp, scale_ub, rp, rows, hidden, g.tpr, eps)
   if constexpr (VEC == 1) {
-    if (g.nv == 4) MCOP_LAUNCH(4, false); else MCOP_LAUNCH(16, false);
+    MCOP_LAUNCH(4, FORM_ROWS);
+  } else if constexpr (RAG) {
+    switch (g.nv) {
+      case 1: MCOP_LAUNCH(1, FORM_RAGGED); break;
+      case 2: MCOP_LAUNCH(2, FORM_RAGGED); break;
+      case 4: MCOP_LAUNCH(4, FORM_RAGGED); break;
+      default: MCOP_LAUNCH(8, FORM_RAGGED); break;
+    }
   } else {
     // exact rows (one row per workgroup, every lane in it) take the EX form at two vectors a
     // lane, and at four or eight for at most 256 rows (the latency path): at four and eight it
@@ -506,23 +522,38 @@ static void launch_nv(const Geometry& g, void* out, float* scales, const void* x
 #define MCOP_EX(NVV, EXX)                                                                      \
   (ex && exact_form_ok(                                                                        \
              reinterpret_cast<const void*>(&k_rms_norm_quant<E, VEC, NVV, FP8, RES, MODE, EXX>)))
+    constexpr int kWideForm = wide_ex ? FORM_EXACT : FORM_ROWS;
     switch (g.nv) {
-      case 1: MCOP_LAUNCH(1, false); break;
-      case 2: if (MCOP_EX(2, true)) MCOP_LAUNCH(2, true); else MCOP_LAUNCH(2, false); break;
-      case 4: if (MCOP_EX(4, wide_ex)) MCOP_LAUNCH(4, wide_ex); else MCOP_LAUNCH(4, false); break;
-      case 8: if (MCOP_EX(8, wide_ex)) MCOP_LAUNCH(8, wide_ex); else MCOP_LAUNCH(8, false); break;
-      default: MCOP_LAUNCH(16, false); break;
+      case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
+      case 2:
+        if (MCOP_EX(2, FORM_EXACT)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        break;
+      case 4:
+        if (MCOP_EX(4, kWideForm)) MCOP_LAUNCH(4, kWideForm); else MCOP_LAUNCH(4, FORM_ROWS);
+        break;
+      case 8:
+        if (MCOP_EX(8, kWideForm)) MCOP_LAUNCH(8, kWideForm); else MCOP_LAUNCH(8, FORM_ROWS);
+        break;
+      default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
 #undef MCOP_EX
   }
 #undef MCOP_LAUNCH
 }
 
-template <class E, int VEC, bool FP8, bool RES, int MODE>
+template <class E, int VEC, bool FP8, bool RES, int MODE, bool RAG = false>
 static const void* kernel_of(int nv) {
+  auto fn = [](auto k) { return reinterpret_cast<const void*>(k); };
   if constexpr (VEC == 1) {
-    return nv == 4 ? reinterpret_cast<const void*>(&k_rms_norm_quant<E, 1, 4, FP8, RES, MODE>)
-                   : reinterpret_cast<const void*>(&k_rms_norm_quant<E, 1, 16, FP8, RES, MODE>);
+    return nv == 4 ? fn(&k_rms_norm_quant<E, 1, 4, FP8, RES, MODE>) : nullptr;
+  } else if constexpr (RAG) {
+    switch (nv) {
+      case 1: return fn(&k_rms_norm_quant<E, VEC, 1, FP8, RES, MODE, FORM_RAGGED>);
+      case 2: return fn(&k_rms_norm_quant<E, VEC, 2, FP8, RES, MODE, FORM_RAGGED>);
+      case 4: return fn(&k_rms_norm_quant<E, VEC, 4, FP8, RES, MODE, FORM_RAGGED>);
+      case 8: return fn(&k_rms_norm_quant<E, VEC, 8, FP8, RES, MODE, FORM_RAGGED>);
+      default: return nullptr;
+    }
   } else {
     switch (nv) {
       case 1: return reinterpret_cast<const void*>(&k_rms_norm_quant<E, VEC, 1, FP8, RES, MODE>);
@@ -542,11 +573,16 @@ static int dispatch(const char* name, void* out, float* scales, const void* x, c
                     hipStream_t st, uint64_t* scratch = nullptr) {
   constexpr int V = E::VEC;
   const bool vec_ok = hidden % V == 0 && aligned(16, x, w, res) && aligned(V, out);
+  // any other row of at least one vector takes the ragged form, narrower ones one element a load
+  const bool rag = !vec_ok && hidden >= V;
+  const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels =
       vec_ok ? (res ? &kernel_of<E, V, FP8, true, MODE> : &kernel_of<E, V, FP8, false, MODE>)
+      : rag  ? (res ? &kernel_of<E, V, FP8, true, MODE, true>
+                    : &kernel_of<E, V, FP8, false, MODE, true>)
              : (res ? &kernel_of<E, 1, FP8, true, MODE> : &kernel_of<E, 1, FP8, false, MODE>);
   if constexpr (MODE != QM_MC_7168) {
-    if (!row_fits(hidden, vec_ok ? V : 1, kernels)) {
+    if (!row_fits(hidden, vec, kernels)) {
       if (vec_ok && split_rows_enabled()) {
         const int rc =
             res ? launch_split<E, V, FP8, true, MODE>(name, out, scales, x, w, scale_ub, res,
@@ -575,7 +611,7 @@ static int dispatch(const char* name, void* out, float* scales, const void* x, c
     }
   }
   Geometry g;
-  if (!choose_geometry(name, rows, hidden, vec_ok ? V : 1, kernels, &g, 16,
+  if (!choose_geometry(name, rows, hidden, vec, kernels, &g, 16,
                        /*wide_nv4=*/false)) {
     return MCOP_E_UNSUPPORTED;
   }
@@ -583,6 +619,9 @@ static int dispatch(const char* name, void* out, float* scales, const void* x, c
   if (g.vec == 1) {
     if (res) launch_nv<E, 1, FP8, true, MODE>(g, out, scales, x, w, scale_ub, res, rows, h, eps, st);
     else launch_nv<E, 1, FP8, false, MODE>(g, out, scales, x, w, scale_ub, res, rows, h, eps, st);
+  } else if (rag) {
+    if (res) launch_nv<E, V, FP8, true, MODE, true>(g, out, scales, x, w, scale_ub, res, rows, h, eps, st);
+    else launch_nv<E, V, FP8, false, MODE, true>(g, out, scales, x, w, scale_ub, res, rows, h, eps, st);
   } else {
     if (res) launch_nv<E, V, FP8, true, MODE>(g, out, scales, x, w, scale_ub, res, rows, h, eps, st);
     else launch_nv<E, V, FP8, false, MODE>(g, out, scales, x, w, scale_ub, res, rows, h, eps, st);

@@ -179,6 +179,126 @@ __device__ __forceinline__ void widen(float* f, const Pack<typename E::S, N>& p)
 }
 
 // ---------------------------------------------------------------------------------------------
+// Forms of a register kernel.
+//   FORM_ROWS    16-byte vectors, all tensors and rows aligned to them
+//   FORM_EXACT   the same, one row a workgroup and every lane in it
+//   FORM_RAGGED  16-byte vectors at element alignment: rows of any width >= VEC, any row stride or
+//                base address (global memory takes unaligned vectors).  A row has ceil(hidden /
+//                VEC) vectors; the last one, if it is not whole, is the row's last VEC elements, so
+//                every access stays inside the row.  Its first `skip` elements belong to the
+//                vector before: they are left out of sums, give the same maxima, and are stored
+//                twice with the same bits.  A kernel that stores over its inputs must read those
+//                elements before their owner stores them: both are in one wave's instruction,
+//                whose loads end before its stores begin, unless the last vector starts a wave's
+//                run of lanes (`apart`); then they are read as zeros and not stored.
+// Before, one element a load: 2048 x 5137 fp8 with a residual 28.3 us, 20.7 so; 4096 x 4099 norm
+// with a residual 58.5 and 35.5; 65536 x 67 norm 13.0 and 8.2; 4096 x 30001 int8 521 and 223.
+enum Form { FORM_ROWS = 0, FORM_EXACT = 1, FORM_RAGGED = 2 };
+
+template <int FORM, int VEC>
+__device__ __forceinline__ int vec_count(int hidden) {
+  return FORM == FORM_RAGGED ? (int)(((unsigned)hidden + (VEC - 1)) / VEC) : hidden / VEC;
+}
+
+// Element offset a lane's loads of vector j use; vectors past the row end re-read one of the row.
+template <int FORM, int VEC>
+__device__ __forceinline__ int64_t vec_off(int j, int nvec, int hidden) {
+  if constexpr (FORM == FORM_EXACT) return (int64_t)j * VEC;
+  if constexpr (FORM == FORM_RAGGED) return min(j * VEC, hidden - VEC);
+  return (int64_t)(j < nvec ? j : 0) * VEC;
+}
+
+// Leading elements of the lane's vector j that are not its own (VEC or more past the row end).
+template <int FORM, int VEC>
+__device__ __forceinline__ int vec_skip(int j, int hidden) {
+  if constexpr (FORM != FORM_RAGGED) return 0;
+  return max(j * VEC - (hidden - VEC), 0);
+}
+
+typedef u32x4 u32x4_loose __attribute__((aligned(1)));
+typedef u32x2 u32x2_loose __attribute__((aligned(1)));
+template <int B> struct LooseOf;
+template <> struct LooseOf<8> { using T = u32x2_loose; };
+template <> struct LooseOf<16> { using T = u32x4_loose; };
+
+// Load / streaming load of one vector in a kernel's form.
+template <int FORM, class T, int N>
+__device__ __forceinline__ Pack<T, N> ldf(const T* p) {
+  if constexpr (FORM != FORM_RAGGED) {
+    return ld<T, N>(p);
+  } else {
+    Pack<T, N> v;
+    __builtin_memcpy(&v, p, sizeof(v));
+    return v;
+  }
+}
+template <int FORM, class T, int N>
+__device__ __forceinline__ Pack<T, N> ldf_nt(const T* p) {
+  if constexpr (FORM != FORM_RAGGED) {
+    return ld_nt<T, N>(p);
+  } else {
+    using R = typename LooseOf<(int)sizeof(T) * N>::T;
+    using A = typename RawOf<(int)sizeof(T) * N>::T;
+    const A a = __builtin_nontemporal_load(reinterpret_cast<const R*>(p));
+    return __builtin_bit_cast(Pack<T, N>, a);
+  }
+}
+
+// Whether the row's last vector is apart from the one before (above): uniform over the row.
+__device__ __forceinline__ bool vec_apart(int nvec, int tpr) {
+  return ((nvec - 1) & ((tpr < 64 ? tpr : 64) - 1)) == 0;
+}
+
+// Zeroes a vector's elements that are not its own, where the last vector is apart.
+template <int FORM, class T, int N>
+__device__ __forceinline__ void trim(Pack<T, N>& p, int skip, bool apart) {
+  if constexpr (FORM == FORM_RAGGED) {
+    if (apart && __builtin_amdgcn_ballot_w64(skip > 0) != 0) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) p.v[e] = e < skip ? T(0) : p.v[e];
+    }
+  }
+}
+
+// Streaming store of one vector in a kernel's form: `p` is the address of the vector as loaded.
+template <int FORM, class T, int N>
+__device__ __forceinline__ void stf_nt(T* p, const Pack<T, N>& v, int skip = 0,
+                                       bool apart = false) {
+  if constexpr (FORM != FORM_RAGGED) {
+    st_nt<T, N>(p, v);
+  } else if (!apart || skip == 0) {
+    using R = typename LooseOf<(int)sizeof(T) * N>::T;
+    using A = typename RawOf<(int)sizeof(T) * N>::T;
+    __builtin_nontemporal_store(__builtin_bit_cast(A, v), reinterpret_cast<R*>(p));
+  } else {
+#pragma unroll
+    for (int e = 1; e < N; ++e) {
+      if (e >= skip) p[e] = v.v[e];
+    }
+  }
+}
+
+// The sum of squares `vs` of a vector's values without the elements that are not its own (behind
+// a wave-uniform branch: only the wave with the row's last vector has any).
+template <int FORM, class E, int N, bool RES>
+__device__ __forceinline__ double own_squares(double vs, const Pack<typename E::S, N>& x,
+                                              const Pack<typename E::S, N>& r, int skip) {
+  if constexpr (FORM == FORM_RAGGED) {
+    if (__builtin_amdgcn_ballot_w64(skip > 0) != 0) {
+      vs = 0.0;
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        float t = E::to_f(x.v[e]);
+        if constexpr (RES) t += E::to_f(r.v[e]);
+        const double d = e < skip ? 0.0 : (double)t;
+        vs = __builtin_fma(d, d, vs);
+      }
+    }
+  }
+  return vs;
+}
+
+// ---------------------------------------------------------------------------------------------
 // Quantizers.
 
 // rne(v) converted to int32 by the hardware conversion, whose results are defined for every
@@ -210,6 +330,27 @@ template <int N>
 __device__ __forceinline__ void st_codes_nt(uint8_t* p, const Codes<N>& q) {
   if constexpr (N % 4 == 0) st_nt<uint32_t, N / 4>(reinterpret_cast<uint32_t*>(p), q);
   else st_nt<uint8_t, N>(p, q);
+}
+
+// The same in a kernel's form (as stf_nt).
+template <int FORM, int N>
+__device__ __forceinline__ void stf_codes_nt(uint8_t* p, const Codes<N>& q, int skip = 0,
+                                             bool apart = false) {
+  if constexpr (FORM != FORM_RAGGED) {
+    st_codes_nt<N>(p, q);
+  } else if (!apart || skip == 0) {
+    if constexpr (N == 8) {
+      __builtin_nontemporal_store(__builtin_bit_cast(u32x2, q),
+                                  reinterpret_cast<u32x2_loose*>(p));
+    } else {
+      __builtin_memcpy(p, &q, N);
+    }
+  } else {
+#pragma unroll
+    for (int e = 1; e < N; ++e) {
+      if (e >= skip) p[e] = code_of<N>(q, e);
+    }
+  }
 }
 
 // The low bytes of N words as codes, four to a dword by three byte permutes.
@@ -680,7 +821,8 @@ struct Geometry {
   int64_t blocks;
 };
 
-// The kernel instantiation used for a given number of vectors per lane (for occupancy queries).
+// The kernel instantiation used for a given number of vectors per lane (for occupancy queries);
+// NULL where there is none (the ragged forms have one to eight, the element-wise ones four).
 using KernelOfNv = const void* (*)(int nv);
 
 // Picks the launch shape of a row kernel. `vec` is 1 or the 16-byte vector width.  Returns false,

@@ -23,13 +23,13 @@ constexpr int kSdqSplitRows = 2;
 // The smooth scales are fp32, two loads per 16-byte input vector; even as cache hits they took
 // 20% of the kernel's time in a compute-free model of this access pattern at 16384 x 7168, and
 // sharing them between two rows recovers about half of that.
-template <int VEC, int NV, int R>
+template <int VEC, int NV, int R, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
 k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
                       const uint16_t* __restrict__ x, const float* __restrict__ sm, int64_t rows,
                       int hidden, int tpr) {
   __shared__ uint32_t red_max[16 * R];
-  const int nvec = hidden / VEC;
+  const int nvec = vec_count<FORM, VEC>(hidden);
   RowPos p[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) p[k] = row_pos_of(rows, tpr, k, R);
@@ -37,8 +37,8 @@ k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   Pack<float, VEC> sv[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    sv[v] = ld<float, VEC>(
-        row_elem<true>(sm, 0, (int64_t)load_index(vec_index(v, tpr, p[0].lt), nvec) * VEC));
+    sv[v] = ldf<FORM, float, VEC>(
+        row_elem<true>(sm, 0, vec_off<FORM, VEC>(vec_index(v, tpr, p[0].lt), nvec, hidden)));
   }
   shared_loads_first();
   Pack<uint16_t, VEC> xv[R][NV];
@@ -46,14 +46,15 @@ k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   for (int k = 0; k < R; ++k) {
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      xv[k][v] = ld_nt<uint16_t, VEC>(x + p[k].lrow * (int64_t)hidden +
-                                      (int64_t)load_index(vec_index(v, tpr, p[k].lt), nvec) * VEC);
+      xv[k][v] = ldf_nt<FORM, uint16_t, VEC>(
+          x + p[k].lrow * (int64_t)hidden +
+          vec_off<FORM, VEC>(vec_index(v, tpr, p[k].lt), nvec, hidden));
     }
   }
 
   float a[R][NV][VEC];
   float amax[R];
-  // Lanes past the row end hold a copy of vector 0, which does not change the max.
+  // Elements past the row end are copies of the row's, which do not change the max.
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     amax[k] = 0.0f;
@@ -80,7 +81,8 @@ k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
       const int j = vec_index(v, tpr, p[k].lt);
       if (p[k].live && j < nvec) {
         const Codes<VEC> q = i8_codes<-128, VEC>(a[k][v], inv);
-        st_codes_nt<VEC>(out + base + (int64_t)j * VEC, q);
+        const int skip = vec_skip<FORM, VEC>(j, hidden);
+        stf_codes_nt<FORM, VEC>(out + base + (int64_t)j * VEC - skip, q);
       }
     }
   }
@@ -259,17 +261,18 @@ static int rows_per_lane(const Geometry& g, int64_t rows) {
   return g.vec > 1 && g.nv <= 4 && rows >= 2048 ? 2 : 1;
 }
 
-template <int VEC>
+template <int VEC, bool RAG = false>
 static void launch_nv(const Geometry& g, int8_t* out, float* scales, const void* x,
                       const float* sm, int64_t rows, int hidden, hipStream_t st) {
   const dim3 block((unsigned)(g.tpr * g.rpb));
   auto* o = reinterpret_cast<uint8_t*>(out);
   auto* xp = static_cast<const uint16_t*>(x);
+  constexpr int FORM = RAG ? FORM_RAGGED : FORM_ROWS;
   if constexpr (VEC > 1) {
     if (rows_per_lane(g, rows) == 2) {
       const dim3 grid((unsigned)((rows + 2 * g.rpb - 1) / (2 * g.rpb)));
 #define MCOP_LAUNCH(NVV)                                                                       \
-  hipLaunchKernelGGL((k_scale_dynamic_quant<VEC, NVV, 2>), grid, block, 0, st, o, scales, xp,   \
+  hipLaunchKernelGGL((k_scale_dynamic_quant<VEC, NVV, 2, FORM>), grid, block, 0, st, o, scales, xp,   \
                      sm, rows, hidden, g.tpr)
       switch (g.nv) {
         case 1: MCOP_LAUNCH(1); break;
@@ -282,10 +285,17 @@ static void launch_nv(const Geometry& g, int8_t* out, float* scales, const void*
   }
   const dim3 grid((unsigned)g.blocks);
 #define MCOP_LAUNCH(NVV)                                                                       \
-  hipLaunchKernelGGL((k_scale_dynamic_quant<VEC, NVV, 1>), grid, block, 0, st, o, scales, xp,   \
+  hipLaunchKernelGGL((k_scale_dynamic_quant<VEC, NVV, 1, FORM>), grid, block, 0, st, o, scales, xp,   \
                      sm, rows, hidden, g.tpr)
   if constexpr (VEC == 1) {
-    if (g.nv == 4) MCOP_LAUNCH(4); else MCOP_LAUNCH(16);
+    MCOP_LAUNCH(4);
+  } else if constexpr (RAG) {
+    switch (g.nv) {
+      case 1: MCOP_LAUNCH(1); break;
+      case 2: MCOP_LAUNCH(2); break;
+      case 4: MCOP_LAUNCH(4); break;
+      default: MCOP_LAUNCH(8); break;
+    }
   } else {
     switch (g.nv) {
       case 1: MCOP_LAUNCH(1); break;
@@ -298,11 +308,18 @@ static void launch_nv(const Geometry& g, int8_t* out, float* scales, const void*
 #undef MCOP_LAUNCH
 }
 
-template <int VEC>
+template <int VEC, bool RAG = false>
 static const void* kernel_of(int nv) {
   if constexpr (VEC == 1) {
-    return nv == 4 ? reinterpret_cast<const void*>(&k_scale_dynamic_quant<1, 4, 1>)
-                   : reinterpret_cast<const void*>(&k_scale_dynamic_quant<1, 16, 1>);
+    return nv == 4 ? reinterpret_cast<const void*>(&k_scale_dynamic_quant<1, 4, 1>) : nullptr;
+  } else if constexpr (RAG) {
+    switch (nv) {
+      case 1: return reinterpret_cast<const void*>(&k_scale_dynamic_quant<VEC, 1, 1, FORM_RAGGED>);
+      case 2: return reinterpret_cast<const void*>(&k_scale_dynamic_quant<VEC, 2, 1, FORM_RAGGED>);
+      case 4: return reinterpret_cast<const void*>(&k_scale_dynamic_quant<VEC, 4, 1, FORM_RAGGED>);
+      case 8: return reinterpret_cast<const void*>(&k_scale_dynamic_quant<VEC, 8, 1, FORM_RAGGED>);
+      default: return nullptr;
+    }
   } else {
     switch (nv) {
       case 1: return reinterpret_cast<const void*>(&k_scale_dynamic_quant<VEC, 1, 1>);
@@ -363,8 +380,11 @@ extern "C" int mcop_scale_dynamic_quant(int8_t* out, float* scales, const void* 
   constexpr int V = BF16::VEC;
   const bool vec_ok = hidden_size % V == 0 && aligned(16, input, smooth) && aligned(V, out);
   auto st = static_cast<hipStream_t>(stream);
-  const KernelOfNv kernels = vec_ok ? &kernel_of<V> : &kernel_of<1>;
-  if (!row_fits(hidden_size, vec_ok ? V : 1, kernels)) {
+  // any other row of at least one vector takes the ragged form, narrower ones one element a load
+  const bool rag = !vec_ok && hidden_size >= V;
+  const int vec = vec_ok || rag ? V : 1;
+  const KernelOfNv kernels = vec_ok ? &kernel_of<V> : rag ? &kernel_of<V, true> : &kernel_of<1>;
+  if (!row_fits(hidden_size, vec, kernels)) {
     auto* o = reinterpret_cast<uint8_t*>(out);
     auto* xp = static_cast<const uint16_t*>(input);
     if (vec_ok && split_rows_enabled()) {
@@ -382,12 +402,13 @@ extern "C" int mcop_scale_dynamic_quant(int8_t* out, float* scales, const void* 
     return check_launch("scale_dynamic_quant");
   }
   Geometry g;
-  if (!choose_geometry("scale_dynamic_quant", num_tokens, hidden_size, vec_ok ? V : 1, kernels,
-                       &g)) {
+  if (!choose_geometry("scale_dynamic_quant", num_tokens, hidden_size, vec, kernels, &g)) {
     return MCOP_E_UNSUPPORTED;
   }
   if (g.vec == 1) {
     launch_nv<1>(g, out, scales, input, smooth, num_tokens, (int)hidden_size, st);
+  } else if (rag) {
+    launch_nv<V, true>(g, out, scales, input, smooth, num_tokens, (int)hidden_size, st);
   } else {
     launch_nv<V>(g, out, scales, input, smooth, num_tokens, (int)hidden_size, st);
   }

@@ -52,7 +52,7 @@ __device__ __forceinline__ Codes<VEC> sq_fp8_codes(const float* v, float amax, f
 
 // The lane's streamed vectors of one row's slice [j0, j0 + jn) (the whole row: 0, nvec): x
 // (and the residual); lanes past the slice end load its first vector.
-template <class E, int VEC, int NV, bool RES, bool EX, bool UA = EX>
+template <class E, int VEC, int NV, bool RES, bool EX, bool UA = EX, int FORM = FORM_ROWS>
 __device__ __forceinline__ void sq_load(const RowPos& p, int j0, int jn,
                                         const typename E::S* __restrict__ x,
                                         const typename E::S* __restrict__ res, int hidden,
@@ -63,9 +63,11 @@ __device__ __forceinline__ void sq_load(const RowPos& p, int j0, int jn,
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int k = vec_index(v, tpr, p.lt);
-    const int64_t lj = (int64_t)(j0 + (EX ? k : load_index(k, jn))) * VEC;
-    xv[v] = ld_nt<S, VEC>(row_elem<UA>(x, lbase, lj));
-    if constexpr (RES) rv[v] = ld_nt<S, VEC>(row_elem<UA>(res, lbase, lj));
+    const int64_t lj = FORM == FORM_RAGGED
+                           ? vec_off<FORM, VEC>(k, jn, hidden)
+                           : (int64_t)(j0 + (EX ? k : load_index(k, jn))) * VEC;
+    xv[v] = ldf_nt<FORM, S, VEC>(row_elem<UA>(x, lbase, lj));
+    if constexpr (RES) rv[v] = ldf_nt<FORM, S, VEC>(row_elem<UA>(res, lbase, lj));
   }
 }
 
@@ -88,10 +90,10 @@ struct WgRowReduce {
 // (LATE) when it is called: then they are requested two vectors ahead, and b(a) is held in the
 // dtype until its vector's turn.
 template <class E, class EW, class ES, int VEC, int NV, bool FP8, bool RES, bool EX, bool UA,
-          bool LATE, class Shared, class Red>
+          bool LATE, int FORM, class Shared, class Red>
 __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
-                                       const Pack<typename E::S, VEC>* xv,
-                                       const Pack<typename E::S, VEC>* rv,
+                                       Pack<typename E::S, VEC>* xv,
+                                       Pack<typename E::S, VEC>* rv,
                                        Shared&& shared,
                                        uint8_t* __restrict__ out, float* __restrict__ scales,
                                        typename E::S* __restrict__ ares,
@@ -110,6 +112,7 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     const int j = j0 + k;
     const bool in = EX || k < jn;
     if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
+    const int skip = vec_skip<FORM, VEC>(k, hidden);
     Pack<S, VEC> o;
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
 #pragma unroll
@@ -122,8 +125,11 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
       a[v][e] = E::to_f(o.v[e]);  // b(a): what the later passes of the reference re-read
     }
     if constexpr (LATE) z[v] = o;
+    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], skip);
     ss += in ? vs : 0.0;
-    if (ares != nullptr && p.live && in) st_nt<S, VEC>(row_elem<UA>(ares, base, (int64_t)j * VEC), o);
+    if (ares != nullptr && p.live && in) {
+      stf_nt<FORM>(row_elem<UA>(ares, base, (int64_t)j * VEC - skip), o);
+    }
   }
 
   ss = red.sum(ss);
@@ -205,7 +211,8 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
       amax = __builtin_fmaxf(amax, __builtin_fabsf(vv));
     }
     if (anorm != nullptr && p.live && (EX || k < jn)) {
-      st_nt<S, VEC>(row_elem<UA>(anorm, base, (int64_t)j * VEC), o);
+      const int skip = vec_skip<FORM, VEC>(k, hidden);
+      stf_nt<FORM>(row_elem<UA>(anorm, base, (int64_t)j * VEC - skip), o);
     }
   }
   amax = red.max(amax);
@@ -228,7 +235,8 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
       } else {
         q = i8_codes<-127, VEC>(a[v], inv);
       }
-      st_codes_nt<VEC>(row_elem<UA>(out, base, (int64_t)j * VEC), q);
+      const int skip = vec_skip<FORM, VEC>(k, hidden);
+      stf_codes_nt<FORM, VEC>(row_elem<UA>(out, base, (int64_t)j * VEC - skip), q);
     }
   }
 }
@@ -237,16 +245,17 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
 // row's own streamed loads.
 // EX (exact): one row per workgroup and every lane in the row (tpr == blockDim.x, NV * tpr ==
 // hidden / VEC): uniform row index, scalar base addresses with 32-bit offsets, no bounds tests.
-template <class E, class EW, class ES, int VEC, int NV, bool FP8, bool RES, bool EX = false>
+template <class E, class EW, class ES, int VEC, int NV, bool FP8, bool RES, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
 k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
                         const typename E::S* __restrict__ x, const typename EW::S* __restrict__ w,
                         const typename ES::S* __restrict__ sm, typename E::S* __restrict__ ares,
                         typename E::S* __restrict__ anorm, const typename E::S* __restrict__ res,
                         int64_t rows, int hidden, int tpr, float eps, uint32_t flags) {
+  constexpr bool EX = FORM == FORM_EXACT;
   __shared__ double red_sum[16];
   __shared__ uint32_t red_max[16];
-  const int nvec = hidden / VEC;
+  const int nvec = vec_count<FORM, VEC>(hidden);
   RowPos p;
   if constexpr (EX) {
     p = row_pos_one();
@@ -255,9 +264,9 @@ k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   }
   auto load_shared = [&](int v, WVec<EW, VEC>& w_, WVec<ES, VEC>& s_) {
     const int j = vec_index(v, tpr, EX ? p.lt : store_lane<NV>(p.lt));
-    const int64_t lj = (int64_t)(EX ? j : load_index(j, nvec)) * VEC;
-    w_.p = ld<typename EW::S, VEC>(row_elem<EX>(w, 0, lj));
-    s_.p = ld<typename ES::S, VEC>(row_elem<EX>(sm, 0, lj));
+    const int64_t lj = vec_off<FORM, VEC>(j, nvec, hidden);
+    w_.p = ldf<FORM, typename EW::S, VEC>(row_elem<EX>(w, 0, lj));
+    s_.p = ldf<FORM, typename ES::S, VEC>(row_elem<EX>(sm, 0, lj));
   };
   // With eight or more 16-bit vectors a lane they are loaded after the first reduction, vector by
   // vector: held from the start they took half the registers (bf16 at eight vectors with fp32
@@ -283,10 +292,10 @@ k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     }
   };
   Pack<typename E::S, VEC> xv[NV], rv[NV];
-  sq_load<E, VEC, NV, RES, EX>(p, 0, nvec, x, res, hidden, tpr, xv, rv);
+  sq_load<E, VEC, NV, RES, EX, EX, FORM>(p, 0, nvec, x, res, hidden, tpr, xv, rv);
   WgRowReduce<EX> red{red_sum, red_max, tpr};
-  sq_row<E, EW, ES, VEC, NV, FP8, RES, EX, EX, late>(p, 0, nvec, xv, rv, shared, out, scales, ares,
-                                                anorm, hidden, tpr, eps, flags, red);
+  sq_row<E, EW, ES, VEC, NV, FP8, RES, EX, EX, late, FORM>(
+      p, 0, nvec, xv, rv, shared, out, scales, ares, anorm, hidden, tpr, eps, flags, red);
 }
 
 // Rows too wide for one workgroup's registers, read once (split_row.h): workgroup b takes slice
@@ -330,8 +339,8 @@ k_rms_norm_smooth_quant_split(uint8_t* __restrict__ out, float* __restrict__ sca
   SplitRowReduce red{red_sum, red_max, tpr, ws, p.row, slices, sl,
                      ws + split_ws_words(rows, slices) - 1, timeout_ticks, &x_sum, &x_max,
                      &x_fail};
-  sq_row<E, EW, ES, VEC, NV, FP8, RES, false, true, true>(p, j0, jn, xv, rv, shared, out, scales, ares,
-                                                     anorm, hidden, tpr, eps, flags, red);
+  sq_row<E, EW, ES, VEC, NV, FP8, RES, false, true, true, FORM_ROWS>(
+      p, j0, jn, xv, rv, shared, out, scales, ares, anorm, hidden, tpr, eps, flags, red);
   if (red.failed() && p.lt == 0) scales[p.row] = __builtin_nanf("");
 }
 
@@ -526,7 +535,7 @@ struct Args {
   uint32_t flags;
 };
 
-template <class E, class EW, class ES, int VEC, bool FP8, bool RES>
+template <class E, class EW, class ES, int VEC, bool FP8, bool RES, bool RAG = false>
 static void launch_nv(const Geometry& g, const Args& a, hipStream_t st) {
   using S = typename E::S;
   const dim3 grid((unsigned)g.blocks), block((unsigned)(g.tpr * g.rpb));
@@ -548,7 +557,14 @@ static void launch_nv(const Geometry& g, const Args& a, hipStream_t st) {
                      block, lds, st, o, a.scales, xp, wp, sp, arp, anp, rp, a.rows, a.hidden,      \
                      g.tpr, a.eps, a.flags)
   if constexpr (VEC == 1) {
-    if (g.nv == 4) MCOP_LAUNCH(4, false); else MCOP_LAUNCH(16, false);
+    MCOP_LAUNCH(4, FORM_ROWS);
+  } else if constexpr (RAG) {
+    switch (g.nv) {
+      case 1: MCOP_LAUNCH(1, FORM_RAGGED); break;
+      case 2: MCOP_LAUNCH(2, FORM_RAGGED); break;
+      case 4: MCOP_LAUNCH(4, FORM_RAGGED); break;
+      default: MCOP_LAUNCH(8, FORM_RAGGED); break;
+    }
   } else {
     // exact rows (one row per workgroup, every lane in it) on the latency path (at most 256
     // rows) take the EX form; bandwidth-bound shapes keep the generic one (a uniform-row form
@@ -557,25 +573,38 @@ static void launch_nv(const Geometry& g, const Args& a, hipStream_t st) {
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == a.hidden / VEC && a.rows <= 256;
 #define MCOP_EX(NVV)                                                                           \
   (ex && exact_form_ok(reinterpret_cast<const void*>(                                          \
-             &k_rms_norm_smooth_quant<E, EW, ES, VEC, NVV, FP8, RES, true>)))
+             &k_rms_norm_smooth_quant<E, EW, ES, VEC, NVV, FP8, RES, FORM_EXACT>)))
     switch (g.nv) {
-      case 1: MCOP_LAUNCH(1, false); break;
-      case 2: if (MCOP_EX(2)) MCOP_LAUNCH(2, true); else MCOP_LAUNCH(2, false); break;
-      case 4: if (MCOP_EX(4)) MCOP_LAUNCH(4, true); else MCOP_LAUNCH(4, false); break;
-      case 8: if (MCOP_EX(8)) MCOP_LAUNCH(8, true); else MCOP_LAUNCH(8, false); break;
-      default: MCOP_LAUNCH(16, false); break;
+      case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
+      case 2:
+        if (MCOP_EX(2)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        break;
+      case 4:
+        if (MCOP_EX(4)) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
+        break;
+      case 8:
+        if (MCOP_EX(8)) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
+        break;
+      default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
 #undef MCOP_EX
   }
 #undef MCOP_LAUNCH
 }
 
-template <class E, class EW, class ES, int VEC, bool FP8, bool RES>
+template <class E, class EW, class ES, int VEC, bool FP8, bool RES, bool RAG = false>
 static const void* kernel_of(int nv) {
+  auto fn = [](auto k) { return reinterpret_cast<const void*>(k); };
   if constexpr (VEC == 1) {
-    return nv == 4
-               ? reinterpret_cast<const void*>(&k_rms_norm_smooth_quant<E, EW, ES, 1, 4, FP8, RES>)
-               : reinterpret_cast<const void*>(&k_rms_norm_smooth_quant<E, EW, ES, 1, 16, FP8, RES>);
+    return nv == 4 ? fn(&k_rms_norm_smooth_quant<E, EW, ES, 1, 4, FP8, RES>) : nullptr;
+  } else if constexpr (RAG) {
+    switch (nv) {
+      case 1: return fn(&k_rms_norm_smooth_quant<E, EW, ES, VEC, 1, FP8, RES, FORM_RAGGED>);
+      case 2: return fn(&k_rms_norm_smooth_quant<E, EW, ES, VEC, 2, FP8, RES, FORM_RAGGED>);
+      case 4: return fn(&k_rms_norm_smooth_quant<E, EW, ES, VEC, 4, FP8, RES, FORM_RAGGED>);
+      case 8: return fn(&k_rms_norm_smooth_quant<E, EW, ES, VEC, 8, FP8, RES, FORM_RAGGED>);
+      default: return nullptr;
+    }
   } else {
     switch (nv) {
       case 1: return reinterpret_cast<const void*>(&k_rms_norm_smooth_quant<E, EW, ES, VEC, 1, FP8, RES>);
@@ -626,10 +655,15 @@ static int dispatch(const Args& a, hipStream_t st) {
   const bool vec_ok = a.hidden % V == 0 && aligned(16, a.x, a.ares, a.anorm, a.res) &&
                       aligned(WB, a.w) && aligned(SB, a.sm) && aligned(V, a.out);
   const bool r = a.res != nullptr;
+  // any other row of at least one vector takes the ragged form, narrower ones one element a load
+  const bool rag = !vec_ok && a.hidden >= V;
+  const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels =
       vec_ok ? (r ? &kernel_of<E, EW, ES, V, FP8, true> : &kernel_of<E, EW, ES, V, FP8, false>)
+      : rag  ? (r ? &kernel_of<E, EW, ES, V, FP8, true, true>
+                  : &kernel_of<E, EW, ES, V, FP8, false, true>)
              : (r ? &kernel_of<E, EW, ES, 1, FP8, true> : &kernel_of<E, EW, ES, 1, FP8, false>);
-  if (!row_fits(a.hidden, vec_ok ? V : 1, kernels)) {
+  if (!row_fits(a.hidden, vec, kernels)) {
     const char* name = "rms_norm_dynamic_per_token_quant (smooth)";
     if (vec_ok && split_rows_enabled()) {
       const int rc = r ? launch_split<E, EW, ES, V, FP8, true>(name, a, st)
@@ -659,13 +693,16 @@ static int dispatch(const Args& a, hipStream_t st) {
   }
   Geometry g;
   if (!choose_geometry("rms_norm_dynamic_per_token_quant (smooth)", a.rows, a.hidden,
-                       vec_ok ? V : 1, kernels, &g)) {
+                       vec, kernels, &g)) {
     return MCOP_E_UNSUPPORTED;
   }
   const bool has_res = a.res != nullptr;
   if (g.vec == 1) {
     if (has_res) launch_nv<E, EW, ES, 1, FP8, true>(g, a, st);
     else launch_nv<E, EW, ES, 1, FP8, false>(g, a, st);
+  } else if (rag) {
+    if (has_res) launch_nv<E, EW, ES, V, FP8, true, true>(g, a, st);
+    else launch_nv<E, EW, ES, V, FP8, false, true>(g, a, st);
   } else {
     if (has_res) launch_nv<E, EW, ES, V, FP8, true>(g, a, st);
     else launch_nv<E, EW, ES, V, FP8, false>(g, a, st);
