@@ -1,6 +1,6 @@
 """``mcoplib.custom_ops`` wrappers of the fused norm/quant path (reference
-mcoplib/custom_ops.py:7-45): allocate the outputs the way the reference does, then call the
-``op`` entry point."""
+mcoplib/custom_ops.py:7-45): allocate the outputs the way the reference does and call the
+``op`` entry point, both in the _torch_ops extension."""
 
 from __future__ import annotations
 
@@ -8,7 +8,8 @@ from typing import Optional, Tuple
 
 import torch
 
-from . import op as ops
+from . import op as ops  # noqa: F401  (loads the library, then the extension)
+from . import _torch_ops
 
 
 def fused_add_rms_norm_dynamic_per_token_quant_padding_output(
@@ -19,18 +20,8 @@ def fused_add_rms_norm_dynamic_per_token_quant_padding_output(
     returns (output, residual, output_rms, output_quant_int8, scales); ``residual`` is updated
     in place (reference mcoplib/custom_ops.py:7-27)."""
     assert input.is_contiguous()
-    shape = list(input.shape)
-    shape[-1] = pad_size
-    output = torch.empty(shape, dtype=torch.bfloat16, device=input.device)
     assert weight.is_contiguous()
-    output_rms = torch.empty_like(input)
-    output_quant_int8 = torch.empty_like(input, dtype=torch.int8)
-    scales = torch.empty((input.numel() // input.shape[-1], 1), device=input.device,
-                         dtype=torch.float32)
-    ops.fused_add_rms_norm_dynamic_per_token_quant_padding_output(
-        output.view(dtype=torch.int8), output_rms, output_quant_int8, scales, input, residual,
-        weight, pad_size, epsilon)
-    return output, residual, output_rms, output_quant_int8, scales
+    return _torch_ops.padded_new(input, residual, weight, pad_size, epsilon)
 
 
 def rms_norm_dynamic_per_token_quant(input: torch.Tensor, weight: torch.Tensor, epsilon: float,
@@ -40,9 +31,4 @@ def rms_norm_dynamic_per_token_quant(input: torch.Tensor, weight: torch.Tensor, 
                                      ) -> Tuple[torch.Tensor, torch.Tensor]:
     """Returns (codes like input in quant_dtype, scales [T, 1] fp32); updates ``residual`` in
     place when given.  ``quant_dtype`` must be int8, as for the reference custom op."""
-    output = torch.empty_like(input, dtype=quant_dtype)
-    scales = torch.empty((input.numel() // input.shape[-1], 1), device=input.device,
-                         dtype=torch.float32)
-    ops.rms_norm_dynamic_per_token_quant_custom(output, input, weight, scales, epsilon, scale_ub,
-                                                residual)
-    return output, scales
+    return _torch_ops.custom_new(input, weight, epsilon, quant_dtype, scale_ub, residual)
