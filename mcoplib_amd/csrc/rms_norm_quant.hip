@@ -498,8 +498,18 @@ static void launch_nv(const Geometry& g, void* out, float* scales, const void* x
   auto* xp = static_cast<const S*>(x);
   auto* wp = static_cast<const S*>(w);
   auto* rp = static_cast<S*>(res);
+  // Eight-wave workgroups: three resident on a CU at two vectors a lane, two at four (bf16), by
+  // dynamic LDS that they do not use (resident_cap): fewer rows in flight than their registers
+  // allow stream faster here.  int8 with a residual: 8192 x 8192 75.9 us at four, 75.2 at three;
+  // 4096 x 16384 80.0 at three, 79.1 at two (32768 x 16384 622 either way).  fp16 at four vectors
+  // needs the third to hide its conversions (4096 x 14336 fp8 72.5, 75.6 at two).
+  const int cap = VEC == 1 || g.tpr * g.rpb != 512          ? 0
+                  : g.nv == 2                               ? 3
+                  : g.nv == 4 && std::is_same<E, BF16>::value ? 2
+                                                            : 0;
+  const unsigned lds = resident_cap(cap, g.blocks);
 #define MCOP_LAUNCH(NVV, EXX)                                                                  \
-  hipLaunchKernelGGL((k_rms_norm_quant<E, VEC, NVV, FP8, RES, MODE, EXX>), grid, block, 0, st, o, \
+  hipLaunchKernelGGL((k_rms_norm_quant<E, VEC, NVV, FP8, RES, MODE, EXX>), grid, block, lds, st, o, \
                      scales, xp, wp, scale_ub, rp, rows, hidden, g.tpr, eps)
   if constexpr (VEC == 1) {
     MCOP_LAUNCH(4, FORM_ROWS);

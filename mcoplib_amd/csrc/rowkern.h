@@ -854,6 +854,14 @@ bool split_rows_enabled();
 bool wide_rows_ok(const char* op, int64_t rows);
 constexpr int kWideLanes = 1024;
 
+// Dynamic LDS (which the kernel does not use) that lets at most `per_cu` of a kernel's workgroups
+// be resident on a CU: 0 for per_cu 0, or when the launch has fewer than four rounds of them on
+// the 256 CUs (then every workgroup that fits should run).
+inline unsigned resident_cap(int per_cu, int64_t blocks) {
+  if (per_cu == 0 || blocks < (int64_t)4 * 256 * per_cu) return 0;
+  return (unsigned)(160 * 1024 / (per_cu + 1) + 1024);
+}
+
 // True when every non-null pointer is aligned to `bytes`.
 bool aligned(int bytes, const void* p0, const void* p1 = nullptr, const void* p2 = nullptr,
              const void* p3 = nullptr, const void* p4 = nullptr, const void* p5 = nullptr);

@@ -550,8 +550,7 @@ static void launch_nv(const Geometry& g, const Args& a, hipStream_t st) {
   // do not use (their registers would let four in).  The memory side of this write-heavy row
   // prefers fewer rows in flight: 16384 x 7168 fp8 143.4 us at three, 145.7 at four; 8192 x 4096
   // 42.5 and 43.6.
-  const bool cap = VEC > 1 && g.nv == 4 && a.rows > 256 && g.tpr * g.rpb == 256;
-  const unsigned lds = cap ? 44 * 1024 : 0;
+  const unsigned lds = resident_cap(VEC > 1 && g.nv == 4 && g.tpr * g.rpb == 256 ? 3 : 0, g.blocks);
 #define MCOP_LAUNCH(NVV, EXX)                                                                   \
   hipLaunchKernelGGL((k_rms_norm_smooth_quant<E, EW, ES, VEC, NVV, FP8, RES, EXX>), grid,      \
                      block, lds, st, o, a.scales, xp, wp, sp, arp, anp, rp, a.rows, a.hidden,      \
