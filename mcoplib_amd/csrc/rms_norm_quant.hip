@@ -63,7 +63,7 @@ __device__ __forceinline__ Codes<VEC> row_codes(const float* y, float rho, float
                                                         float inv, bool s_ok, bool bounded,
                                                         bool has_ub) {
   constexpr int LO = MODE == QM_VLLM ? -128 : -127;
-  if constexpr (FP8) return fp8_quotient_codes<VEC>(y, s, inv, s_ok, bounded);
+  if constexpr (FP8) return fp8_quotient_codes<VEC, true>(y, s, inv, s_ok, bounded);
   float t[VEC];
 #pragma unroll
   for (int e = 0; e < VEC; ++e) t[e] = MODE == QM_MC_7168 ? y[e] * rho : y[e];
@@ -162,7 +162,7 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     }
   }
 
-  ss = row_reduce<EX, (NV < 8)>(ss, red_sum, tpr, SumOp());
+  ss = row_reduce<EX, (NV < 4)>(ss, red_sum, tpr, SumOp());
   const float rho = row_inv_rms(ss, hidden, eps);
 
   // The absmax must skip the copies of vector 0 held past the row end: with an in-place
@@ -180,7 +180,7 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
       amax = __builtin_fmaxf(amax, in ? __builtin_fabsf(a[v][e]) : 0.0f);
     }
   }
-  amax = row_absmax<EX, (NV < 8)>(amax, red_max, tpr);
+  amax = row_absmax<EX, (NV < 4)>(amax, red_max, tpr);
 
   float A;
   const float s = row_scale<FP8, MODE>(amax, rho, scale_ub, &A);
