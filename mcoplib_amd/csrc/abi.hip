@@ -133,7 +133,10 @@ int blocks_per_cu(const void* kernel, int block) {
 //     from the kernel's occupancy); else nv = 4 (e.g. 7-wave workgroups leave a third of the
 //     wave slots empty); 8 or 16 only for rows that do not fit otherwise.  Kernels that spill
 //     registers are skipped while another shape fits.
-// Scalar path (hidden not a multiple of the vector width, or misaligned pointers): nv in {4,16}.
+// Rows that are not whole aligned vectors (hidden not a multiple of the vector width, odd strides
+// or misaligned pointers): the same search over the ragged kernels, nv in {1,2,4,8}.  Only a row
+// narrower than one vector (and the group kernel's element-wise form, nv in {4,16}) is taken an
+// element at a time.
 // Lanes per row for n lanes of work: whole waves, or 16 / 32 lanes when the row is that short.
 static int64_t row_lanes(int64_t n, int min_tpr) {
   if (n <= 32 && min_tpr <= 32) return n <= 16 && min_tpr <= 16 ? 16 : 32;

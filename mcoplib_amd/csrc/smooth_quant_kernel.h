@@ -620,8 +620,10 @@ static const void* kernel_of(int nv) {
 template <class E, class EW, class ES, int VEC, bool FP8, bool RES>
 static int launch_split(const char* name, const Args& a, hipStream_t st) {
   using S = typename E::S;
-  // 512-lane workgroups (half the slices, so half the exchanges per row for the same resident
-  // vectors per CU): 450 us against 469 us at 256 lanes for 2048 x 131072 bf16 fp8
+  // Two shapes of 2048-vector slices, chosen by how many vectors each keeps resident: eight a lane
+  // over 256 lanes ran 375 us for 2048 x 131072 bf16 fp8 against 446 us for four over 512 lanes
+  // (three waves per SIMD hold half as many again); where the eight-vector form's registers do not
+  // pay, four over 512 lanes, whose half as many slices as 256 lanes beat it 450 us to 469
   const SplitKernel k4{reinterpret_cast<const void*>(
                            &k_rms_norm_smooth_quant_split<E, EW, ES, VEC, 4, FP8, RES>), 4, 512};
   const SplitKernel k8{reinterpret_cast<const void*>(
