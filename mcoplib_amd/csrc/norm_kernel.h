@@ -121,6 +121,8 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
     p = row_pos(rows, tpr);
   }
   const int nvec = vec_count<FORM, VEC>(hidden);
+  // after_res may be the residual or the input itself: the last vector apart, as in place
+  const bool apart = FORM == FORM_RAGGED && RES && vec_apart(nvec, tpr);
   const RowOffsets lo = row_offsets(map, p.lrow);
   const int64_t out_base = p.row == p.lrow ? lo.out : 0;
   const int64_t rbase = p.row * (int64_t)hidden;
@@ -150,6 +152,10 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
     const int j = vec_index(v, tpr, p.lt);
     const bool in = EX || j < nvec;
     const int skip = vec_skip<FORM, VEC>(j, hidden);
+    if constexpr (RES) {
+      trim<FORM>(xv[v], skip, apart);
+      trim<FORM>(rv[v], skip, apart);
+    }
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
     Pack<S, VEC> o;
 #pragma unroll
@@ -169,7 +175,7 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
     ss += in ? vs : 0.0;
     if constexpr (RES) {
       if (p.live && in) {
-        stf_nt<FORM>(row_elem<EX>(ares, rbase, (int64_t)j * VEC - skip), o);
+        stf_nt<FORM>(row_elem<EX>(ares, rbase, (int64_t)j * VEC - skip), o, skip, apart);
       }
     }
   }
@@ -228,7 +234,7 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
       for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(n[e] * wv[v].at(e));
     }
     const int skip = vec_skip<FORM, VEC>(j, hidden);
-    stf_nt<FORM>(row_elem<EX>(out, out_base, (int64_t)j * VEC - skip), o);
+    stf_nt<FORM>(row_elem<EX>(out, out_base, (int64_t)j * VEC - skip), o, skip, apart);
   }
 }
 

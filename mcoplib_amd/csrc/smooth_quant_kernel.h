@@ -103,6 +103,8 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
   const int64_t base = p.row * (int64_t)hidden;
 
   const int slt = EX ? p.lt : store_lane<NV>(p.lt);
+  // after_res may be the residual or the input itself: the last vector apart, as in place
+  const bool apart = FORM == FORM_RAGGED && ares != nullptr && vec_apart(jn, tpr);
   float a[NV][VEC];
   Pack<S, VEC> z[LATE ? NV : 1];
   double ss = 0.0;
@@ -113,6 +115,8 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     const bool in = EX || k < jn;
     if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
     const int skip = vec_skip<FORM, VEC>(k, hidden);
+    trim<FORM>(xv[v], skip, apart);
+    if constexpr (RES) trim<FORM>(rv[v], skip, apart);
     Pack<S, VEC> o;
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
 #pragma unroll
@@ -128,7 +132,7 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], skip);
     ss += in ? vs : 0.0;
     if (ares != nullptr && p.live && in) {
-      stf_nt<FORM>(row_elem<UA>(ares, base, (int64_t)j * VEC - skip), o);
+      stf_nt<FORM>(row_elem<UA>(ares, base, (int64_t)j * VEC - skip), o, skip, apart);
     }
   }
 
@@ -208,11 +212,14 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
       o.v[e] = E::from_f(u);
       const float vv = u * sv.at(e);
       a[v][e] = vv;
-      amax = __builtin_fmaxf(amax, __builtin_fabsf(vv));
+      // ragged lanes past the row end may hold a copy of the last vector that already has the
+      // residual in it twice
+      const bool in = FORM != FORM_RAGGED || k < jn;
+      amax = __builtin_fmaxf(amax, in ? __builtin_fabsf(vv) : 0.0f);
     }
     if (anorm != nullptr && p.live && (EX || k < jn)) {
       const int skip = vec_skip<FORM, VEC>(k, hidden);
-      stf_nt<FORM>(row_elem<UA>(anorm, base, (int64_t)j * VEC - skip), o);
+      stf_nt<FORM>(row_elem<UA>(anorm, base, (int64_t)j * VEC - skip), o, skip, apart);
     }
   }
   amax = red.max(amax);
@@ -236,7 +243,7 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
         q = i8_codes<-127, VEC>(a[v], inv);
       }
       const int skip = vec_skip<FORM, VEC>(k, hidden);
-      stf_codes_nt<FORM, VEC>(row_elem<UA>(out, base, (int64_t)j * VEC - skip), q);
+      stf_codes_nt<FORM, VEC>(row_elem<UA>(out, base, (int64_t)j * VEC - skip), q, skip, apart);
     }
   }
 }

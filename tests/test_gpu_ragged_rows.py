@@ -104,3 +104,30 @@ def test_smooth_scale_and_padded(H, T):
     assert_scales(s, s_ref, "padded scales")
     assert_codes(q, q_ref, "codes")
     assert_exact(p.view(torch.uint8), p_ref, "padded rows, the bytes between them untouched")
+
+
+@pytest.mark.parametrize("H", [513, 1025, 1537, 2049, 4097, 5121, 8193])
+def test_after_res_over_the_residual(H):
+    """after_res given as the residual's (or the input's) own buffer, where the last vector of a
+    row starts a wave and overlaps one that another wave stores."""
+    T, eps = 300, 1e-6
+    x, r, w, xd, rd, wd = rows(H, T, BF, 0)
+    sm = 0.5 + torch.rand(H, generator=gen(H + 3))
+    ar, out, ref = torch.empty_like(xd), torch.empty_like(xd), torch.empty_like(xd)
+    op.rms_norm(ref, xd, wd, eps, ar, rd, False)
+    for own in ("residual", "input"):
+        xx, rr = xd.clone(), rd.clone()
+        over = rr if own == "residual" else xx
+        op.rms_norm(out, xx, wd, eps, over, rr, False)
+        assert_exact(over, (x.float() + r.float()).to(BF), f"norm after_res over the {own}")
+        assert_exact(out, ref.cpu(), f"norm over the {own}")
+    q_ref, s_ref, ar_ref, an_ref = oracle.rms_norm_smooth_quant(x, w, sm, eps, torch.int8, r)
+    for own in ("residual", "input"):
+        xx, rr, an = xd.clone(), rd.clone(), torch.empty_like(xd)
+        over = rr if own == "residual" else xx
+        q, s = torch.empty(T, H, dtype=torch.int8, device=DEV), torch.empty(T, device=DEV)
+        op.rms_norm_dynamic_per_token_quant(q, xx, wd, sm.to(DEV), s, eps, over, an, rr)
+        assert_exact(over, ar_ref, f"H4 after_res over the {own}")
+        assert_exact(an, an_ref, f"H4 after_norm over the {own}")
+        assert_scales(s, s_ref, f"H4 scales over the {own}")
+        assert_codes(q, q_ref, f"H4 codes over the {own}")
