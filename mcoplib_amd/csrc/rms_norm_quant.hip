@@ -498,15 +498,19 @@ static void launch_nv(const Geometry& g, void* out, float* scales, const void* x
   auto* xp = static_cast<const S*>(x);
   auto* wp = static_cast<const S*>(w);
   auto* rp = static_cast<S*>(res);
-  // Eight-wave workgroups: three resident on a CU at two vectors a lane, two at four (bf16), by
-  // dynamic LDS that they do not use (resident_cap): fewer rows in flight than their registers
-  // allow stream faster here.  int8 with a residual: 8192 x 8192 75.9 us at four, 75.2 at three;
-  // 4096 x 16384 80.0 at three, 79.1 at two (32768 x 16384 622 either way).  fp16 at four vectors
-  // needs the third to hide its conversions (4096 x 14336 fp8 72.5, 75.6 at two).
-  const int cap = VEC == 1 || g.tpr * g.rpb != 512          ? 0
-                  : g.nv == 2                               ? 3
-                  : g.nv == 4 && std::is_same<E, BF16>::value ? 2
-                                                            : 0;
+  // Rows with a residual: three eight-wave workgroups resident on a CU at two vectors a lane, two
+  // of six to eight waves at four, by dynamic LDS that they do not use (resident_cap): fewer rows
+  // in flight than their registers allow stream faster where as much is written as read.  us
+  // uncapped and so: 8192 x 8192 int8 75.6 and 75.2; 4096 x 12288 62.8 and 59.9, 14336 71.0 and
+  // 69.4, 16384 79.1 and 78.3; fp16 fp8 14336 73.5 and 70.4; fp32 8192 x 6144 108.5 and 104.7.
+  // Smaller workgroups do not gain throughout (4096 x 8704 fp16 fp8 46.7, 49.2 at two), and rows
+  // without a residual, mostly reads, want every load in flight (8192 x 8192 int8 38.0, 41.5 at
+  // three; 4096 x 16384 fp8 40.1, 41.1 at two).
+  const int lanes = g.tpr * g.rpb;
+  const int cap = !RES || VEC == 1                              ? 0
+                  : g.nv == 2 && lanes == 512                   ? 3
+                  : g.nv == 4 && lanes >= 384 && lanes <= 512 ? 2
+                                                              : 0;
   const unsigned lds = resident_cap(cap, g.blocks);
 #define MCOP_LAUNCH(NVV, EXX)                                                                  \
   hipLaunchKernelGGL((k_rms_norm_quant<E, VEC, NVV, FP8, RES, MODE, EXX>), grid, block, lds, st, o, \

@@ -191,8 +191,8 @@ __device__ __forceinline__ void widen(float* f, const Pack<typename E::S, N>& p)
 //                elements before their owner stores them: both are in one wave's instruction,
 //                whose loads end before its stores begin, unless the last vector starts a wave's
 //                run of lanes (`apart`); then they are read as zeros and not stored.
-// Before, one element a load: 2048 x 5137 fp8 with a residual 28.3 us, 20.7 so; 4096 x 4099 norm
-// with a residual 58.5 and 35.5; 65536 x 67 norm 13.0 and 8.2; 4096 x 30001 int8 521 and 223.
+// Before, one element a load: 2048 x 5137 fp8 with a residual 30.6 us, 20.7 so; 4096 x 4099 norm
+// with a residual 52.6 and 33.3; 65536 x 67 norm 13.0 and 8.2; 4096 x 30001 int8 521 and 223.
 enum Form { FORM_ROWS = 0, FORM_EXACT = 1, FORM_RAGGED = 2 };
 
 template <int FORM, int VEC>
