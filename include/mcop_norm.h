@@ -114,7 +114,7 @@ int mcop_rms_norm_dynamic_per_token_quant_noalloc(void* out, mcop_dtype out_dtyp
  *   fp8 (this library's extension; the reference's operator is int8 only): s = A/448,
  *   q = e4m3fn(clamp(v / s, -448, 448));  A == 0 gives s = 0 and q = 0.
  * `weight_dtype` and `smooth_dtype` are each `in_dtype` or MCOP_F32. after_res, after_norm and
- * residual may be NULL.
+ * residual may be NULL. after_res may be the residual's or the input's own buffer.
  * Replaces rms_norm_dynamic_per_token_quant(), op/fused_rms_norm_dq.cu:646-667
  * (pybind op/pybind.cpp:42, declaration include/fused_rms_norm_dq.h:3-12). */
 int mcop_rms_norm_smooth_quant(void* out, mcop_dtype out_dtype, float* scales,
@@ -184,6 +184,7 @@ int mcop_rms_norm_dynamic_per_token_quant_custom(int8_t* out, float* scales, con
  *   else 8); otherwise its element-wise chain: out <- b((a~ / rho) * w) (rms_div) or
  *   b((a~ * rho) * w), a~ = b(a) with a residual, x without.  rho = 1/sqrt(sum(a^2)/H + eps).
  * input, out, residual, after_res: [T,H] contiguous in_dtype; weight [H] in_dtype or fp32.
+ * after_res may be the residual's or the input's own buffer.
  * Replaces rms_norm(), op/fused_rms_norm_dq.cu:980-998 (dispatch :814-978, kernels :305-420;
  * pybind op/pybind.cpp:44). */
 int mcop_rms_norm(void* out, const void* input, const void* weight, mcop_dtype weight_dtype,

@@ -103,14 +103,17 @@ __device__ __forceinline__ Pack<typename E::S, VEC> norm_out(const float* a,
   return o;
 }
 
+// x and the residual: after_res (stored with a residual only) may be either one's own buffer.
+template <class E, bool RES>
+using RowIn = std::conditional_t<RES, const typename E::S*, const typename E::S* __restrict__>;
+
 // EX (exact): one row per workgroup and every lane in the row (tpr == blockDim.x, NV * tpr ==
 // hidden / VEC): uniform row index, scalar base addresses with 32-bit offsets, no bounds tests.
 template <class E, class EW, int VEC, int NV, bool RES, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
-k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
-           const typename E::S* __restrict__ x, const typename EW::S* __restrict__ w,
-           const typename E::S* __restrict__ res, RowMap map, int64_t rows, int hidden, int tpr,
-           float eps, int mode, int rms_div) {
+k_rms_norm(typename E::S* __restrict__ out, typename E::S* ares, RowIn<E, RES> x,
+           const typename EW::S* __restrict__ w, RowIn<E, RES> res, RowMap map, int64_t rows,
+           int hidden, int tpr, float eps, int mode, int rms_div) {
   using S = typename E::S;
   constexpr bool EX = FORM == FORM_EXACT;
   __shared__ double red_sum[16];
@@ -246,11 +249,10 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
 // within the row.
 template <class E, class EW, int VEC, int NV, bool RES>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
-k_rms_norm_split(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
-                 const typename E::S* __restrict__ x, const typename EW::S* __restrict__ w,
-                 const typename E::S* __restrict__ res, RowMap map, int64_t row0, int64_t rows,
-                 int hidden, float eps, int mode, int rms_div, int slices, int slice_vecs,
-                 uint64_t* __restrict__ ws, int64_t timeout_ticks) {
+k_rms_norm_split(typename E::S* __restrict__ out, typename E::S* ares, RowIn<E, RES> x,
+                 const typename EW::S* __restrict__ w, RowIn<E, RES> res, RowMap map,
+                 int64_t row0, int64_t rows, int hidden, float eps, int mode, int rms_div,
+                 int slices, int slice_vecs, uint64_t* __restrict__ ws, int64_t timeout_ticks) {
   using S = typename E::S;
   __shared__ double red_sum[16];
   __shared__ double x_sum;
@@ -366,10 +368,9 @@ k_rms_norm_split(typename E::S* __restrict__ out, typename E::S* __restrict__ ar
 // row, and the weight.
 template <class E, class EW, int VEC, bool RES>
 __global__ void __launch_bounds__(kWideLanes)
-k_rms_norm_wide(typename E::S* __restrict__ out, typename E::S* __restrict__ ares,
-                const typename E::S* __restrict__ x, const typename EW::S* __restrict__ w,
-                const typename E::S* __restrict__ res, RowMap map, int hidden, float eps,
-                int mode, int rms_div) {
+k_rms_norm_wide(typename E::S* __restrict__ out, typename E::S* ares, RowIn<E, RES> x,
+                const typename EW::S* __restrict__ w, RowIn<E, RES> res, RowMap map, int hidden,
+                float eps, int mode, int rms_div) {
   using S = typename E::S;
   // NC: the largest register head that compiles without spills at 1024 lanes (fp16 conversions
   // take more registers)

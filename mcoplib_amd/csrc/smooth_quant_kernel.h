@@ -54,9 +54,8 @@ __device__ __forceinline__ Codes<VEC> sq_fp8_codes(const float* v, float amax, f
 // (and the residual); lanes past the slice end load its first vector.
 template <class E, int VEC, int NV, bool RES, bool EX, bool UA = EX, int FORM = FORM_ROWS>
 __device__ __forceinline__ void sq_load(const RowPos& p, int j0, int jn,
-                                        const typename E::S* __restrict__ x,
-                                        const typename E::S* __restrict__ res, int hidden,
-                                        int tpr, Pack<typename E::S, VEC>* xv,
+                                        const typename E::S* x, const typename E::S* res,
+                                        int hidden, int tpr, Pack<typename E::S, VEC>* xv,
                                         Pack<typename E::S, VEC>* rv) {
   using S = typename E::S;
   const int64_t lbase = p.lrow * (int64_t)hidden;
@@ -88,7 +87,8 @@ struct WgRowReduce {
 // (scalar row base, one 32-bit offset per vector: row_elem<true>).
 // `shared(v, w, s)` gives the lane's v-th weight and smooth vectors: loaded ahead of the row's, or
 // (LATE) when it is called: then they are requested two vectors ahead, and b(a) is held in the
-// dtype until its vector's turn.
+// dtype until its vector's turn.  ares may be the buffer of x or of the residual, in every kernel
+// of this operator: those three are not __restrict__.
 template <class E, class EW, class ES, int VEC, int NV, bool FP8, bool RES, bool EX, bool UA,
           bool LATE, int FORM, class Shared, class Red>
 __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
@@ -96,7 +96,7 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
                                        Pack<typename E::S, VEC>* rv,
                                        Shared&& shared,
                                        uint8_t* __restrict__ out, float* __restrict__ scales,
-                                       typename E::S* __restrict__ ares,
+                                       typename E::S* ares,
                                        typename E::S* __restrict__ anorm, int hidden, int tpr,
                                        float eps, uint32_t flags, Red& red) {
   using S = typename E::S;
@@ -206,17 +206,18 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     } else {
       div_by_const<VEC>(n, a[v], rho, inv_rho, rho_ok);
     }
+    float vm = 0.0f;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       const float u = n[e] * wv.at(e);
       o.v[e] = E::from_f(u);
-      const float vv = u * sv.at(e);
-      a[v][e] = vv;
-      // ragged lanes past the row end may hold a copy of the last vector that already has the
-      // residual in it twice
-      const bool in = FORM != FORM_RAGGED || k < jn;
-      amax = __builtin_fmaxf(amax, in ? __builtin_fabsf(vv) : 0.0f);
+      a[v][e] = u * sv.at(e);
+      vm = __builtin_fmaxf(vm, __builtin_fabsf(a[v][e]));
     }
+    // Lanes past the end hold a copy of one of the row's (slice's) vectors, which must not count:
+    // with after_res over the residual or the input, the wave that owns the vector may have
+    // stored after_res there before the copy was read, and the copy has the residual in it twice.
+    amax = __builtin_fmaxf(amax, EX || k < jn ? vm : 0.0f);
     if (anorm != nullptr && p.live && (EX || k < jn)) {
       const int skip = vec_skip<FORM, VEC>(k, hidden);
       stf_nt<FORM>(row_elem<UA>(anorm, base, (int64_t)j * VEC - skip), o, skip, apart);
@@ -255,9 +256,9 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
 template <class E, class EW, class ES, int VEC, int NV, bool FP8, bool RES, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
 k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
-                        const typename E::S* __restrict__ x, const typename EW::S* __restrict__ w,
-                        const typename ES::S* __restrict__ sm, typename E::S* __restrict__ ares,
-                        typename E::S* __restrict__ anorm, const typename E::S* __restrict__ res,
+                        const typename E::S* x, const typename EW::S* __restrict__ w,
+                        const typename ES::S* __restrict__ sm, typename E::S* ares,
+                        typename E::S* __restrict__ anorm, const typename E::S* res,
                         int64_t rows, int hidden, int tpr, float eps, uint32_t flags) {
   constexpr bool EX = FORM == FORM_EXACT;
   __shared__ double red_sum[16];
@@ -312,13 +313,10 @@ k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
 template <class E, class EW, class ES, int VEC, int NV, bool FP8, bool RES>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
 k_rms_norm_smooth_quant_split(uint8_t* __restrict__ out, float* __restrict__ scales,
-                              const typename E::S* __restrict__ x,
-                              const typename EW::S* __restrict__ w,
-                              const typename ES::S* __restrict__ sm,
-                              typename E::S* __restrict__ ares,
-                              typename E::S* __restrict__ anorm,
-                              const typename E::S* __restrict__ res, int64_t rows, int hidden,
-                              int slices, int slice_vecs, float eps, uint32_t flags,
+                              const typename E::S* x, const typename EW::S* __restrict__ w,
+                              const typename ES::S* __restrict__ sm, typename E::S* ares,
+                              typename E::S* __restrict__ anorm, const typename E::S* res,
+                              int64_t rows, int hidden, int slices, int slice_vecs, float eps, uint32_t flags,
                               uint64_t* __restrict__ ws, int64_t timeout_ticks) {
   __shared__ double red_sum[16];
   __shared__ uint32_t red_max[16];
@@ -358,12 +356,10 @@ k_rms_norm_smooth_quant_split(uint8_t* __restrict__ out, float* __restrict__ sca
 template <class E, class EW, class ES, int VEC, bool FP8, bool RES>
 __global__ void __launch_bounds__(kWideLanes)
 k_rms_norm_smooth_quant_wide(uint8_t* __restrict__ out, float* __restrict__ scales,
-                             const typename E::S* __restrict__ x,
-                             const typename EW::S* __restrict__ w,
-                             const typename ES::S* __restrict__ sm,
-                             typename E::S* __restrict__ ares, typename E::S* __restrict__ anorm,
-                             const typename E::S* __restrict__ res, int hidden, float eps,
-                             uint32_t flags) {
+                             const typename E::S* x, const typename EW::S* __restrict__ w,
+                             const typename ES::S* __restrict__ sm, typename E::S* ares,
+                             typename E::S* __restrict__ anorm, const typename E::S* res,
+                             int hidden, float eps, uint32_t flags) {
   using S = typename E::S;
   // The row head (the lane's first NC vectors of x, and of the residual) is loaded once and
   // kept in registers across the three passes, the next NL in LDS; the passes re-read only the
