@@ -53,6 +53,9 @@ FOUR_WAVE_KERNELS = (
     r"^void mcop::k_fused_add_rms_norm<mcop::BF16, 8, 8, (false|0)>\(",
     r"^void mcop::k_rms_norm_quant_split<mcop::BF16, 8, 8, false, (true|false), [0-9]>\(",
 )
+# Exact-row forms, which the launch takes by the row's shape alone: none may spill.
+EXACT_KERNELS = (r"^void mcop::k_(rms_norm_quant|fused_add_rms_norm|rms_norm|rms_norm_smooth_quant|"
+                 r"add_rms_norm_quant_padded|per_token_quant|rms_norm_group_quant)<.*, (true|1)>\(")
 RESOURCES = "resource_usage.json"
 
 
@@ -104,6 +107,7 @@ def _demangle(records: list[dict]) -> None:
 def check_resources(records: list[dict]) -> list[str]:
     """Problems with the compiled kernels' resources (empty = fine):
     - a multi-pass kernel (k_*_wide) that spills (they are launched without a resource check);
+    - an exact-row form that spills (launched without a resource check too);
     - a kernel built with the four-waves request that spills or misses four waves per SIMD;
     - no kernel matching one of those requests (a renamed kernel would escape the check).
     Register-resident kernels may spill at 8 or 16 vectors per lane: the launch code skips
@@ -113,6 +117,8 @@ def check_resources(records: list[dict]) -> list[str]:
         k = r.get("kernel", r["mangled"])
         if "_wide<" in k and r.get("scratch", 0) != 0:
             bad.append(f"multi-pass kernel spills {r['scratch']} B/lane: {k}")
+        if re.search(EXACT_KERNELS, k) and r.get("scratch", 0) != 0:
+            bad.append(f"exact-row kernel spills {r['scratch']} B/lane: {k}")
     for pat in FOUR_WAVE_KERNELS:
         hits = [r for r in records if re.search(pat, r.get("kernel", ""))]
         if not hits:

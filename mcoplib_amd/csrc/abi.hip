@@ -163,17 +163,6 @@ bool row_fits(int64_t hidden, int vec, KernelOfNv kernels, int min_tpr) {
 
 bool split_rows_enabled() { return g_no_split == 0; }
 
-bool exact_form_ok(const void* ex_kernel) {
-  const KernelInfo k = kernel_info(ex_kernel);
-  if (k.ok && !k.spills) return true;
-  if (trace_enabled()) {
-    fprintf(stdout, "[mcop]   exact-row form %s: generic form\n",
-            k.ok ? "spills registers" : "has no attributes");
-    fflush(stdout);
-  }
-  return false;
-}
-
 __global__ void __launch_bounds__(256) k_fill_u64(uint64_t* __restrict__ p, int64_t n,
                                                    uint64_t last) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -23,17 +23,13 @@ namespace mcop {
 
 // With eight vectors a lane the kernel asks for four waves per SIMD (at most 128 VGPRs, met
 // without spilling; 138 and three waves left free): rows of 20480-24576 bf16 elements ran 5-9%
-// faster.  fp16 would spill under that bound and keeps the default, and so does the bf16 EX form
-// (at most 256 rows at this width: one workgroup a CU whatever its registers).  The fp32 EX form
-// is to beat the generic one's four waves or give way to it: it asks for five, which it misses by
-// two registers, so its rows take the generic form.
+// faster.  fp16 would spill under that bound and keeps the default, and so do the EX forms (at most
+// 256 rows at this width: one workgroup a CU whatever their registers).
 // EX (exact): one row per workgroup and every lane in the row (tpr == blockDim.x, NV * tpr ==
 // hidden / VEC): uniform row index, scalar base addresses with 32-bit offsets, no bounds tests.
 template <class E, int NV, int FORM>
 __host__ __device__ constexpr int h1_waves() {
-  if (NV != 8 || FORM == FORM_RAGGED || std::is_same<E, F16>::value) return 1;
-  if (FORM != FORM_EXACT) return 4;
-  return std::is_same<E, F32>::value ? 5 : 1;
+  return NV == 8 && FORM == FORM_ROWS && !std::is_same<E, F16>::value ? 4 : 1;
 }
 template <class E, int VEC, int NV, int FORM = FORM_ROWS>
 __global__ void __launch_bounds__(max_tpr(VEC, NV))
@@ -347,26 +343,25 @@ static void launch_nv(const Geometry& g, void* x, int64_t xs, void* res, const v
     }
   } else {
     // exact rows (one row per workgroup, every lane in it): the EX form at two vectors a lane,
-    // and at four or eight on the latency path (at most 256 rows)
-    // (and only when that form keeps its registers)
+    // and at four or eight on the latency path (at most 256 rows; fp32 at eight at most 32: us of
+    // eight replayed calls, generic and EX: 1 x 10240 34.1 and 30.5, 8 x 14336 46.8 and 45.3,
+    // 32 x 16384 56.4 and 56.6, 64 x 16384 59.7 and 61.1, 256 x 16384 101.3 and 102.8)
+    const int few = std::is_same<E, F32>::value && g.nv == 8 ? 32 : 256;
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == hidden / VEC &&
-                    (g.nv == 2 || rows <= 256);
-#define MCOP_EX(NVV) \
-  (ex && exact_form_ok(reinterpret_cast<const void*>(&k_fused_add_rms_norm<E, VEC, NVV, FORM_EXACT>)))
+                    (g.nv == 2 || rows <= few);
     switch (g.nv) {
       case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
       case 2:
-        if (MCOP_EX(2)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
         break;
       case 4:
-        if (MCOP_EX(4)) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
         break;
       case 8:
-        if (MCOP_EX(8)) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
         break;
       default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
-#undef MCOP_EX
   }
 #undef MCOP_LAUNCH
 }

@@ -384,25 +384,22 @@ static void launch_nv(const Geometry& g, const PtqArgs& a, hipStream_t st) {
     }
   } else {
     // exact rows (one row per workgroup, every lane in it): the EX form at two vectors a lane,
-    // and at four or eight on the latency path (at most 256 rows), when it keeps its registers
+    // and at four or eight on the latency path (at most 256 rows)
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == a.hidden / VEC &&
                     (g.nv == 2 || a.rows <= 256);
-#define MCOP_EX(NVV)                                                                           \
-  (ex && exact_form_ok(reinterpret_cast<const void*>(&k_per_token_quant<E, VEC, NVV, MODE, FORM_EXACT>)))
     switch (g.nv) {
       case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
       case 2:
-        if (MCOP_EX(2)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
         break;
       case 4:
-        if (MCOP_EX(4)) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
         break;
       case 8:
-        if (MCOP_EX(8)) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
         break;
       default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
-#undef MCOP_EX
   }
 #undef MCOP_LAUNCH
 }

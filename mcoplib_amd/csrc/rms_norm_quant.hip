@@ -530,27 +530,22 @@ static void launch_nv(const Geometry& g, void* out, float* scales, const void* x
     // takes more registers (fewer resident waves) for no gain on bandwidth-bound shapes.  The
     // 7168 chain's rows (896 vectors) are exact only at two vectors over 448 lanes.
     constexpr bool wide_ex = MODE != QM_MC_7168;
-    // The EX form only when it keeps its registers.
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == hidden / VEC &&
                     (g.nv == 2 || (wide_ex && rows <= 256));
-#define MCOP_EX(NVV, EXX)                                                                      \
-  (ex && exact_form_ok(                                                                        \
-             reinterpret_cast<const void*>(&k_rms_norm_quant<E, VEC, NVV, FP8, RES, MODE, EXX>)))
     constexpr int kWideForm = wide_ex ? FORM_EXACT : FORM_ROWS;
     switch (g.nv) {
       case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
       case 2:
-        if (MCOP_EX(2, FORM_EXACT)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
         break;
       case 4:
-        if (MCOP_EX(4, kWideForm)) MCOP_LAUNCH(4, kWideForm); else MCOP_LAUNCH(4, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(4, kWideForm); else MCOP_LAUNCH(4, FORM_ROWS);
         break;
       case 8:
-        if (MCOP_EX(8, kWideForm)) MCOP_LAUNCH(8, kWideForm); else MCOP_LAUNCH(8, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(8, kWideForm); else MCOP_LAUNCH(8, FORM_ROWS);
         break;
       default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
-#undef MCOP_EX
   }
 #undef MCOP_LAUNCH
 }

@@ -846,11 +846,6 @@ bool choose_geometry(const char* op, int64_t rows, int64_t hidden, int vec, Kern
 // kernel compiled without spilling registers.  Other rows take the operator's multi-pass kernel.
 bool row_fits(int64_t hidden, int vec, KernelOfNv kernels, int min_tpr = 16);
 
-// True when the exact-row (EX) instantiation `ex_kernel` may replace the generic one the launch
-// shape was chosen for: it compiled without spilling registers.  Otherwise the launch keeps the
-// generic form, which choose_geometry has already checked.
-bool exact_form_ok(const void* ex_kernel);
-
 // Whether rows too wide for the register-resident kernels may take a split-row kernel (rows
 // shared by several workgroups, split_row.h): on unless the calling thread switched it off with
 // mcop_debug_set_split_rows (then they take the multi-pass kernels, as graph captures do).

@@ -280,10 +280,12 @@ k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   // vector: held from the start they took half the registers (bf16 at eight vectors with fp32
   // smooth scales: 216 against 163; 2048 rows of 20480 and 32768 ran 81.6 and 98.8 us, now 73.9
   // and 92.2).  At four they only are for fp16 with both in fp32, which would spend a third
-  // wave's registers on them; bf16 ran 5% slower so.
-  constexpr bool late = !EX && VEC == 8 &&
-                        (NV >= 8 || (NV == 4 && std::is_same_v<E, F16> &&
-                                     sizeof(typename EW::S) + sizeof(typename ES::S) == 8));
+  // wave's registers on them; bf16 ran 5% slower so.  The EX form, whose few rows wait for their
+  // loads, holds them wherever it can: fp16 at eight vectors spills as soon as one is in fp32.
+  constexpr int kSharedBytes = sizeof(typename EW::S) + sizeof(typename ES::S);
+  constexpr bool late =
+      VEC == 8 && (EX ? NV >= 8 && std::is_same_v<E, F16> && kSharedBytes > 4
+                      : NV >= 8 || (NV == 4 && std::is_same_v<E, F16> && kSharedBytes == 8));
   WVec<EW, VEC> wv[late ? 1 : NV];
   WVec<ES, VEC> sv[late ? 1 : NV];
   if constexpr (!late) {
@@ -571,25 +573,20 @@ static void launch_nv(const Geometry& g, const Args& a, hipStream_t st) {
     // exact rows (one row per workgroup, every lane in it) on the latency path (at most 256
     // rows) take the EX form; bandwidth-bound shapes keep the generic one (a uniform-row form
     // measured slower at cfg 4's width)
-    // (and only when the EX form keeps its registers)
     const bool ex = g.rpb == 1 && (int64_t)g.nv * g.tpr == a.hidden / VEC && a.rows <= 256;
-#define MCOP_EX(NVV)                                                                           \
-  (ex && exact_form_ok(reinterpret_cast<const void*>(                                          \
-             &k_rms_norm_smooth_quant<E, EW, ES, VEC, NVV, FP8, RES, FORM_EXACT>)))
     switch (g.nv) {
       case 1: MCOP_LAUNCH(1, FORM_ROWS); break;
       case 2:
-        if (MCOP_EX(2)) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(2, FORM_EXACT); else MCOP_LAUNCH(2, FORM_ROWS);
         break;
       case 4:
-        if (MCOP_EX(4)) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(4, FORM_EXACT); else MCOP_LAUNCH(4, FORM_ROWS);
         break;
       case 8:
-        if (MCOP_EX(8)) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
+        if (ex) MCOP_LAUNCH(8, FORM_EXACT); else MCOP_LAUNCH(8, FORM_ROWS);
         break;
       default: MCOP_LAUNCH(16, FORM_ROWS); break;
     }
-#undef MCOP_EX
   }
 #undef MCOP_LAUNCH
 }

@@ -54,6 +54,9 @@ def test_resource_check_catches_spills():
     wide = {"kernel": "void mcop::k_rms_norm_quant_wide<mcop::F16, 8, true, false, 0>(...)",
             "mangled": "z", "scratch": 16, "occupancy": 4}
     assert any("multi-pass" in p for p in b.check_resources(oks + [wide]))
+    exact = {"kernel": "void mcop::k_rms_norm_smooth_quant<mcop::F16, mcop::F32, mcop::F16, 8, 8, "
+                       "true, true, 1>(...)", "mangled": "e", "scratch": 60, "occupancy": 2}
+    assert any("exact-row" in p for p in b.check_resources(oks + [exact]))
     spilled = dict(ok_four, scratch=20)
     assert any("four-waves" in p for p in b.check_resources([spilled, ok_h1, ok_split]))
     three = dict(ok_h1, occupancy=3)
