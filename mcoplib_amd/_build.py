@@ -108,6 +108,7 @@ def check_resources(records: list[dict]) -> list[str]:
     """Problems with the compiled kernels' resources (empty = fine):
     - a multi-pass kernel (k_*_wide) that spills (they are launched without a resource check);
     - an exact-row form that spills (launched without a resource check too);
+    - a split-row kernel that spills (the planner passes those over: nothing would launch it);
     - a kernel built with the four-waves request that spills or misses four waves per SIMD;
     - no kernel matching one of those requests (a renamed kernel would escape the check).
     Register-resident kernels may spill at 8 or 16 vectors per lane: the launch code skips
@@ -119,6 +120,8 @@ def check_resources(records: list[dict]) -> list[str]:
             bad.append(f"multi-pass kernel spills {r['scratch']} B/lane: {k}")
         if re.search(EXACT_KERNELS, k) and r.get("scratch", 0) != 0:
             bad.append(f"exact-row kernel spills {r['scratch']} B/lane: {k}")
+        if "_split<" in k and r.get("scratch", 0) != 0:
+            bad.append(f"split-row kernel spills {r['scratch']} B/lane: {k}")
     for pat in FOUR_WAVE_KERNELS:
         hits = [r for r in records if re.search(pat, r.get("kernel", ""))]
         if not hits:

@@ -486,8 +486,10 @@ static int launch_split(const char* name, const GqArgs& a, hipStream_t st) {
   using S = typename E::S;
   auto fn = [](auto k) { return reinterpret_cast<const void*>(k); };
   const int gv = a.group / VEC;
-  const SplitKernel k8{fn(&k_rms_norm_group_quant_split<E, VEC, 8, FP8, RES>), 8, kSplitLanes,
-                       gv};
+  // fp8 codes of 16-bit rows would spill at eight vectors under the four-waves request
+  constexpr int most = FP8 && sizeof(S) == 2 ? 4 : 8;
+  const SplitKernel k8{fn(&k_rms_norm_group_quant_split<E, VEC, most, FP8, RES>), most,
+                       kSplitLanes, gv};
   const SplitKernel k4{fn(&k_rms_norm_group_quant_split<E, VEC, 4, FP8, RES>), 4, kSplitLanes,
                        gv};
   return split_run(name, {k8, k4}, a.rows, a.hidden / VEC, nullptr, st,

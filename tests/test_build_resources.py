@@ -57,6 +57,9 @@ def test_resource_check_catches_spills():
     exact = {"kernel": "void mcop::k_rms_norm_smooth_quant<mcop::F16, mcop::F32, mcop::F16, 8, 8, "
                        "true, true, 1>(...)", "mangled": "e", "scratch": 60, "occupancy": 2}
     assert any("exact-row" in p for p in b.check_resources(oks + [exact]))
+    split = {"kernel": "void mcop::k_rms_norm_group_quant_split<mcop::F16, 8, 8, true, true>(...)",
+             "mangled": "g", "scratch": 40, "occupancy": 4}
+    assert any("split-row" in p for p in b.check_resources(oks + [split]))
     spilled = dict(ok_four, scratch=20)
     assert any("four-waves" in p for p in b.check_resources([spilled, ok_h1, ok_split]))
     three = dict(ok_h1, occupancy=3)
