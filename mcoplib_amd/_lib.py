@@ -47,14 +47,16 @@ def _load() -> ctypes.CDLL:
     lib.mcop_vllm_rms_norm.argtypes = [P, P, P, I64, I64, I, I64, I64, I64, I64, I64, I, F, P]
     lib.mcop_rms_norm_dynamic_per_token_quant_custom.argtypes = [P, P, P, P, P, P, I64, I64, I,
                                                                   F, P]
+    lib.mcop_check_row_scalars.argtypes = [P, ctypes.c_uint32, I64, I, F, P]
     lib.mcop_debug_set_launch_override.argtypes = [I, I]
     lib.mcop_debug_set_split_rows.argtypes = [I]
     lib.mcop_debug_fail_split_waits.argtypes = [I]
     for fn in ("mcop_fused_add_rms_norm", "mcop_rms_norm_dynamic_per_token_quant",
                "mcop_rms_norm_dynamic_per_token_quant_noalloc",
                "mcop_rms_norm_smooth_quant", "mcop_scale_dynamic_quant",
-               "mcop_fp8_e4m3fn_from_f32", "mcop_debug_set_launch_override",
-               "mcop_debug_set_split_rows", "mcop_debug_fail_split_waits", "mcop_abi_version",
+               "mcop_fp8_e4m3fn_from_f32", "mcop_check_row_scalars",
+               "mcop_debug_set_launch_override", "mcop_debug_set_split_rows",
+               "mcop_debug_fail_split_waits", "mcop_abi_version",
                "mcop_dynamic_scaled_int8_quant", "mcop_dynamic_per_token_scaled_fp8_quant",
                "mcop_fused_add_rms_norm_dynamic_per_token_quant_padding_output",
                "mcop_rms_norm_per_block_quant", "mcop_rms_norm", "mcop_head_rms_norm",

@@ -20,6 +20,22 @@ extern "C" {
  * conversion can be checked bit for bit against the OCP fp8 definition. */
 int mcop_fp8_e4m3fn_from_f32(uint8_t* out, const float* in, int64_t n, float mul, void* stream);
 
+/* Counts, over the n binary32 values a whose bit patterns start at `first` (n a multiple of 256,
+ * first + n <= 2^32), the results of the row kernels' short scalar sequences that are not bit for
+ * bit the correctly rounded ones; adds to mismatches[MCOP_SCALAR_COUNT]. */
+enum {
+  MCOP_SCALAR_RCP = 0,         /* 1 / a */
+  MCOP_SCALAR_DIV_127 = 1,     /* a / 127, a / 448 */
+  MCOP_SCALAR_DIV_448 = 2,
+  MCOP_SCALAR_RATIO_127 = 3,   /* 127 / a */
+  MCOP_SCALAR_FLOORED_127 = 4, /* max(a / 127, FLT_EPSILON), max(a / 448, 1 / 229376) */
+  MCOP_SCALAR_FLOORED_448 = 5,
+  MCOP_SCALAR_INV_RMS = 6,     /* 1 / sqrt(a / hidden + epsilon), each step rounded */
+  MCOP_SCALAR_COUNT = 7
+};
+int mcop_check_row_scalars(uint64_t* mismatches, uint32_t first, int64_t n, int hidden,
+                           float epsilon, void* stream);
+
 /* Forces the launch shape of the row kernels for later calls made BY THE CALLING THREAD only,
  * for the tests that check results do not depend on the launch shape and for tuning sweeps.
  * Other threads keep the automatic choice. vectors_per_lane in {0,1,2,4,8,16}, lanes_per_row in

@@ -519,9 +519,10 @@ __device__ __forceinline__ Codes<N> fp8_quotient_codes(const float* a, float b, 
 // else of the row overlaps with on the latency path, so each is the shortest sequence that gives
 // the correctly rounded binary32 result.  The compiler's own division takes 10 instructions and
 // its binary64 square root 22 of twice the latency; the forms below take 3 and 7.  They are
-// Newton steps from the hardware's approximations, and were compared with the IEEE operations
-// over every binary32 value of the domains stated (1.7e9 values each): no difference.  Outside
-// these domains (wave-uniform branches: the values are the row's) the IEEE operations stand.
+// Newton steps from the hardware's approximations, each with a final step from the exact remainder
+// (Markstein, IBM J. Res. Dev. 34(1), 1990), and are compared with the correctly rounded forms of
+// numerics.h over every positive binary32 value (scalar_check.hip).  Outside the domains stated
+// (wave-uniform branches: the values are the row's) the IEEE operations stand.
 constexpr float kRowMin = 0x1p-100f, kRowMax = 0x1p100f;
 
 // RN(1/b) for b in [2^-100, 2^100].

@@ -1,13 +1,14 @@
 """The per-row scalars and row reductions against the CPU oracle where they can go wrong: every
 number of waves a row can have (1 to 16, with one and two rows a workgroup), and rows whose sum of
-squares, root or scale falls on either side of the short sequences' domains."""
+squares, root or scale falls on either side of the short sequences' domains; and the sequences
+themselves over every positive binary32 value."""
 
 import pytest
 import torch
 
 import oracle
 import mcoplib_amd._C  # noqa: F401  (registers torch.ops._C.*)
-from mcoplib_amd import op
+from mcoplib_amd import _lib, op
 from gpu_util import DEV, assert_codes, assert_exact, assert_scales, randn, weight
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +57,19 @@ def test_domains_of_the_short_sequences(exponent, eps, qdt):
     assert_exact(an, an_ref, "H4 after_norm")
     assert_scales(s, s_ref, "H4 scales")
     assert_codes(q, q_ref, "H4 codes")
+
+
+SCALARS = ("1/a", "a/127", "a/448", "127/a", "max(a/127, eps)", "max(a/448, 1/229376)", "1/rms")
+
+
+# hidden 1 and eps 0: the root of every value; the others: the quotient by a row's width (powers of
+# two, odd, the narrowest and widest) and its sum with the usual eps
+@pytest.mark.parametrize("hidden,eps", [(1, 0.0), (1, 1e-6), (3, 0.0), (67, 1e-6), (128, 1e-6),
+                                        (4096, 1e-5), (5120, 1e-6), (5137, 1e-6), (7168, 0.0),
+                                        (65535, 1e-6), (131072, 1e-6), (4194303, 0.0)])
+def test_short_sequences_over_every_positive_value(hidden, eps):
+    bad = torch.zeros(len(SCALARS), dtype=torch.int64, device=DEV)
+    _lib.check(_lib.lib.mcop_check_row_scalars(bad.data_ptr(), 0, 1 << 31, hidden, eps,
+                                               _lib.stream_of(bad)))
+    torch.cuda.synchronize()
+    assert dict(zip(SCALARS, bad.tolist())) == dict.fromkeys(SCALARS, 0)
