@@ -301,8 +301,13 @@ at::TensorOptions with_dtype(const Tensor& t, py::handle dtype) {
 std::tuple<Tensor, Tensor> custom_new(const Tensor& input, const Tensor& weight, double epsilon,
                                       py::object quant_dtype, const OptTensor& scale_ub,
                                       const OptTensor& residual) {
-  Tensor out = at::empty_like(input, with_dtype(input, quant_dtype));
-  Tensor scales = at::empty({rows_of(input).first, 1}, input.options().dtype(at::kFloat));
+  const at::TensorOptions opts = with_dtype(input, quant_dtype);
+  Tensor out, scales;
+  {
+    const py::gil_scoped_release allocating;  // it may wait for the device
+    out = at::empty_like(input, opts);
+    scales = at::empty({rows_of(input).first, 1}, input.options().dtype(at::kFloat));
+  }
   op_custom(out, input, weight, scales, epsilon, scale_ub, residual);
   return {out, scales};
 }
@@ -314,10 +319,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> padded_new(const Tensor& inpu
   const int64_t T = rows_of(input).first;
   std::vector<int64_t> shape = input.sizes().vec();
   shape.back() = pad_size;
-  Tensor output = at::empty(shape, input.options().dtype(at::kBFloat16));
-  Tensor rms = at::empty_like(input);
-  Tensor q = at::empty_like(input, input.options().dtype(at::kChar));
-  Tensor scales = at::empty({T, 1}, input.options().dtype(at::kFloat));
+  Tensor output, rms, q, scales;
+  {
+    const py::gil_scoped_release allocating;
+    output = at::empty(shape, input.options().dtype(at::kBFloat16));
+    rms = at::empty_like(input);
+    q = at::empty_like(input, input.options().dtype(at::kChar));
+    scales = at::empty({T, 1}, input.options().dtype(at::kFloat));
+  }
   Tensor bytes = output.view(at::kChar);
   op_padded(bytes, rms, q, scales, input, residual, weight, pad_size, epsilon);
   return {output, residual, rms, q, scales};

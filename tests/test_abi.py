@@ -201,3 +201,40 @@ def test_c_caller_library_links_the_abi():
               "mcop_rms_norm_smooth_quant", "mcop_scale_dynamic_quant", "mcop_last_error",
               "hipStreamCreate", "hipMalloc"):
         assert n in syms, n
+
+
+def test_custom_ops_allocate_without_the_interpreter_lock():
+    """Other threads run while an output is allocated, as under torch.empty: an allocation may wait
+    for the device.  (On the CPU, which the operators then refuse: filling new memory takes the
+    time there that the device would.)"""
+    import threading
+    import time
+
+    w = torch.ones(512, dtype=torch.bfloat16)
+    x = torch.empty(1 << 20, 512, dtype=torch.bfloat16)
+    calls = [lambda: custom_ops.rms_norm_dynamic_per_token_quant(x, w, 1e-6, torch.int8),
+             lambda: custom_ops.fused_add_rms_norm_dynamic_per_token_quant_padding_output(
+                 x, x, w, 512, 1e-6)]
+    for call in calls:
+        ticks, done = [], threading.Event()
+
+        def tick():
+            while not done.is_set():
+                ticks.append(time.perf_counter())
+                time.sleep(0.001)
+
+        thread = threading.Thread(target=tick)
+        torch.use_deterministic_algorithms(True)  # torch fills the memory that it allocates
+        thread.start()
+        try:
+            start = time.perf_counter()
+            with pytest.raises(RuntimeError, match="CUDA"):
+                call()
+            took = time.perf_counter() - start
+        finally:
+            torch.use_deterministic_algorithms(False)
+            done.set()
+            thread.join()
+        within = [start, *(t for t in ticks if start < t < start + took), start + took]
+        longest = max(b - a for a, b in zip(within, within[1:]))
+        assert took > 0.02 and longest < took / 2, (took, longest)
