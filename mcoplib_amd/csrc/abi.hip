@@ -134,9 +134,8 @@ int blocks_per_cu(const void* kernel, int block) {
 //     wave slots empty); 8 or 16 only for rows that do not fit otherwise.  Kernels that spill
 //     registers are skipped while another shape fits.
 // Rows that are not whole aligned vectors (hidden not a multiple of the vector width, odd strides
-// or misaligned pointers): the same search over the ragged kernels, nv in {1,2,4,8}.  Only a row
-// narrower than one vector (and the group kernel's element-wise form, nv in {4,16}) is taken an
-// element at a time.
+// or misaligned pointers): the same search over the ragged kernels, nv in {1,2,4,8}, or one element
+// at a time with nv = 4 (ragged_rows; the group kernel's element-wise form has nv in {4,16}).
 // Lanes per row for n lanes of work: whole waves, or 16 / 32 lanes when the row is that short.
 static int64_t row_lanes(int64_t n, int min_tpr) {
   if (n <= 32 && min_tpr <= 32) return n <= 16 && min_tpr <= 16 ? 16 : 32;
@@ -162,6 +161,35 @@ bool row_fits(int64_t hidden, int vec, KernelOfNv kernels, int min_tpr) {
 }
 
 bool split_rows_enabled() { return g_no_split == 0; }
+
+// The ragged form needs a whole vector.  For fp32 (four elements a vector) it is the better one from
+// there on, except for few rows of a width where two vectors a lane leave a row one or two waves (at
+// most 256 rows; us, element-wise and ragged: 1 x 513 norm with after_res 2.8 and 3.0, 256 x 769 3.6
+// and 3.7, 1 x 1281 3.1 and 3.0).  For 16-bit rows of at most 4096 elements, which the element-wise form
+// holds at four a lane, that form spreads a row over up to eight times the lanes and is better
+//   - for the narrowest rows, whose few vectors leave most lanes idle (us, element-wise and ragged:
+//     16384 x 17 bf16 add + norm 4.3 and 4.7, SmoothQuant 16384 x 33 5.5 and 6.0);
+//   - for few rows (at most 256) at two vectors a lane (1 x 1025 add + norm 2.6 and 3.0, 256 x 1025
+//     fp8 with a residual 4.2 and 4.7; 256 x 2305 the same; 1 x 3073 3.2 and 3.0);
+//   - where the ragged form has at most a wave for each SIMD of the chip (1024) and much to do for
+//     a row: SmoothQuant (300 x 769 4.9 and 8.1, 1024 x 1025 6.9 and 8.5, 1024 x 2305 12.7 and
+//     10.9), and half that with after_res (300 x 769 4.0 and 5.0, 1024 x 1281 5.9 and 5.6).  Its rows
+//     of 257-512 elements, a whole wave at one vector a lane, are the same either way.
+bool ragged_rows(int64_t rows, int64_t hidden, int vec, RowWork work) {
+  if (hidden < vec) return false;
+  if (hidden > 4096) return true;
+  if (vec < 8) return work == ROW_QUANT || rows > 256 || hidden <= 512 || hidden > 1024;
+  if (hidden <= (work == ROW_SMOOTH ? 64 : 32)) return false;
+  if (work == ROW_QUANT) return true;
+  const bool one_vector = hidden <= 64 * vec;  // a lane, so up to a wave a row
+  if (rows <= 256 && !one_vector && hidden <= 2048) return false;
+  const int64_t nvec = ceil_div(hidden, vec);
+  const int64_t lanes = row_lanes(ceil_div(nvec, one_vector ? 1 : rows <= 256 ? 2 : 4), 16);
+  const int64_t waves = rows * lanes / 64;
+  if (work == ROW_SMOOTH) return waves > 1024 || (one_vector && hidden > 256);
+  if (work == ROW_NORM_AFTER_RES) return waves > 512 || one_vector || rows <= 256;
+  return true;
+}
 
 __global__ void __launch_bounds__(256) k_fill_u64(uint64_t* __restrict__ p, int64_t n,
                                                    uint64_t last) {

@@ -47,11 +47,11 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
     p = row_pos(rows, tpr);
   }
   const int nvec = vec_count<FORM, VEC>(hidden);
-  const bool apart = FORM == FORM_RAGGED && vec_apart(nvec, tpr);
+  const bool swap = vec_swap<FORM>(nvec, tpr);
   const int64_t xbase = p.row * x_stride, xlbase = p.lrow * x_stride;
   const int64_t rbase = p.row * (int64_t)hidden, rlbase = p.lrow * (int64_t)hidden;
   auto lj_of = [&](int v) {
-    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), nvec, hidden);
+    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), swap, nvec, hidden);
   };
 
   Pack<S, VEC> xv[NV], rv[NV], wv[NV];
@@ -75,9 +75,6 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, slt);
     const bool in = EX || j < nvec;
-    const int skip = vec_skip<FORM, VEC>(j, hidden);
-    trim<FORM>(xv[v], skip, apart);
-    trim<FORM>(rv[v], skip, apart);
     Pack<S, VEC> o;
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
 #pragma unroll
@@ -88,9 +85,9 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
       const double d = (double)t;
       vs = __builtin_fma(d, d, vs);
     }
-    vs = own_squares<FORM, E, VEC, false>(vs, o, o, skip);
+    vs = own_squares<FORM, E, VEC, false>(vs, o, o, j, swap, nvec, hidden);
     ss += in ? vs : 0.0;
-    if (p.live && in) stf_nt<FORM>(row_elem<EX>(res, rbase, (int64_t)j * VEC - skip), o, skip, apart);
+    if (p.live && in) stf_nt<FORM>(row_elem<EX>(res, rbase, vec_at<FORM, VEC>(j, swap, nvec, hidden)), o);
   }
 
   if constexpr (w_early < NV) {
@@ -106,9 +103,8 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, slt);
     if (p.live && (EX || j < nvec)) {
-      const int skip = vec_skip<FORM, VEC>(j, hidden);
-      stf_nt<FORM>(row_elem<EX>(x, xbase, (int64_t)j * VEC - skip),
-                   norm_store<E, VEC>(z[v], rho, wv[v]), skip, apart);
+      stf_nt<FORM>(row_elem<EX>(x, xbase, vec_at<FORM, VEC>(j, swap, nvec, hidden)),
+                   norm_store<E, VEC>(z[v], rho, wv[v]));
     }
   }
 }
@@ -329,8 +325,12 @@ static void launch_nv(const Geometry& g, void* x, int64_t xs, void* res, const v
   auto* xp = static_cast<S*>(x);
   auto* rp = static_cast<S*>(res);
   auto* wp = static_cast<const S*>(w);
+  // ragged fp32 rows of two or more waves: at most five of these workgroups on a CU (16384 x 2049
+  // 107.0 us uncapped and 100.4 so, 1793 85.3 and 83.3; 513, a row a wave, 26.8 and 28.0)
+  const bool capped = RAG && std::is_same<E, F32>::value && g.nv == 4 && g.tpr >= 128;
+  const unsigned lds = resident_cap(capped ? 5 : 0, g.blocks);
 #define MCOP_LAUNCH(NVV, EXX)                                                                   \
-  hipLaunchKernelGGL((k_fused_add_rms_norm<E, VEC, NVV, EXX>), grid, block, 0, st, xp, xs, rp, wp, \
+  hipLaunchKernelGGL((k_fused_add_rms_norm<E, VEC, NVV, EXX>), grid, block, lds, st, xp, xs, rp, wp, \
                      rows, hidden, g.tpr, eps)
   if constexpr (VEC == 1) {
     MCOP_LAUNCH(4, FORM_ROWS);
@@ -417,8 +417,8 @@ static int dispatch(void* x, int64_t xs, void* res, const void* w, int64_t rows,
                     float eps, hipStream_t st) {
   constexpr int V = E::VEC;
   const bool vec_ok = hidden % V == 0 && xs % V == 0 && aligned(16, x, res, w);
-  // any other row of at least one vector takes the ragged form, narrower ones one element a load
-  const bool rag = !vec_ok && hidden >= V;
+  // other rows take the ragged form or one element a load (ragged_rows)
+  const bool rag = !vec_ok && ragged_rows(rows, hidden, V, ROW_NORM);
   const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels = vec_ok ? &kernel_of<E, V>
                              : rag  ? &kernel_of<E, V, true>

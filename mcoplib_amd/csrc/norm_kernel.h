@@ -124,14 +124,14 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* ares, RowIn<E, RES> x
     p = row_pos(rows, tpr);
   }
   const int nvec = vec_count<FORM, VEC>(hidden);
-  // after_res may be the residual or the input itself: the last vector apart, as in place
-  const bool apart = FORM == FORM_RAGGED && RES && vec_apart(nvec, tpr);
+  // after_res may be the buffer of x or of the residual
+  const bool swap = RES && vec_swap<FORM>(nvec, tpr);
   const RowOffsets lo = row_offsets(map, p.lrow);
   const int64_t out_base = p.row == p.lrow ? lo.out : 0;
   const int64_t rbase = p.row * (int64_t)hidden;
   const int64_t lrbase = p.lrow * (int64_t)hidden;
   auto lj_of = [&](int v) {
-    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), nvec, hidden);
+    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), swap, nvec, hidden);
   };
 
   Pack<S, VEC> xv[NV], rv[NV];
@@ -154,11 +154,6 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* ares, RowIn<E, RES> x
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
     const bool in = EX || j < nvec;
-    const int skip = vec_skip<FORM, VEC>(j, hidden);
-    if constexpr (RES) {
-      trim<FORM>(xv[v], skip, apart);
-      trim<FORM>(rv[v], skip, apart);
-    }
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
     Pack<S, VEC> o;
 #pragma unroll
@@ -174,11 +169,11 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* ares, RowIn<E, RES> x
       }
       a[v][e] = t;
     }
-    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], skip);
+    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], j, swap, nvec, hidden);
     ss += in ? vs : 0.0;
     if constexpr (RES) {
       if (p.live && in) {
-        stf_nt<FORM>(row_elem<EX>(ares, rbase, (int64_t)j * VEC - skip), o, skip, apart);
+        stf_nt<FORM>(row_elem<EX>(ares, rbase, vec_at<FORM, VEC>(j, swap, nvec, hidden)), o);
       }
     }
   }
@@ -236,8 +231,7 @@ k_rms_norm(typename E::S* __restrict__ out, typename E::S* ares, RowIn<E, RES> x
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(n[e] * wv[v].at(e));
     }
-    const int skip = vec_skip<FORM, VEC>(j, hidden);
-    stf_nt<FORM>(row_elem<EX>(out, out_base, (int64_t)j * VEC - skip), o, skip, apart);
+    stf_nt<FORM>(row_elem<EX>(out, out_base, vec_at<FORM, VEC>(j, swap, nvec, hidden)), o);
   }
 }
 
@@ -600,8 +594,8 @@ static int norm_dispatch(const char* name, const NormArgs& a, hipStream_t st) {
   constexpr int V = E::VEC;
   const bool vec_ok = norm_vec_ok<E, EW>(a);
   const bool r = a.res != nullptr;
-  // any other row of at least one vector takes the ragged form, narrower ones one element a load
-  const bool rag = !vec_ok && a.hidden >= V;
+  // other rows take the ragged form or one element a load (ragged_rows)
+  const bool rag = !vec_ok && ragged_rows(a.rows, a.hidden, V, r ? ROW_NORM_AFTER_RES : ROW_NORM);
   const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels =
       vec_ok ? (r ? &norm_kernel_of<E, EW, V, true> : &norm_kernel_of<E, EW, V, false>)

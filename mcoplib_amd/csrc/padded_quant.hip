@@ -48,12 +48,12 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
     p = row_pos(rows, tpr);
   }
   const int nvec = vec_count<FORM, VEC>(hidden);
-  const bool apart = FORM == FORM_RAGGED && vec_apart(nvec, tpr);
+  const bool swap = vec_swap<FORM>(nvec, tpr);
   const int64_t base = p.row * (int64_t)hidden;
   const int64_t lbase = p.lrow * (int64_t)hidden;
   const int64_t pbase = p.row * pad_bytes;
   auto lj_of = [&](int v) {
-    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), nvec, hidden);
+    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), swap, nvec, hidden);
   };
 
   Pack<uint16_t, VEC> xv[NV], rv[NV], wv[NV];
@@ -76,9 +76,6 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
     const bool in = EX || j < nvec;
-    const int skip = vec_skip<FORM, VEC>(j, hidden);
-    trim<FORM>(xv[v], skip, apart);
-    trim<FORM>(rv[v], skip, apart);
     double vs = 0.0;
     float m[VEC];
     Pack<uint16_t, VEC> o;
@@ -101,9 +98,9 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
     for (int e = 0; e < VEC; ++e) {
       amax = __builtin_fmaxf(amax, (full || in) ? __builtin_fabsf(m[e]) : 0.0f);
     }
-    vs = own_squares<FORM, E, VEC, true>(vs, xv[v], rv[v], skip);
+    vs = own_squares<FORM, E, VEC, true>(vs, xv[v], rv[v], j, swap, nvec, hidden);
     ss += in ? vs : 0.0;
-    if (p.live && in) stf_nt<FORM>(row_elem<EX>(res, base, (int64_t)j * VEC - skip), o, skip, apart);
+    if (p.live && in) stf_nt<FORM>(row_elem<EX>(res, base, vec_at<FORM, VEC>(j, swap, nvec, hidden)), o);
   }
   ss = row_reduce<EX>(ss, red_sum, tpr, SumOp());
   amax = row_absmax<EX>(amax, red_max, tpr);
@@ -135,11 +132,10 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
         widen<E, VEC>(a[v], o);
       }
       const Codes<VEC> q = i8_codes<-127, VEC>(a[v], inv);
-      const int skip = vec_skip<FORM, VEC>(j, hidden);
-      const int64_t at = (int64_t)j * VEC - skip;
-      stf_nt<FORM>(row_elem<EX>(rms, base, at), o, skip, apart);
-      stf_codes_nt<FORM, VEC>(row_elem<EX>(q_out, base, at), q, skip, apart);
-      stf_codes_nt<FORM, VEC>(row_elem<EX>(padded, pbase, at), q, skip, apart);
+      const int64_t at = vec_at<FORM, VEC>(j, swap, nvec, hidden);
+      stf_nt<FORM>(row_elem<EX>(rms, base, at), o);
+      stf_codes_nt<FORM, VEC>(row_elem<EX>(q_out, base, at), q);
+      stf_codes_nt<FORM, VEC>(row_elem<EX>(padded, pbase, at), q);
     }
   }
 }
@@ -449,8 +445,8 @@ static int dispatch(const PadArgs& a, hipStream_t st) {
   const char* name = "fused_add_rms_norm_dynamic_per_token_quant_padding_output";
   const bool vec_ok = a.hidden % 8 == 0 && a.pad_bytes % 8 == 0 &&
                       aligned(16, a.x, a.res, a.w, a.rms) && aligned(8, a.q, a.padded);
-  // any other row of at least one vector takes the ragged form, narrower ones one element a load
-  const bool rag = !vec_ok && a.hidden >= 8;
+  // other rows take the ragged form or one element a load (ragged_rows)
+  const bool rag = !vec_ok && ragged_rows(a.rows, a.hidden, 8, ROW_NORM);
   const int vec = vec_ok || rag ? 8 : 1;
   const KernelOfNv kernels = vec_ok ? &kernel_of<8, OPT>
                              : rag  ? &kernel_of<8, OPT, true>

@@ -152,7 +152,7 @@ k_per_token_quant(uint8_t* __restrict__ out, float* __restrict__ scales, int32_t
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
-    xv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(x, lbase, vec_off<FORM, VEC>(j, nvec, hidden)));
+    xv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(x, lbase, vec_off<FORM, VEC>(j, false, nvec, hidden)));
   }
   // Elements past the row end are copies of the row's (read only: no effect on max or min).
   float a[NV][VEC];
@@ -177,8 +177,7 @@ k_per_token_quant(uint8_t* __restrict__ out, float* __restrict__ scales, int32_t
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, p.lt);
     if (p.live && (EX || j < nvec)) {
-      const int skip = vec_skip<FORM, VEC>(j, hidden);
-      stf_codes_nt<FORM, VEC>(row_elem<EX>(out, obase, (int64_t)j * VEC - skip),
+      stf_codes_nt<FORM, VEC>(row_elem<EX>(out, obase, vec_at<FORM, VEC>(j, false, nvec, hidden)),
                               ptq_codes<E, VEC, MODE>(a[v], r));
     }
   }
@@ -434,8 +433,8 @@ static int dispatch(const char* name, const PtqArgs& a, hipStream_t st) {
   constexpr int V = E::VEC;
   const bool vec_ok = a.hidden % V == 0 && a.in_stride % V == 0 && a.out_stride % V == 0 &&
                       aligned(16, a.x) && aligned(V, a.out);
-  // any other row of at least one vector takes the ragged form, narrower ones one element a load
-  const bool rag = !vec_ok && a.hidden >= V;
+  // other rows take the ragged form or one element a load (ragged_rows)
+  const bool rag = !vec_ok && ragged_rows(a.rows, a.hidden, V, ROW_QUANT);
   const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels = vec_ok ? &kernel_of<E, V, MODE>
                              : rag  ? &kernel_of<E, V, MODE, true>

@@ -105,10 +105,10 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     p = row_pos(rows, tpr);
   }
   const int nvec = vec_count<FORM, VEC>(hidden);
-  const bool apart = FORM == FORM_RAGGED && vec_apart(nvec, tpr);
+  const bool swap = RES && vec_swap<FORM>(nvec, tpr);
   const int64_t base = p.lrow * (int64_t)hidden;  // the lane's row, where it stores at all
   auto lj_of = [&](int v) {  // element offset of the lane's vector v (loads)
-    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), nvec, hidden);
+    return vec_off<FORM, VEC>(vec_index(v, tpr, p.lt), swap, nvec, hidden);
   };
 
   // All loads first, unconditionally (out-of-row lanes re-read vector 0 of their row).
@@ -135,11 +135,6 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   for (int v = 0; v < NV; ++v) {
     const int j = vec_index(v, tpr, slt);
     const bool in = EX || j < nvec;
-    const int skip = vec_skip<FORM, VEC>(j, hidden);
-    if constexpr (RES) {
-      trim<FORM>(xv[v], skip, apart);
-      trim<FORM>(rv[v], skip, apart);
-    }
     // Lanes past the row end hold a copy of vector 0: it must not count in the sum.
     double vs = 0.0;
 #pragma unroll
@@ -150,14 +145,14 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
       const double d = (double)t;
       vs = __builtin_fma(d, d, vs);
     }
-    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], skip);
+    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], j, swap, nvec, hidden);
     ss += in ? vs : 0.0;
     if constexpr (RES) {
       if (p.live && in) {
         Pack<S, VEC> o;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) o.v[e] = E::from_f(a[v][e]);
-        stf_nt<FORM>(row_elem<EX>(res, base, (int64_t)j * VEC - skip), o, skip, apart);
+        stf_nt<FORM>(row_elem<EX>(res, base, vec_at<FORM, VEC>(j, swap, nvec, hidden)), o);
       }
     }
   }
@@ -195,9 +190,7 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     if (p.live && (EX || j < nvec)) {
       const Codes<VEC> q =
           row_codes<E, VEC, FP8, MODE>(a[v], rho, s, inv, s_ok, bounded, scale_ub != nullptr);
-      const int skip = vec_skip<FORM, VEC>(j, hidden);
-      stf_codes_nt<FORM, VEC>(row_elem<EX>(out, base, (int64_t)j * VEC - skip), q, skip,
-                              RES && apart);
+      stf_codes_nt<FORM, VEC>(row_elem<EX>(out, base, vec_at<FORM, VEC>(j, swap, nvec, hidden)), q);
     }
   }
 }
@@ -505,12 +498,14 @@ static void launch_nv(const Geometry& g, void* out, float* scales, const void* x
   // 69.4, 16384 79.1 and 78.3; fp16 fp8 14336 73.5 and 70.4; fp32 8192 x 6144 108.5 and 104.7.
   // Smaller workgroups do not gain throughout (4096 x 8704 fp16 fp8 46.7, 49.2 at two), and rows
   // without a residual, mostly reads, want every load in flight (8192 x 8192 int8 38.0, 41.5 at
-  // three; 4096 x 16384 fp8 40.1, 41.1 at two).
+  // three; 4096 x 16384 fp8 40.1, 41.1 at two).  Ragged fp32 rows of two or more waves: five (16384 x
+  // 2049 int8 84.5 and 80.5, 3073 119.1 and 117.2; 513, a row a wave, 22.8 and 25.4).
   const int lanes = g.tpr * g.rpb;
-  const int cap = !RES || VEC == 1                              ? 0
-                  : g.nv == 2 && lanes == 512                   ? 3
-                  : g.nv == 4 && lanes >= 384 && lanes <= 512 ? 2
-                                                              : 0;
+  const int cap = !RES || VEC == 1                                             ? 0
+                  : RAG && std::is_same_v<E, F32> && g.nv == 4 && g.tpr >= 128 ? 5
+                  : g.nv == 2 && lanes == 512                                  ? 3
+                  : g.nv == 4 && lanes >= 384 && lanes <= 512                  ? 2
+                                                                               : 0;
   const unsigned lds = resident_cap(cap, g.blocks);
 #define MCOP_LAUNCH(NVV, EXX)                                                                  \
   hipLaunchKernelGGL((k_rms_norm_quant<E, VEC, NVV, FP8, RES, MODE, EXX>), grid, block, lds, st, o, \
@@ -582,8 +577,8 @@ static int dispatch(const char* name, void* out, float* scales, const void* x, c
                     hipStream_t st, uint64_t* scratch = nullptr) {
   constexpr int V = E::VEC;
   const bool vec_ok = hidden % V == 0 && aligned(16, x, w, res) && aligned(V, out);
-  // any other row of at least one vector takes the ragged form, narrower ones one element a load
-  const bool rag = !vec_ok && hidden >= V;
+  // other rows take the ragged form or one element a load (ragged_rows)
+  const bool rag = !vec_ok && ragged_rows(rows, hidden, V, ROW_NORM);
   const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels =
       vec_ok ? (res ? &kernel_of<E, V, FP8, true, MODE> : &kernel_of<E, V, FP8, false, MODE>)

@@ -184,15 +184,19 @@ __device__ __forceinline__ void widen(float* f, const Pack<typename E::S, N>& p)
 //   FORM_EXACT   the same, one row a workgroup and every lane in it
 //   FORM_RAGGED  16-byte vectors at element alignment: rows of any width >= VEC, any row stride or
 //                base address (global memory takes unaligned vectors).  A row has ceil(hidden /
-//                VEC) vectors; the last one, if it is not whole, is the row's last VEC elements, so
-//                every access stays inside the row.  Its first `skip` elements belong to the
-//                vector before: they are left out of sums, give the same maxima, and are stored
-//                twice with the same bits.  A kernel that stores over its inputs must read those
-//                elements before their owner stores them: both are in one wave's instruction,
-//                whose loads end before its stores begin, unless the last vector starts a wave's
-//                run of lanes (`apart`); then they are read as zeros and not stored.
-// Before, one element a load: 2048 x 5137 fp8 with a residual 30.6 us, 20.7 so; 4096 x 4099 norm
-// with a residual 52.6 and 33.3; 65536 x 67 norm 13.0 and 8.2; 4096 x 30001 int8 521 and 223.
+//                VEC) vectors at multiples of VEC; the last is the row's last VEC elements, so that
+//                every access stays inside the row, and overlaps the one before where the row is
+//                not whole vectors.  The overlap counts once in sums, gives the same maxima, and is
+//                stored twice with the same bits.  A kernel that stores over its inputs has both
+//                vectors in one wave's instruction, whose loads end before its stores begin: they
+//                are neighbouring lanes', and where the last would be the first of a wave's run of
+//                lanes, it changes places with the third last (`swap`).  Storing such a vector an
+//                element at a time took 20 registers a lane and up to 2 us a row.  Turning the row
+//                by two lanes, or counting the vectors from its end, moves all its loads: 5% and,
+//                for 16-bit weights then loaded from odd 2-byte addresses, 25% (16384 x 3585 bf16
+//                norm 48.8 us and 61.5).
+// Against one element a load: 2048 x 5137 fp8 with a residual 30.6 and 19.8 us; 4096 x 4099 norm with
+// a residual 52.4 and 32.1; 65536 x 67 norm 13.0 and 8.1; 4096 x 30001 int8 517 and 214.
 enum Form { FORM_ROWS = 0, FORM_EXACT = 1, FORM_RAGGED = 2 };
 
 template <int FORM, int VEC>
@@ -200,19 +204,30 @@ __device__ __forceinline__ int vec_count(int hidden) {
   return FORM == FORM_RAGGED ? (int)(((unsigned)hidden + (VEC - 1)) / VEC) : hidden / VEC;
 }
 
-// Element offset a lane's loads of vector j use; vectors past the row end re-read one of the row.
-template <int FORM, int VEC>
-__device__ __forceinline__ int64_t vec_off(int j, int nvec, int hidden) {
-  if constexpr (FORM == FORM_EXACT) return (int64_t)j * VEC;
-  if constexpr (FORM == FORM_RAGGED) return min(j * VEC, hidden - VEC);
-  return (int64_t)(j < nvec ? j : 0) * VEC;
+// Whether a row of a kernel that stores over its inputs has the two vectors' places changed (above).
+template <int FORM>
+__device__ __forceinline__ bool vec_swap(int nvec, int tpr) {
+  const int run = tpr < 64 ? tpr : 64;
+  return FORM == FORM_RAGGED && nvec > 1 && ((nvec - 1) & (run - 1)) == 0;
 }
-
-// Leading elements of the lane's vector j that are not its own (VEC or more past the row end).
+// The row's vector that lane index j holds.
+__device__ __forceinline__ int vec_of(int j, bool swap, int nvec) {
+  return swap && (j == nvec - 1 || j == nvec - 3) ? 2 * nvec - 4 - j : j;
+}
+// Element offset of that vector, and the one its loads use: lanes past the row end re-read one of
+// the row.  (The two are written differently for the ragged form so that the loads' offsets are not
+// held for the stores: 8-20 registers.)
 template <int FORM, int VEC>
-__device__ __forceinline__ int vec_skip(int j, int hidden) {
-  if constexpr (FORM != FORM_RAGGED) return 0;
-  return max(j * VEC - (hidden - VEC), 0);
+__device__ __forceinline__ int64_t vec_at(int j, bool swap, int nvec, int hidden) {
+  if constexpr (FORM != FORM_RAGGED) return (int64_t)j * VEC;
+  const int k = vec_of(j, swap, nvec);
+  return (int64_t)k * VEC - max(k * VEC - (hidden - VEC), 0);
+}
+template <int FORM, int VEC>
+__device__ __forceinline__ int64_t vec_off(int j, bool swap, int nvec, int hidden) {
+  if constexpr (FORM == FORM_EXACT) return (int64_t)j * VEC;
+  if constexpr (FORM == FORM_RAGGED) return min(vec_of(j, swap, nvec) * VEC, hidden - VEC);
+  return (int64_t)(j < nvec ? j : 0) * VEC;
 }
 
 typedef u32x4 u32x4_loose __attribute__((aligned(1)));
@@ -244,53 +259,33 @@ __device__ __forceinline__ Pack<T, N> ldf_nt(const T* p) {
   }
 }
 
-// Whether the row's last vector is apart from the one before (above): uniform over the row.
-__device__ __forceinline__ bool vec_apart(int nvec, int tpr) {
-  return ((nvec - 1) & ((tpr < 64 ? tpr : 64) - 1)) == 0;
-}
-
-// Zeroes a vector's elements that are not its own, where the last vector is apart.
+// Streaming store of one vector in a kernel's form.
 template <int FORM, class T, int N>
-__device__ __forceinline__ void trim(Pack<T, N>& p, int skip, bool apart) {
-  if constexpr (FORM == FORM_RAGGED) {
-    if (apart && __builtin_amdgcn_ballot_w64(skip > 0) != 0) {
-#pragma unroll
-      for (int e = 0; e < N; ++e) p.v[e] = e < skip ? T(0) : p.v[e];
-    }
-  }
-}
-
-// Streaming store of one vector in a kernel's form: `p` is the address of the vector as loaded.
-template <int FORM, class T, int N>
-__device__ __forceinline__ void stf_nt(T* p, const Pack<T, N>& v, int skip = 0,
-                                       bool apart = false) {
+__device__ __forceinline__ void stf_nt(T* p, const Pack<T, N>& v) {
   if constexpr (FORM != FORM_RAGGED) {
     st_nt<T, N>(p, v);
-  } else if (!apart || skip == 0) {
+  } else {
     using R = typename LooseOf<(int)sizeof(T) * N>::T;
     using A = typename RawOf<(int)sizeof(T) * N>::T;
     __builtin_nontemporal_store(__builtin_bit_cast(A, v), reinterpret_cast<R*>(p));
-  } else {
-#pragma unroll
-    for (int e = 1; e < N; ++e) {
-      if (e >= skip) p[e] = v.v[e];
-    }
   }
 }
 
-// The sum of squares `vs` of a vector's values without the elements that are not its own (behind
-// a wave-uniform branch: only the wave with the row's last vector has any).
+// The sum of squares `vs` of the vector that lane index j holds, without the elements that the vector
+// before has too (behind a wave-uniform branch: only the wave with the row's last vector has any).
 template <int FORM, class E, int N, bool RES>
 __device__ __forceinline__ double own_squares(double vs, const Pack<typename E::S, N>& x,
-                                              const Pack<typename E::S, N>& r, int skip) {
+                                              const Pack<typename E::S, N>& r, int j, bool swap,
+                                              int nvec, int hidden) {
   if constexpr (FORM == FORM_RAGGED) {
-    if (__builtin_amdgcn_ballot_w64(skip > 0) != 0) {
+    const int twice = vec_of(j, swap, nvec) * N - (hidden - N);
+    if (__builtin_amdgcn_ballot_w64(twice > 0) != 0) {
       vs = 0.0;
 #pragma unroll
       for (int e = 0; e < N; ++e) {
         float t = E::to_f(x.v[e]);
         if constexpr (RES) t += E::to_f(r.v[e]);
-        const double d = e < skip ? 0.0 : (double)t;
+        const double d = e < twice ? 0.0 : (double)t;
         vs = __builtin_fma(d, d, vs);
       }
     }
@@ -334,22 +329,13 @@ __device__ __forceinline__ void st_codes_nt(uint8_t* p, const Codes<N>& q) {
 
 // The same in a kernel's form (as stf_nt).
 template <int FORM, int N>
-__device__ __forceinline__ void stf_codes_nt(uint8_t* p, const Codes<N>& q, int skip = 0,
-                                             bool apart = false) {
+__device__ __forceinline__ void stf_codes_nt(uint8_t* p, const Codes<N>& q) {
   if constexpr (FORM != FORM_RAGGED) {
     st_codes_nt<N>(p, q);
-  } else if (!apart || skip == 0) {
-    if constexpr (N == 8) {
-      __builtin_nontemporal_store(__builtin_bit_cast(u32x2, q),
-                                  reinterpret_cast<u32x2_loose*>(p));
-    } else {
-      __builtin_memcpy(p, &q, N);
-    }
+  } else if constexpr (N == 8) {
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x2, q), reinterpret_cast<u32x2_loose*>(p));
   } else {
-#pragma unroll
-    for (int e = 1; e < N; ++e) {
-      if (e >= skip) p[e] = code_of<N>(q, e);
-    }
+    __builtin_memcpy(p, &q, N);
   }
 }
 
@@ -851,6 +837,14 @@ bool row_fits(int64_t hidden, int vec, KernelOfNv kernels, int min_tpr = 16);
 // shared by several workgroups, split_row.h): on unless the calling thread switched it off with
 // mcop_debug_set_split_rows (then they take the multi-pass kernels, as graph captures do).
 bool split_rows_enabled();
+
+// What an operator does to a row, for ragged_rows: quantizes it; normalizes it; stores after_res on
+// the way; stores after_res and after_norm and reads fp32 smooth scales (SmoothQuant).
+enum RowWork { ROW_QUANT, ROW_NORM, ROW_NORM_AFTER_RES, ROW_SMOOTH };
+
+// Whether rows that are not whole aligned vectors take the ragged form (FORM_RAGGED) rather than
+// one element a load.
+bool ragged_rows(int64_t rows, int64_t hidden, int vec, RowWork work);
 
 // Launch check of the multi-pass kernels for rows too wide for the register-resident ones
 // (one 1024-lane workgroup per row): false, with the message set, beyond 2^31 - 1 rows.

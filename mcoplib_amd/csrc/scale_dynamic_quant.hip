@@ -38,7 +38,7 @@ k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
     sv[v] = ldf<FORM, float, VEC>(
-        row_elem<true>(sm, 0, vec_off<FORM, VEC>(vec_index(v, tpr, p[0].lt), nvec, hidden)));
+        row_elem<true>(sm, 0, vec_off<FORM, VEC>(vec_index(v, tpr, p[0].lt), false, nvec, hidden)));
   }
   shared_loads_first();
   Pack<uint16_t, VEC> xv[R][NV];
@@ -48,7 +48,7 @@ k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     for (int v = 0; v < NV; ++v) {
       xv[k][v] = ldf_nt<FORM, uint16_t, VEC>(
           x + p[k].lrow * (int64_t)hidden +
-          vec_off<FORM, VEC>(vec_index(v, tpr, p[k].lt), nvec, hidden));
+          vec_off<FORM, VEC>(vec_index(v, tpr, p[k].lt), false, nvec, hidden));
     }
   }
 
@@ -81,8 +81,7 @@ k_scale_dynamic_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
       const int j = vec_index(v, tpr, p[k].lt);
       if (p[k].live && j < nvec) {
         const Codes<VEC> q = i8_codes<-128, VEC>(a[k][v], inv);
-        const int skip = vec_skip<FORM, VEC>(j, hidden);
-        stf_codes_nt<FORM, VEC>(out + base + (int64_t)j * VEC - skip, q);
+        stf_codes_nt<FORM, VEC>(out + base + vec_at<FORM, VEC>(j, false, nvec, hidden), q);
       }
     }
   }
@@ -380,8 +379,8 @@ extern "C" int mcop_scale_dynamic_quant(int8_t* out, float* scales, const void* 
   constexpr int V = BF16::VEC;
   const bool vec_ok = hidden_size % V == 0 && aligned(16, input, smooth) && aligned(V, out);
   auto st = static_cast<hipStream_t>(stream);
-  // any other row of at least one vector takes the ragged form, narrower ones one element a load
-  const bool rag = !vec_ok && hidden_size >= V;
+  // other rows take the ragged form or one element a load (ragged_rows)
+  const bool rag = !vec_ok && ragged_rows(num_tokens, hidden_size, V, ROW_NORM);
   const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels = vec_ok ? &kernel_of<V> : rag ? &kernel_of<V, true> : &kernel_of<1>;
   if (!row_fits(hidden_size, vec, kernels)) {

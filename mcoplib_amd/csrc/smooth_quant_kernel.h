@@ -53,7 +53,7 @@ __device__ __forceinline__ Codes<VEC> sq_fp8_codes(const float* v, float amax, f
 // The lane's streamed vectors of one row's slice [j0, j0 + jn) (the whole row: 0, nvec): x
 // (and the residual); lanes past the slice end load its first vector.
 template <class E, int VEC, int NV, bool RES, bool EX, bool UA = EX, int FORM = FORM_ROWS>
-__device__ __forceinline__ void sq_load(const RowPos& p, int j0, int jn,
+__device__ __forceinline__ void sq_load(const RowPos& p, int j0, int jn, bool swap,
                                         const typename E::S* x, const typename E::S* res,
                                         int hidden, int tpr, Pack<typename E::S, VEC>* xv,
                                         Pack<typename E::S, VEC>* rv) {
@@ -63,7 +63,7 @@ __device__ __forceinline__ void sq_load(const RowPos& p, int j0, int jn,
   for (int v = 0; v < NV; ++v) {
     const int k = vec_index(v, tpr, p.lt);
     const int64_t lj = FORM == FORM_RAGGED
-                           ? vec_off<FORM, VEC>(k, jn, hidden)
+                           ? vec_off<FORM, VEC>(k, swap, jn, hidden)
                            : (int64_t)(j0 + (EX ? k : load_index(k, jn))) * VEC;
     xv[v] = ldf_nt<FORM, S, VEC>(row_elem<UA>(x, lbase, lj));
     if constexpr (RES) rv[v] = ldf_nt<FORM, S, VEC>(row_elem<UA>(res, lbase, lj));
@@ -91,9 +91,9 @@ struct WgRowReduce {
 // of this operator: those three are not __restrict__.
 template <class E, class EW, class ES, int VEC, int NV, bool FP8, bool RES, bool EX, bool UA,
           bool LATE, int FORM, class Shared, class Red>
-__device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
-                                       Pack<typename E::S, VEC>* xv,
-                                       Pack<typename E::S, VEC>* rv,
+__device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn, bool swap,
+                                       const Pack<typename E::S, VEC>* xv,
+                                       const Pack<typename E::S, VEC>* rv,
                                        Shared&& shared,
                                        uint8_t* __restrict__ out, float* __restrict__ scales,
                                        typename E::S* ares,
@@ -103,8 +103,6 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
   const int64_t base = p.row * (int64_t)hidden;
 
   const int slt = EX ? p.lt : store_lane<NV>(p.lt);
-  // after_res may be the residual or the input itself: the last vector apart, as in place
-  const bool apart = FORM == FORM_RAGGED && ares != nullptr && vec_apart(jn, tpr);
   float a[NV][VEC];
   Pack<S, VEC> z[LATE ? NV : 1];
   double ss = 0.0;
@@ -114,9 +112,6 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     const int j = j0 + k;
     const bool in = EX || k < jn;
     if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
-    const int skip = vec_skip<FORM, VEC>(k, hidden);
-    trim<FORM>(xv[v], skip, apart);
-    if constexpr (RES) trim<FORM>(rv[v], skip, apart);
     Pack<S, VEC> o;
     double vs = 0.0;  // lanes past the row end (a copy of vector 0) do not count
 #pragma unroll
@@ -129,10 +124,10 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
       a[v][e] = E::to_f(o.v[e]);  // b(a): what the later passes of the reference re-read
     }
     if constexpr (LATE) z[v] = o;
-    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], skip);
+    vs = own_squares<FORM, E, VEC, RES>(vs, xv[v], rv[v], k, swap, jn, hidden);
     ss += in ? vs : 0.0;
     if (ares != nullptr && p.live && in) {
-      stf_nt<FORM>(row_elem<UA>(ares, base, (int64_t)j * VEC - skip), o, skip, apart);
+      stf_nt<FORM>(row_elem<UA>(ares, base, vec_at<FORM, VEC>(j, swap, jn, hidden)), o);
     }
   }
 
@@ -219,8 +214,7 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
     // stored after_res there before the copy was read, and the copy has the residual in it twice.
     amax = __builtin_fmaxf(amax, EX || k < jn ? vm : 0.0f);
     if (anorm != nullptr && p.live && (EX || k < jn)) {
-      const int skip = vec_skip<FORM, VEC>(k, hidden);
-      stf_nt<FORM>(row_elem<UA>(anorm, base, (int64_t)j * VEC - skip), o, skip, apart);
+      stf_nt<FORM>(row_elem<UA>(anorm, base, vec_at<FORM, VEC>(j, swap, jn, hidden)), o);
     }
   }
   amax = red.max(amax);
@@ -243,8 +237,7 @@ __device__ __forceinline__ void sq_row(const RowPos& p, int j0, int jn,
       } else {
         q = i8_codes<-127, VEC>(a[v], inv);
       }
-      const int skip = vec_skip<FORM, VEC>(k, hidden);
-      stf_codes_nt<FORM, VEC>(row_elem<UA>(out, base, (int64_t)j * VEC - skip), q, skip, apart);
+      stf_codes_nt<FORM, VEC>(row_elem<UA>(out, base, vec_at<FORM, VEC>(j, swap, jn, hidden)), q);
     }
   }
 }
@@ -264,6 +257,7 @@ k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   __shared__ double red_sum[16];
   __shared__ uint32_t red_max[16];
   const int nvec = vec_count<FORM, VEC>(hidden);
+  const bool swap = ares != nullptr && vec_swap<FORM>(nvec, tpr);
   RowPos p;
   if constexpr (EX) {
     p = row_pos_one();
@@ -272,7 +266,7 @@ k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
   }
   auto load_shared = [&](int v, WVec<EW, VEC>& w_, WVec<ES, VEC>& s_) {
     const int j = vec_index(v, tpr, EX ? p.lt : store_lane<NV>(p.lt));
-    const int64_t lj = vec_off<FORM, VEC>(j, nvec, hidden);
+    const int64_t lj = vec_off<FORM, VEC>(j, swap, nvec, hidden);
     w_.p = ldf<FORM, typename EW::S, VEC>(row_elem<EX>(w, 0, lj));
     s_.p = ldf<FORM, typename ES::S, VEC>(row_elem<EX>(sm, 0, lj));
   };
@@ -302,10 +296,10 @@ k_rms_norm_smooth_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     }
   };
   Pack<typename E::S, VEC> xv[NV], rv[NV];
-  sq_load<E, VEC, NV, RES, EX, EX, FORM>(p, 0, nvec, x, res, hidden, tpr, xv, rv);
+  sq_load<E, VEC, NV, RES, EX, EX, FORM>(p, 0, nvec, swap, x, res, hidden, tpr, xv, rv);
   WgRowReduce<EX> red{red_sum, red_max, tpr};
   sq_row<E, EW, ES, VEC, NV, FP8, RES, EX, EX, late, FORM>(
-      p, 0, nvec, xv, rv, shared, out, scales, ares, anorm, hidden, tpr, eps, flags, red);
+      p, 0, nvec, swap, xv, rv, shared, out, scales, ares, anorm, hidden, tpr, eps, flags, red);
 }
 
 // Rows too wide for one workgroup's registers, read once (split_row.h): workgroup b takes slice
@@ -342,12 +336,12 @@ k_rms_norm_smooth_quant_split(uint8_t* __restrict__ out, float* __restrict__ sca
     s_.p = ld<typename ES::S, VEC>(row_elem<true>(sm, 0, lj));
   };
   Pack<typename E::S, VEC> xv[NV], rv[NV];
-  sq_load<E, VEC, NV, RES, false, true>(p, j0, jn, x, res, hidden, tpr, xv, rv);
+  sq_load<E, VEC, NV, RES, false, true>(p, j0, jn, false, x, res, hidden, tpr, xv, rv);
   SplitRowReduce red{red_sum, red_max, tpr, ws, p.row, slices, sl,
                      ws + split_ws_words(rows, slices) - 1, timeout_ticks, &x_sum, &x_max,
                      &x_fail};
   sq_row<E, EW, ES, VEC, NV, FP8, RES, false, true, true, FORM_ROWS>(
-      p, j0, jn, xv, rv, shared, out, scales, ares, anorm, hidden, tpr, eps, flags, red);
+      p, j0, jn, false, xv, rv, shared, out, scales, ares, anorm, hidden, tpr, eps, flags, red);
   if (red.failed() && p.lt == 0) scales[p.row] = __builtin_nanf("");
 }
 
@@ -656,8 +650,8 @@ static int dispatch(const Args& a, hipStream_t st) {
   const bool vec_ok = a.hidden % V == 0 && aligned(16, a.x, a.ares, a.anorm, a.res) &&
                       aligned(WB, a.w) && aligned(SB, a.sm) && aligned(V, a.out);
   const bool r = a.res != nullptr;
-  // any other row of at least one vector takes the ragged form, narrower ones one element a load
-  const bool rag = !vec_ok && a.hidden >= V;
+  // other rows take the ragged form or one element a load (ragged_rows)
+  const bool rag = !vec_ok && ragged_rows(a.rows, a.hidden, V, ROW_SMOOTH);
   const int vec = vec_ok || rag ? V : 1;
   const KernelOfNv kernels =
       vec_ok ? (r ? &kernel_of<E, EW, ES, V, FP8, true> : &kernel_of<E, EW, ES, V, FP8, false>)

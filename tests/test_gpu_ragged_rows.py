@@ -1,7 +1,8 @@
 """Rows that are not whole aligned vectors (any width of at least one vector, any base address)
 against the CPU oracle, through every operator that has a ragged form: one element past and before
-whole vectors, the last vector alone in its wave (8 * 64 * k + 1 wide: in-place operators store it
-element by element there), the narrowest rows, and the widest that the registers hold."""
+whole vectors, the last vector the first of a wave's run of lanes (8 * 64 * k + 1 wide: in-place
+operators turn the row there), the narrowest rows, and the widest that the registers hold; with few
+rows, which mostly load one element at a time, and with many."""
 
 import pytest
 import torch
@@ -71,7 +72,7 @@ def test_norms_and_quantizers(H, dtype, T):
     assert_codes(q, q_ref, "fp8 codes")
 
 
-@pytest.mark.parametrize("T", [3, 300])
+@pytest.mark.parametrize("T", [3, 300, 2100])
 @pytest.mark.parametrize("H", WIDTHS)
 def test_smooth_scale_and_padded(H, T):
     if T * H > 3_000_000:
@@ -109,10 +110,10 @@ def test_smooth_scale_and_padded(H, T):
 @pytest.mark.parametrize("H", [513, 1025, 1537, 2049, 4097, 5121, 8193, 5120, 7168, 7176, 50000])
 def test_after_res_over_the_residual(H):
     """after_res given as the residual's (or the input's) own buffer: odd widths, where the last
-    vector of a row starts a wave and overlaps one that another wave stores; whole vectors that
-    leave lanes over (640, 896 and 897 of them), which load a copy of a vector that another wave
+    vector of a row would start a wave and overlaps the one before; whole vectors that leave lanes
+    over (640, 896 and 897 of them), which load a copy of a vector that another wave
     stores; and the same in every slice of a split row (6250 vectors)."""
-    T, eps = 300 if H < 10000 else 40, 1e-6
+    T, eps = 2100 if H < 5000 else 300 if H < 10000 else 40, 1e-6
     x, r, w, xd, rd, wd = rows(H, T, BF, 0)
     sm = 0.5 + torch.rand(H, generator=gen(H + 3))
     ar, out, ref = torch.empty_like(xd), torch.empty_like(xd), torch.empty_like(xd)
@@ -133,3 +134,33 @@ def test_after_res_over_the_residual(H):
         assert_exact(an, an_ref, f"H4 after_norm over the {own}")
         assert_scales(s, s_ref, f"H4 scales over the {own}")
         assert_codes(q, q_ref, f"H4 codes over the {own}")
+
+
+# either side of each line between the element-wise and the ragged form: the narrowest rows, few
+# rows, one vector a lane, the chip's SIMDs with a wave each, the element-wise form's widest row
+@pytest.mark.parametrize("T,H", [(300, 31), (300, 33), (300, 63), (300, 66), (256, 511), (256, 513),
+                                 (257, 513), (256, 2047), (256, 2049), (1000, 1023), (1025, 1023),
+                                 (1024, 769), (256, 769), (1025, 769), (2048, 769), (2100, 769), (4, 4095),
+                                 (4, 4097)])
+@pytest.mark.parametrize("dtype", [BF, HF, F32])
+def test_lines_between_the_forms(dtype, T, H):
+    eps = 1e-6
+    x, r, w, xd, rd, wd = rows(H, T, dtype, 0)
+    sm = 0.5 + torch.rand(H, generator=gen(H + 3))
+    x_ref, r_ref = oracle.fused_add_rms_norm(x, r, w, eps)
+    xx, rr = xd.clone(), rd.clone()
+    torch.ops._C.fused_add_rms_norm(xx, rr, wd, eps)
+    assert_exact(rr, r_ref, "H1 residual")
+    assert_exact(xx, x_ref, "H1 output")
+    out, ar, an = torch.empty_like(xd), torch.empty_like(xd), torch.empty_like(xd)
+    op.rms_norm(out, xd, wd, eps, ar, rd, False)
+    out_ref, ar_ref = oracle.rms_norm(x, w, eps, r, False)
+    assert_exact(ar, ar_ref, "norm after_res")
+    assert_exact(out, out_ref, "norm")
+    q_ref, s_ref, ar_ref, an_ref = oracle.rms_norm_smooth_quant(x, w, sm, eps, torch.int8, r)
+    q, s = torch.empty(T, H, dtype=torch.int8, device=DEV), torch.empty(T, device=DEV)
+    op.rms_norm_dynamic_per_token_quant(q, xd, wd, sm.to(DEV), s, eps, ar, an, rd)
+    assert_exact(ar, ar_ref, "H4 after_res")
+    assert_exact(an, an_ref, "H4 after_norm")
+    assert_scales(s, s_ref, "H4 scales")
+    assert_codes(q, q_ref, "H4 codes")
