@@ -454,9 +454,12 @@ static void launch_nv(const Geometry& g, const GqArgs& a, hipStream_t st) {
   auto* xp = static_cast<const S*>(a.x);
   auto* wp = static_cast<const S*>(a.w);
   auto* rp = static_cast<S*>(a.res);
-  // four-wave workgroups at four vectors a lane: four resident on a CU (8192 x 8192 fp8 79.0 us at
-  // the six that their registers allow, 78.2 at four, 78.4 at three)
-  const unsigned lds = resident_cap(VEC > 1 && g.nv == 4 && g.tpr * g.rpb == 256 ? 4 : 0, g.blocks);
+  // Rows with a residual in four-wave workgroups at four vectors a lane: four resident on a CU (us
+  // uncapped and so: 8192 x 8192 bf16 fp8 79.3 and 78.3; 16384 x 3072 fp32, 16384 x 4096 fp16 and
+  // 32768 x 2048 bf16 the same).  Rows without one, mostly reads, want every load in flight (8192 x
+  // 7168 int8 38.3, capped 41.6; 16384 x 1536 fp32 26.5 and 32.3).
+  const unsigned lds =
+      resident_cap(RES && VEC > 1 && g.nv == 4 && g.tpr * g.rpb == 256 ? 4 : 0, g.blocks);
 #define MCOP_LAUNCH(NVV, EXX)                                                                   \
   hipLaunchKernelGGL((k_rms_norm_group_quant<E, VEC, NVV, FP8, RES, EXX>), grid, block, lds, st, o, \
                      a.scales, xp, wp, a.scale_ub, rp, a.rows, a.hidden, g.tpr, a.eps, a.group, \

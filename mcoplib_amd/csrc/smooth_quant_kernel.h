@@ -548,8 +548,12 @@ static void launch_nv(const Geometry& g, const Args& a, hipStream_t st) {
   // Four-wave workgroups at four vectors a lane: at most three on a CU, by dynamic LDS that they
   // do not use (their registers would let four in).  The memory side of this write-heavy row
   // prefers fewer rows in flight: 16384 x 7168 fp8 143.4 us at three, 145.7 at four; 8192 x 4096
-  // 42.5 and 43.6.
-  const unsigned lds = resident_cap(VEC > 1 && g.nv == 4 && g.tpr * g.rpb == 256 ? 3 : 0, g.blocks);
+  // 42.5 and 43.6; 8192 x 8192 int8 79.7 and 83.2, fp32 8192 x 4096 93.9 and 97.9.  Rows that leave
+  // more than an eighth of their lanes empty have fewer in flight as it is (16384 x 3072 64.7 and 63.4,
+  // fp32 16384 x 1536 60.7 and 58.5).
+  const bool full = 8 * (int64_t)a.hidden >= 7 * (int64_t)VEC * 4 * g.tpr;
+  const unsigned lds =
+      resident_cap(VEC > 1 && g.nv == 4 && g.tpr * g.rpb == 256 && full ? 3 : 0, g.blocks);
 #define MCOP_LAUNCH(NVV, EXX)                                                                   \
   hipLaunchKernelGGL((k_rms_norm_smooth_quant<E, EW, ES, VEC, NVV, FP8, RES, EXX>), grid,      \
                      block, lds, st, o, a.scales, xp, wp, sp, arp, anp, rp, a.rows, a.hidden,      \
