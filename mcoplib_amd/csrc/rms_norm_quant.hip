@@ -586,7 +586,15 @@ static int dispatch(const char* name, void* out, float* scales, const void* x, c
                     : &kernel_of<E, V, FP8, false, MODE, true>)
              : (res ? &kernel_of<E, 1, FP8, true, MODE> : &kernel_of<E, 1, FP8, false, MODE>);
   if constexpr (MODE != QM_MC_7168) {
-    if (!row_fits(hidden, vec, kernels)) {
+    const bool fits = row_fits(hidden, vec, kernels);
+    // 16-bit rows that only sixteen vectors a lane hold (one workgroup of eight waves on a CU) are
+    // split all the same where there are many.  us at sixteen and split, int8: 2048 x 40960 fp16
+    // with a residual 131 and 109, 2048 x 65536 bf16 171 and 164, 1024 x 36864 bf16 63.5 and 58.2,
+    // 512 x 40960 fp16 35.9 and 40.9; without one 2048 x 40960 bf16 81.9 and 71.5, 1024 x 50000 46.9
+    // and 51.6.  (The no-allocation entry point's shared scratch is kept to rows that need it.)
+    const bool split16 = V == 8 && scratch == nullptr && hidden > 8 * max_tpr(V, 8) * V &&
+                         rows >= (res ? 1024 : 2048);
+    if (!fits || split16) {
       if (vec_ok && split_rows_enabled()) {
         const int rc =
             res ? launch_split<E, V, FP8, true, MODE>(name, out, scales, x, w, scale_ub, res,
@@ -595,6 +603,8 @@ static int dispatch(const char* name, void* out, float* scales, const void* x, c
                                                        rows, (int)hidden, eps, scratch, st);
         if (rc != MCOP_E_UNSUPPORTED) return rc;
       }
+    }
+    if (!fits) {
       if (!wide_rows_ok(name, rows)) return MCOP_E_UNSUPPORTED;
       using S = typename E::S;
       auto* o = static_cast<uint8_t*>(out);

@@ -686,3 +686,47 @@ def test_split_launch_decisions_are_traced():
     assert re.search(r"rows=4: split-row kernel, (8 slices of 2048|16 slices of 1024) vectors "
                      r"over 256 lanes", out.stdout)
     assert "rows=4: multi-pass kernel" in out.stdout
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("res", [True, False])
+@pytest.mark.parametrize("H", [32776, 40960, 65536])
+def test_many_rows_that_sixteen_vectors_a_lane_hold(H, res, dtype):
+    """Norm-quant rows that the registers hold at sixteen vectors a lane only are split where there
+    are many, and not in a graph: the same bits either way, and the oracle's."""
+    T = 1024 if res else 2048
+    say(f"split rows that fit: {dtype} {T}x{H} residual {res}")
+    g = torch.Generator(device=DEV).manual_seed(H)
+    x = torch.randn(T, H, generator=g, device=DEV).to(dtype)
+    r = torch.randn(T, H, generator=g, device=DEV).to(dtype) if res else None
+    w = (1 + 0.1 * torch.randn(H, generator=g, device=DEV)).to(dtype)
+    for qdt in (torch.int8, torch.float8_e4m3fn):
+        def run():
+            torch.ops._C.rms_norm_dynamic_per_token_quant(q, x, w, s, 1e-6, None, rr)
+
+        got = []
+        for split in (True, False):
+            q = torch.empty(T, H, dtype=qdt, device=DEV)
+            s = torch.empty(T, 1, device=DEV)
+            rr = r.clone() if res else None
+            _lib.set_split_rows(split)
+            try:
+                run()
+            finally:
+                _lib.set_split_rows(True)
+            got.append((q.view(torch.int8), s, rr))
+        graph = torch.cuda.CUDAGraph()
+        q, s, rr = torch.empty_like(q), torch.empty_like(s), r.clone() if res else None
+        with torch.cuda.graph(graph):
+            run()
+        graph.replay()
+        torch.cuda.synchronize()
+        got.append((q.view(torch.int8), s, rr))
+        for other in got[1:]:
+            assert all(a is None or torch.equal(a, b) for a, b in zip(got[0], other))
+        q_ref, s_ref, r_ref = oracle.rms_norm_dynamic_per_token_quant(
+            x[:8].cpu(), w.cpu(), 1e-6, qdt, residual=r[:8].cpu() if res else None)
+        assert_codes(got[0][0][:8].view(qdt), q_ref, "codes")
+        assert_scales(got[0][1][:8], s_ref, "scales")
+        if res:
+            assert_exact(got[0][2][:8], r_ref, "residual")
