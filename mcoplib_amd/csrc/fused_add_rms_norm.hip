@@ -59,7 +59,9 @@ k_fused_add_rms_norm(typename E::S* __restrict__ x, int64_t x_stride,
   // are summed (the latency falls into the reduction): all three at once spill.
   constexpr int w_early = NV >= 16 && std::is_same<E, F16>::value ? 12 : NV;
 #pragma unroll
-  for (int v = 0; v < w_early; ++v) wv[v] = ldf<FORM, S, VEC>(row_elem<true>(w, 0, lj_of(v)));
+  for (int v = 0; v < w_early; ++v) {
+    wv[v] = ldf<FORM, S, VEC>(row_elem<(EX || NV >= 4)>(w, 0, lj_of(v)));
+  }
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {

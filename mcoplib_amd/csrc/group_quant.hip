@@ -92,7 +92,9 @@ k_rms_norm_group_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
 
   Pack<S, VEC> xv[NV], rv[NV], wv[NV];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) wv[v] = ld<S, VEC>(row_elem<true>(w, 0, lj_of(v)));
+  for (int v = 0; v < NV; ++v) {
+    wv[v] = ld<S, VEC>(row_elem<(EX || NV >= 4)>(w, 0, lj_of(v)));
+  }
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {

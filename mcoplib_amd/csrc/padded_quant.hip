@@ -58,7 +58,9 @@ k_add_rms_norm_quant_padded(uint8_t* __restrict__ padded, uint16_t* __restrict__
 
   Pack<uint16_t, VEC> xv[NV], rv[NV], wv[NV];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) wv[v] = ldf<FORM, uint16_t, VEC>(row_elem<true>(w, 0, lj_of(v)));
+  for (int v = 0; v < NV; ++v) {
+    wv[v] = ldf<FORM, uint16_t, VEC>(row_elem<(EX || NV >= 4)>(w, 0, lj_of(v)));
+  }
   shared_loads_first();
 #pragma unroll
   for (int v = 0; v < NV; ++v) {

@@ -125,7 +125,7 @@ k_rms_norm_quant(uint8_t* __restrict__ out, float* __restrict__ scales,
     if constexpr (RES) rv[v] = ldf_nt<FORM, S, VEC>(row_elem<EX>(res, base, lj));
     // with fewer vectors per lane the weight loads interleave with the streamed ones (measured
     // 1.5% faster at 8192 x 8192, two vectors per lane; shared-first won at four)
-    if constexpr (NV < 4) wv[v] = ldf<FORM, S, VEC>(row_elem<true>(w, 0, lj));
+    if constexpr (NV < 4) wv[v] = ldf<FORM, S, VEC>(row_elem<EX>(w, 0, lj));
   }
 
   const int slt = store_lane<NV>(p.lt);
