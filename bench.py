@@ -282,6 +282,8 @@ WORKLOADS = {
     "head-norm": Workload("head-norm", 65536 * 8, 128, 1e-6, "head_norm"),
     # the un-normed SmoothQuant sibling (scale_dynamic_quant) at SmoothQuant's shape
     "sdq": Workload("sdq", 16384, 7168, 0.0, "sdq"),
+    # rows of an odd width, none of whose addresses is a multiple of 16 bytes past the first
+    "ragged-int8": Workload("ragged-int8", 8192, 5137, 1e-6, "add_norm_int8"),
     # rows wider than the registers hold: the split-row kernels of H1, H2/H3, H4 and H5 (the row
     # shared by several workgroups, read once), each other operator's multi-pass kernel
     "wide-int8": Workload("wide-int8", 2048, 131072, 1e-6, "add_norm_int8"),
